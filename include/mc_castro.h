@@ -263,11 +263,11 @@ int mc_level_blast_radius(mc_level_t *L, double *blast_mass, double *blast_radiu
 double mc_level_time(const mc_level_t *L);
 double mc_level_dt(const mc_level_t *L);
 int mc_level_sync(mc_level_t *L);
-/* The fused engine keeps its face-stage arrays (traces, fluxes: about
-   3.1 KB per cell) for the whole level, or for one z-slab of `planes` cell
-   planes at a time, the face stages and the update then running slab after
-   slab (about 0.35 KB per cell plus 3.1 KB per cell of one slab and its
-   two ring planes).  Results are the same bit for bit.  planes = -1 (the
+/* The fused engine keeps its primitives and face-stage arrays (traces,
+   fluxes: about 1.8 KB per cell together) for the whole level, or for one
+   z-slab of `planes` cell planes at a time, the stages then running slab
+   after slab (the state's 0.16 KB per cell plus 1.8 KB per cell of one slab
+   and its neighbouring planes).  Results are the same bit for bit.  planes = -1 (the
    default) keeps the whole level when that takes at most half the free
    device memory, else picks the deepest slab that does; 0 forces the whole
    level.  Changing it rebuilds the engine (state and clock kept).

@@ -107,16 +107,20 @@ __global__ __launch_bounds__(256) void A_update(Plan p, Ctx x, ACtx a)
     clean_hydro(ua, x.tab);
     const SpeciesPairs P0 = species_pairs(F0, I, NFN, FN_X), P1 = species_pairs(F1, I, NFN, FN_X),
                        P2 = species_pairs(F2, I, NFN, FN_X);
+    const double c0 = species_fac(P0, e, EF(F0, I, NFN, URHO, e)), c0x = species_fac(P0, ex, EF(F0, I, NFN, URHO, ex)),
+                 c1 = species_fac(P1, e, EF(F1, I, NFN, URHO, e)), c1y = species_fac(P1, ey, EF(F1, I, NFN, URHO, ey)),
+                 c2 = species_fac(P2, e, EF(F2, I, NFN, URHO, e)), c2z = species_fac(P2, ez, EF(F2, I, NFN, URHO, ez));
 #pragma unroll
     for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const dbl2 f0 = SP2(P0, pr, e), f0x = SP2(P0, pr, ex), f1 = SP2(P1, pr, e), f1y = SP2(P1, pr, ey),
-                   f2 = SP2(P2, pr, e), f2z = SP2(P2, pr, ez);
+        const dbl2 f0 = SP2(P0, pr, e) * c0, f0x = SP2(P0, pr, ex) * c0x, f1 = SP2(P1, pr, e) * c1,
+                   f1y = SP2(P1, pr, ey) * c1y, f2 = SP2(P2, pr, e) * c2, f2z = SP2(P2, pr, ez) * c2z;
         const int n = UFS + 2 * pr;
         u1[n] = ua[n] + dt * flux_div(f0.x, f0x.x, f1.x, f1y.x, f2.x, f2z.x, a0, a1, a2, volinv);
         if (n + 1 < NVAR) u1[n + 1] = ua[n + 1] + dt * flux_div(f0.y, f0x.y, f1.y, f1y.y, f2.y, f2z.y, a0, a1, a2, volinv);
     }
+    u1[UTEMP] = ua[UTEMP];  // no flux
 #pragma unroll
-    for (int n = 0; n < UFS; ++n) {
+    for (int n = 0; n < UTEMP; ++n) {
         double s = flux_div(EF(F0, I, NFN, n, e), EF(F0, I, NFN, n, ex), EF(F1, I, NFN, n, e), EF(F1, I, NFN, n, ey),
                             EF(F2, I, NFN, n, e), EF(F2, I, NFN, n, ez), a0, a1, a2, volinv);
         if (n == UEINT) {

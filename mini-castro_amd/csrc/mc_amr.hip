@@ -93,10 +93,12 @@ __global__ void k_reg_fine_add(Box fb, long n, double *reg, Arr flx, int dir, in
 // as k_store_flux forms it before the sum of k_reg_fine_add
 __device__ __forceinline__ double fn_component(double *FN, const FInst &I, int c, idx_t e)
 {
+    if (c == UTEMP) return 0.0;
     if (c < UFS) return EF(FN, I, NFN, c, e);
     const int sp = c - UFS;
-    const dbl2 v = SP2(species_pairs(FN, I, NFN, FN_X), sp >> 1, e);
-    return (sp & 1) ? v.y : v.x;
+    const SpeciesPairs X = species_pairs(FN, I, NFN, FN_X);
+    const dbl2 v = SP2(X, sp >> 1, e);
+    return ((sp & 1) ? v.y : v.x) * species_fac(X, e, EF(FN, I, NFN, URHO, e));
 }
 
 __global__ void k_reg_fine_add_fn(Box fb, long n, double *reg, double *FN, const FInst *inst, int dir, int r0,

@@ -10,9 +10,12 @@
 //   K_flux1   faces   CGF fluxes of the PPM states           F^d
 //   K_trans1  faces   one-direction transverse update + flux  F^{t|d}
 //   K_final   faces   two-direction transverse update + final flux,
-//                     artificial viscosity, species flux normalisation
-//   K_update  cells   flux divergence and p dV source, S_new = S_old + dt
-//                     src, clean_state twice, estdt min-reduction
+//                     artificial viscosity
+//   K_species columns the thirteen species from their traces to their final
+//                     fluxes (mc_species.h), launched with the final fluxes
+//   K_update  cells   species flux normalisation, flux divergence and p dV
+//                     source, S_new = S_old + dt src, clean_state twice, estdt
+//                     min-reduction
 //   K_dt      1 block the CFL / change_max / init_shrink time-step control
 //
 // Why the result equals the per-box path bit for bit: every stage applies the
@@ -35,11 +38,12 @@
 // Layout: per instance, structure-of-arrays; a cell array with C components
 // holds component c of cell (i,j,k) at C*off + c*ncell + i + n0*(j + n1*k);
 // extended arrays cover [-1, n] in each direction.  The face arrays hold
-// their components in interleaved pairs, and the species of q and of the
-// cleaned state sit apart in arrays of pairs (EF, EF2, SP2 in
-// mc_fused_impl.h), so one 16-byte access moves two components.  dt lives on
+// their components in interleaved pairs, and the species of the cleaned state
+// sit apart in an array of pairs (EF, EF2, SP2 in mc_fused_impl.h), so one
+// 16-byte access moves two components.  dt lives on
 // the device (one slot per instance), so a step can be captured in a hipGraph.
 #include <float.h>
+#include <math.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -53,6 +57,7 @@
 #include "mc_fused_impl.h"
 #include "mc_hydro.h"
 #include "mc_internal.h"
+#include "mc_species.h"
 
 namespace mc {
 
@@ -77,55 +82,77 @@ __global__ __launch_bounds__(256) void K_est(Plan p, Ctx x)
 
 // S_old clean (Castro_advance.cpp:51), Sborder clean (:66), ctoprim.
 // Held to 2 waves per SIMD like K_update (3.85 -> 3.65 ms at 256^3).
+// SLABS: the planes [zlo, zlo + zn) that a slab adds to the ring buffer of
+// primitives.  Planes outside a periodic instance are its images, made from
+// the saved boundary planes (Ctx::UB) and not stored back.
+template <bool SLABS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void K_prim(Plan p, Ctx x)
 {
     int m, i, j, k;
     if (!plan_cell(p, m, i, j, k)) return;
     const FInst &I = p.inst[m];
-    const idx_t c = cidx(I, i, j, k);
+    const bool own = !SLABS || (k >= 0 && k < I.n[2]);
+    const idx_t c = cidx(I, i, j, k), cw = SLABS ? widx(I, i, j, k) : c;
     double u[NVAR];
+    if (own) {
 #pragma unroll
-    for (int n = 0; n < NVAR; ++n) u[n] = CA(x.U, I, NVAR, n, c);
+        for (int n = 0; n < NVAR; ++n) u[n] = CA(x.U, I, NVAR, n, c);
+    } else {
+        const long np = (long)I.n[0] * I.n[1] * 2 * WHALO;
+        const double *ub = x.UB + NVAR * I.offP + i + (long)I.n[0] * (j + (long)I.n[1] * (k < 0 ? k + 2 * WHALO : k - I.n[2]));
+#pragma unroll
+        for (int n = 0; n < NVAR; ++n) u[n] = ub[n * np];
+    }
     clean_cell(u, x.tab); /* S_old clean, Castro_advance.cpp:51 */
     // S_old is replaced by its clean in place: K_update starts from it
     // instead of cleaning S_old a second time (nothing between reads U)
+    if (own) {
 #pragma unroll
-    for (int n = 0; n < NVAR; ++n) CA(x.U, I, NVAR, n, c) = u[n];
+        for (int n = 0; n < NVAR; ++n) CA(x.U, I, NVAR, n, c) = u[n];
+    }
     clean_cell(u, x.tab); /* Sborder clean, Castro_advance.cpp:66 */
 #pragma unroll
-    for (int n = 0; n < NU1; ++n) CA(x.U1, I, NU1, n, c) = u[n];
-    {
-        const SpeciesPairs XU = cell_species(x.U1X, I);
-#pragma unroll
-        for (int pr = 0; pr < NSPEC_PAIRS; ++pr)
-            SP2(XU, pr, c) = dbl2{u[UFS + 2 * pr], 2 * pr + 1 < NSPEC ? u[UFS + 2 * pr + 1] : 0.0};
-    }
+    for (int n = 0; n < NU1; ++n) WA(x.U1, I, NU1, n, cw) = u[n];
     // the EOS-free primitives are stored before the EOS call, so they are
-    // not held in registers through it
+    // not held in registers through it; the species of q are those of U1
+    // times 1/rho (FQ_RI)
     PrimPre a;
     {
         double xs[NSPEC];
         ctoprim_pre(u, a, xs);
-        const SpeciesPairs XQ = cell_species(x.QX, I);
-        CA(x.Q, I, NFQ, FQ_RHO, c) = a.rho;
-        CA(x.Q, I, NFQ, FQ_U, c) = a.u;
-        CA(x.Q, I, NFQ, FQ_V, c) = a.v;
-        CA(x.Q, I, NFQ, FQ_W, c) = a.w;
+        const SpeciesPairs XU = cell_species(x.U1X, I);
 #pragma unroll
         for (int pr = 0; pr < NSPEC_PAIRS; ++pr)
-            SP2(XQ, pr, c) = dbl2{xs[2 * pr], 2 * pr + 1 < NSPEC ? xs[2 * pr + 1] : 0.0};
+            SP2(XU, pr, cw) = dbl2{u[UFS + 2 * pr], 2 * pr + 1 < NSPEC ? u[UFS + 2 * pr + 1] : 0.0};
+        WA(x.Q, I, NFQ, FQ_RHO, cw) = a.rho;
+        WA(x.Q, I, NFQ, FQ_U, cw) = a.u;
+        WA(x.Q, I, NFQ, FQ_V, cw) = a.v;
+        WA(x.Q, I, NFQ, FQ_W, cw) = a.w;
+        WA(x.Q, I, NFQ, FQ_RI, cw) = 1.0 / a.rho;
     }
     Prim q;
     ctoprim_eos(x.tab, a, q);
-    CA(x.Q, I, NFQ, FQ_P, c) = q.p;
-    CA(x.Q, I, NFQ, FQ_RE, c) = q.rhoe;
-    CA(x.Q, I, NFQ, FQ_C, c) = q.cs;
-    CA(x.Q, I, NFQ, FQ_G, c) = q.gamc;
+    WA(x.Q, I, NFQ, FQ_P, cw) = q.p;
+    WA(x.Q, I, NFQ, FQ_RE, cw) = q.rhoe;
+    WA(x.Q, I, NFQ, FQ_C, cw) = q.cs;
+    WA(x.Q, I, NFQ, FQ_G, cw) = q.gamc;
 }
 
-__device__ __forceinline__ double qv(const Ctx &x, const FInst &I, int comp, int i, int j, int k)
+// Slabs: the first and last WHALO planes of every instance's state (wrapped
+// for instances shallower than that), before the step's first clean.
+__global__ __launch_bounds__(256) void K_save_planes(const FInst *inst, int ninst, long n, Ctx x)
 {
-    return CA(x.Q, I, NFQ, comp, cidx(I, i, j, k));
+    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    int m = 0;
+    while (m + 1 < ninst && inst[m + 1].offP <= t) ++m;
+    const FInst &I = inst[m];
+    t -= I.offP;
+    const long nxy = (long)I.n[0] * I.n[1], np = nxy * 2 * WHALO;
+    const int q = (int)(t / nxy), k = bmap(q < WHALO ? q : q - 2 * WHALO, I.n[2], 1);
+    const double *u = x.U + NVAR * I.offD + (t % nxy) + nxy * k;
+    double *o = x.UB + NVAR * I.offP + t;
+    for (int c = 0; c < NVAR; ++c) o[c * np] = u[c * I.nD];
 }
 
 // uflatten (Source/ppm.F90:11-128) and divu (Source/Castro_hydro_nd.F90:11-69)
@@ -135,22 +162,30 @@ __global__ __launch_bounds__(256) void K_flat(Plan p, Ctx x)
     if (!plan_cell(p, m, i, j, k)) return;
     const FInst &I = p.inst[m];
     const idx_t e = eidx(I, i, j, k);
+    // rows and planes of the cells up to three away (offset s at s + 3)
+    idx_t ix[7], iy[7], iz[7];
+#pragma unroll
+    for (int s = -3; s <= 3; ++s) {
+        ix[s + 3] = (idx_t)bmap(i + s, I.n[0], I.periodic);
+        iy[s + 3] = (idx_t)I.n[0] * (idx_t)bmap(j + s, I.n[1], I.periodic);
+        iz[s + 3] = (idx_t)I.n[0] * (idx_t)I.n[1] * (idx_t)plane_w(I, k + s);
+    }
     double flatn = 1.0;
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const int ei = (d == 0), ej = (d == 1), ek = (d == 2);
         double p7[7], u7[7];
 #pragma unroll
-        for (int s = -3; s <= 3; ++s) {
-            const idx_t c = cidx(I, i + s * ei, j + s * ej, k + s * ek);
-            p7[s + 3] = CA(x.Q, I, NFQ, FQ_P, c);
-            u7[s + 3] = CA(x.Q, I, NFQ, FQ_U + d, c);
+        for (int s = 0; s < 7; ++s) {
+            const idx_t c = ix[d == 0 ? s : 3] + iy[d == 1 ? s : 3] + iz[d == 2 ? s : 3];
+            p7[s] = WA(x.Q, I, NFQ, FQ_P, c);
+            u7[s] = WA(x.Q, I, NFQ, FQ_U + d, c);
         }
         flatn = fmin(flatn, flatten_dir(p7, u7));
     }
     EA(x.FL, I, 1, 0, e) = flatn;
     if (i >= 0 && j >= 0 && k >= 0) {
         const double dxinv = 1.0 / I.dx[0], dyinv = 1.0 / I.dx[1], dzinv = 1.0 / I.dx[2];
-#define QQ(c, a, b, cc) qv(x, I, c, a, b, cc)
+#define QQ(c, a, b, cc) WA(x.Q, I, NFQ, c, ix[(a) - i + 3] + iy[(b) - j + 3] + iz[(cc) - k + 3])
         const double ux = FOURTH *
                           (+QQ(FQ_U, i, j, k) - QQ(FQ_U, i - 1, j, k) + QQ(FQ_U, i, j, k - 1) -
                            QQ(FQ_U, i - 1, j, k - 1) + QQ(FQ_U, i, j - 1, k) - QQ(FQ_U, i - 1, j - 1, k) +
@@ -171,16 +206,6 @@ __global__ __launch_bounds__(256) void K_flat(Plan p, Ctx x)
     }
 }
 
-// What the species part of a cell's trace takes from its hydro part: the
-// stencil, the wave speed and dt/dx, which states the cell stores, and the
-// species pair bases (taken before any store, see SpeciesPairs).
-struct TraceCtx {
-    idx_t cs[5], ep, em;
-    double flatn, un, dtdx;
-    bool do_p, do_m;
-    SpeciesPairs XP, XM, XQ;
-};
-
 // hydro part of a traced state, velocities in absolute order
 struct StateH {
     double rho, u, v, w, p, rhoe;
@@ -190,6 +215,7 @@ struct StateH {
 // of n threads with b cells along its direction stages (b + 4) n / b cells
 // (the stencil's two cells either side), at most QTILE.
 constexpr int QTILE = 448;
+constexpr int NQT = FQ_G + 1;  // components of the tile (all but 1/rho)
 
 // PPM reconstruction + characteristic tracing (Source/ppm.F90:309-743) of
 // cell (i,j,k) of instance m in direction d, hydro part: the plus state of
@@ -201,29 +227,27 @@ constexpr int QTILE = 448;
 // instead of the cell arrays.
 template <bool STAGED>
 __device__ __forceinline__ void trace_hydro(const Ctx &x, int m, const FInst &I, int d, int i, int j, int k,
-                                            bool own_p, TraceCtx &t, FaceH &fp, FaceH &fm,
-                                            const double *tile = nullptr, int self = 0, int sr = 0)
+                                            bool own_p, FaceH &fp, FaceH &fm, const double *tile = nullptr,
+                                            int self = 0, int sr = 0)
 {
     const int di = (d == 0), dj = (d == 1), dk = (d == 2);
     const int pos = d == 0 ? i : (d == 1 ? j : k);
-    t.do_p = own_p && pos >= 0;
+    const bool do_p = own_p && pos >= 0;
     // the minus state of face pos + 1; in z it must lie in the slab's faces
-    t.do_m = pos <= I.n[d] - 1 && (d != 2 || k + 1 <= I.zlo + I.zn);
+    const bool do_m = pos <= I.n[d] - 1 && (d != 2 || k + 1 <= I.zlo + I.zn);
     const int cun = FQ_U + d, cut = d == 0 ? FQ_V : (d == 1 ? FQ_W : FQ_U), cutt = d == 0 ? FQ_W : (d == 1 ? FQ_U : FQ_V);
+    idx_t cs[5];
 #pragma unroll
-    for (int s = -2; s <= 2; ++s) t.cs[s + 2] = cidx(I, i + s * di, j + s * dj, k + s * dk);
+    for (int s = -2; s <= 2; ++s) cs[s + 2] = STAGED ? 0u : widx(I, i + s * di, j + s * dj, k + s * dk);
     // component c of the primitives of cell pos - 2 + q
     auto qs = [&](int c, int q) -> double {
         if (STAGED) return tile[c * QTILE + self + q * sr];
-        return CA(x.Q, I, NFQ, c, t.cs[q]);
+        return WA(x.Q, I, NFQ, c, cs[q]);
     };
     const double cc = qs(FQ_C, 2);
     const double un = qs(cun, 2);
     const double flatn = EA(x.FL, I, 1, 0, eidx(I, i, j, k));
     const double dtdx = x.dt_cur[m] / I.dx[d];
-    t.un = un;
-    t.flatn = flatn;
-    t.dtdx = dtdx;
 
     double Ip[3][4], Im[3][4], Ip_ut = 0, Im_ut = 0, Ip_utt = 0, Im_utt = 0;
     const int vars[6] = {FQ_RHO, cun, FQ_P, FQ_RE, cut, cutt};
@@ -255,12 +279,8 @@ __device__ __forceinline__ void trace_hydro(const Ctx &x, int m, const FInst &I,
         (void)a;
         (void)b;
     }
-    t.ep = eidx(I, i, j, k);
-    t.em = eidx(I, i + di, j + dj, k + dk);
+    const idx_t ep = eidx(I, i, j, k), em = eidx(I, i + di, j + dj, k + dk);
     double *SP = x.SP[d], *SM = x.SM[d];
-    t.XP = species_pairs(SP, I, NFS, FS_X);
-    t.XM = species_pairs(SM, I, NFS, FS_X);
-    t.XQ = cell_species(x.QX, I);
     // velocities back in absolute order: the normal one is FS_U + d, the
     // first transverse FS_V, FS_W, FS_U and the second FS_W, FS_U, FS_V for
     // d = 0, 1, 2; stored as the pairs (rho, u), (v, w), (p, rhoe)
@@ -285,66 +305,36 @@ __device__ __forceinline__ void trace_hydro(const Ctx &x, int m, const FInst &I,
         EF2(S, I, NFS, FS_V, ee) = dbl2{o.v, o.w};
         EF2(S, I, NFS, FS_P, ee) = dbl2{o.p, o.rhoe};
     };
+    double rho_p;
     {
         double r, u_, e, pp;
         ppm_project<true>(Im, gam_m, un, cc, r, u_, e, pp);
         StateH sp;
         to_abs(sp, fp, r, u_, Im_ut, Im_utt, e, pp);
-        if (t.do_p) store_state(SP, t.ep, sp);
+        if (do_p) store_state(SP, ep, sp);
+        rho_p = sp.rho;
     }
     {
         double r, u_, e, pp;
         ppm_project<false>(Ip, gam_p, un, cc, r, u_, e, pp);
         StateH sm;
         to_abs(sm, fm, r, u_, Ip_ut, Ip_utt, e, pp);
-        if (t.do_m) store_state(SM, t.em, sm);
+        if (do_m) store_state(SM, em, sm);
+        // the layer below the range's first cell belongs to no brick's own cells
+        if (own_p || pos < lo_index(I, d)) EF2(x.RW, I, 6, 2 * d, ep) = dbl2{rho_p, sm.rho};
     }
-}
-
-// Species pair pr of the trace (after trace_hydro): the plus-state pair of
-// face pos in xp, the minus-state pair of face pos + 1 in xm, both stored
-// where the cell stores its states.  The last pair of an odd species count
-// carries 0 in its second slot.
-__device__ __forceinline__ void trace_species(const TraceCtx &t, int pr, dbl2 &xp, dbl2 &xm)
-{
-    double ipv[2] = {0.0, 0.0}, imv[2] = {0.0, 0.0};
-    dbl2 s2[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) s2[q] = SP2(t.XQ, pr, t.cs[q]);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int ns = 2 * pr + h;
-        if (ns >= NSPEC) break;
-        double s[5], sm, sp;
-#pragma unroll
-        for (int q = 0; q < 5; ++q) s[q] = h == 0 ? s2[q].x : s2[q].y;
-        ppm_reconstruct(s, t.flatn, sm, sp);
-        const double s6 = ppm_s6(sm, sp, s[2]);
-        ppm_int_wave(sm, sp, s6, t.un, t.dtdx, ipv[h], imv[h]);
-    }
-    xp = dbl2{imv[0], imv[1]};
-    xm = dbl2{ipv[0], ipv[1]};
-    if (t.do_p) SP2(t.XP, pr, t.ep) = xp;
-    if (t.do_m) SP2(t.XM, pr, t.em) = xm;
 }
 
 __global__ __launch_bounds__(256) void K_trace(Plan p, Ctx x)
 {
     int m, i, j, k, sub_;
     if (!plan_cell_sub(p, 3, sub_, m, i, j, k)) return;
-    TraceCtx t;
     FaceH fp, fm;
-    trace_hydro<false>(x, m, p.inst[m], sub_, i, j, k, true, t, fp, fm);
-    // species last: their stores come after every read of the instance table
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        dbl2 xp, xm;
-        trace_species(t, pr, xp, xm);
-    }
+    trace_hydro<false>(x, m, p.inst[m], sub_, i, j, k, true, fp, fm);
 }
 
 // Source/riemann.F90:10-331 on the PPM states: F^d on d-face (i,j,k)
-// (d-face index 0..n_d, transverse cells -1..n).  Species are streamed in
-// pairs.
+// (d-face index 0..n_d, transverse cells -1..n).
 __device__ __forceinline__ void flux1_face(const Ctx &x, const FInst &I, int d, int i, int j, int k)
 {
     const idx_t e = eidx(I, i, j, k);
@@ -354,20 +344,6 @@ __device__ __forceinline__ void flux1_face(const Ctx &x, const FInst &I, int d, 
     RiemannH o;
     face_riemann_h(x, I, d, i, j, k, L, R, o);
     store_tflux_h(x.FD[d], I, e, d, o);
-    double *F = x.FD[d];
-    // a side whose weight is zero contributes +-0 to fpl*xl + fmr*xr: its
-    // species are not read
-    const bool useL = o.fpl != 0.0, useR = o.fmr != 0.0;
-    const SpeciesPairs XL = species_pairs(x.SM[d], I, NFS, FS_X), XR = species_pairs(x.SP[d], I, NFS, FS_X),
-                       XF = species_pairs(F, I, NFF, FF_X);
-#pragma unroll 1
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const dbl2 xl = useL ? (dbl2)SP2(XL, pr, e) : dbl2{0.0, 0.0};
-        const dbl2 xr = useR ? (dbl2)SP2(XR, pr, e) : dbl2{0.0, 0.0};
-        const double gx0 = o.fpl * xl.x + o.fmr * xr.x;
-        const double gx1 = o.fpl * xl.y + o.fmr * xr.y;
-        SP2(XF, pr, e) = dbl2{o.f_rho * gx0, o.f_rho * gx1};
-    }
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void K_flux1(Plan p, Ctx x)
@@ -395,23 +371,15 @@ __device__ __forceinline__ int below_of(int tid, int st) { return tid - st; }
 // l >= 1 solves the Riemann problem on its cell's low d-face with the minus
 // state the layer below left in LDS and its own plus state, kept in
 // registers, and the sound speeds and Gamma_1 of the tile: the first-stage
-// flux reads no traced state from memory.  The species follow the same way,
-// all pairs at once.
+// flux reads no traced state from memory.
 // A layer-0 cell belongs to the brick below as its top layer: it stores its
 // minus state (the same values that brick stores) but not its plus state,
 // and solves no Riemann problem.  The sub-launches are the directions,
 // interleaved block by block like the other face stages.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K_tflux(Plan3 p3, Ctx x)
 {
-    // the minus states' hydro part; the primitives' tile, then (after the
-    // barrier that ends its reads) the minus states' species in its memory
-    __shared__ FaceH lds_h[256];
-    __shared__ union {
-        double q[NFQ * QTILE];
-        dbl2 s[NSPEC_PAIRS][256];
-    } lds;
-    double *tile = lds.q;
-    dbl2(&lds_s)[NSPEC_PAIRS][256] = lds.s;
+    __shared__ FaceH lds_h[256];           // the minus states
+    __shared__ double tile[NQT * QTILE];   // the primitives
     int lb = logical_block(), d;
     if (gridDim.y > 1) {
         d = blockIdx.y;
@@ -455,55 +423,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
             b = j0 + c / p.bx;
             cz = k0 - 2 + r;
         }
-        const idx_t ce = cidx(I, a, b, cz);
+        const idx_t ce = widx(I, a, b, cz);
 #pragma unroll
-        for (int n = 0; n < NFQ; ++n) tile[n * QTILE + e] = CA(x.Q, I, NFQ, n, ce);
+        for (int n = 0; n < NQT; ++n) tile[n * QTILE + e] = WA(x.Q, I, NFQ, n, ce);
     }
     const int sr = d == 0 ? 1 : cw;  // tile stride of one row
     const int self = d == 0 ? l + (tj + p.by * tk) * rows : l * cw + (d == 1 ? ti + p.bx * tk : ti + p.bx * tj);
     __syncthreads();
-    TraceCtx t;
     FaceH fp, fm;
     if (ok) {
-        trace_hydro<true>(x, m, I, d, i, j, k, l > 0, t, fp, fm, tile, self, sr);
+        trace_hydro<true>(x, m, I, d, i, j, k, l > 0, fp, fm, tile, self, sr);
         lds_h[tid] = fm;
     }
-    const SpeciesPairs XF = species_pairs(x.FD[d], I, NFF, FF_X);
     __syncthreads();
+    if (!fx) return;
+    const FaceH L = lds_h[below];
     RiemannH o;
-    bool useL = false, useR = false;
-    if (fx) {
-        const FaceH L = lds_h[below];
-        // cells pos - 1 and pos: tile offsets 1 and 2 from the thread's row
-        riemann_hydro(L, fp, tile[FQ_C * QTILE + self + sr], tile[FQ_C * QTILE + self + 2 * sr],
-                      tile[FQ_G * QTILE + self + sr], tile[FQ_G * QTILE + self + 2 * sr], o);
-        store_tflux_h(x.FD[d], I, t.ep, d, o);
-        // a side whose weight is zero contributes +-0 to fpl*xl + fmr*xr
-        useL = o.fpl != 0.0;
-        useR = o.fmr != 0.0;
-    }
-    __syncthreads();  // the tile is read: its memory takes the species
-    // every pair's species trace first (the minus states to LDS, the plus
-    // states kept), so that their loads are in flight together; one barrier
-    dbl2 xpv[NSPEC_PAIRS];
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        dbl2 xp = dbl2{0.0, 0.0}, xm = dbl2{0.0, 0.0};
-        if (ok) trace_species(t, pr, xp, xm);
-        lds_s[pr][tid] = xm;
-        xpv[pr] = xp;
-    }
-    __syncthreads();
-    if (fx) {
-#pragma unroll
-        for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-            const dbl2 xl = useL ? lds_s[pr][below] : dbl2{0.0, 0.0};
-            const dbl2 xr = useR ? xpv[pr] : dbl2{0.0, 0.0};
-            const double gx0 = o.fpl * xl.x + o.fmr * xr.x;
-            const double gx1 = o.fpl * xl.y + o.fmr * xr.y;
-            SP2(XF, pr, t.ep) = dbl2{o.f_rho * gx0, o.f_rho * gx1};
-        }
-    }
+    // cells pos - 1 and pos: tile offsets 1 and 2 from the thread's row
+    riemann_hydro(L, fp, tile[FQ_C * QTILE + self + sr], tile[FQ_C * QTILE + self + 2 * sr],
+                  tile[FQ_G * QTILE + self + sr], tile[FQ_G * QTILE + self + 2 * sr], o);
+    store_tflux_h(x.FD[d], I, eidx(I, i, j, k), d, o);
 }
 
 // trans1 (Source/trans.F90:14-243) of the t-face states by the d-flux, then
@@ -541,14 +480,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void K
             // only faces of the extended array (the brick may reach past it)
             if (gx < -1 || gx > I.n[0] || gy < -1 || gy > I.n[1] || gz < I.zlo - 1 || gz > I.zlo + I.zn) continue;
             const idx_t ge = eidx(I, gx, gy, gz);
-            const dbl2 a = EF2(FDd, I, NFF, FF_RHO, ge), b = EF2(FDd, I, NFF, FF_MY, ge), cc = EF2(FDd, I, NFF, FF_E, ge);
-            ftile[e] = a.x;
-            ftile[nT + e] = a.y;
-            ftile[2 * nT + e] = b.x;
-            ftile[3 * nT + e] = b.y;
-            ftile[4 * nT + e] = cc.x;
-            ftile[5 * nT + e] = cc.y;
-            ftile[6 * nT + e] = EF(FDd, I, NFF, FF_GU, ge);
+            double v[UEDEN + 1], gp, gu;
+            load_tflux_h(FDd, I, ge, v, gp, gu);
+#pragma unroll
+            for (int n = 0; n <= UEDEN; ++n) ftile[n * nT + e] = v[n];
+            ftile[5 * nT + e] = gp;
+            ftile[6 * nT + e] = gu;
         }
     }
     __syncthreads();
@@ -564,18 +501,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void K
         gu = ftile[6 * nT + q];
     };
     const idx_t e = eidx(I, i, j, k);
-    const int et[3] = {t == 0, t == 1, t == 2}, ed[3] = {d == 0, d == 1, d == 2};
     const double cdtdx = x.dt_cur[m] / I.dx[d];
     const double cdt = cdtdx / 3.0;
     FaceH side[2];
-    idx_t el[2], er[2];
-    double rho[2], rrnew[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const int sh = s - 1;  // -1: minus state (zone t-1), 0: plus state (zone t)
-        const int il = i + sh * et[0], jl = j + sh * et[1], kl = k + sh * et[2];
-        el[s] = eidx(I, il, jl, kl);
-        er[s] = eidx(I, il + ed[0], jl + ed[1], kl + ed[2]);
+        const int il = i + sh * et0, jl = j + sh * et1, kl = k + sh * et2;
         QInH lq;
         load_qin_h(s == 0 ? x.SM[t] : x.SP[t], I, e, lq);
         double fr[UEDEN + 1], fl[UEDEN + 1], pgp, ugp, pgm, ugm;
@@ -584,38 +516,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void K
         const int ql = (ti + s * et0) + Tx * ((tj + s * et1) + Ty * (tk + s * et2));
         tile_tflux(ql + (ed0 + Tx * (ed1 + Ty * ed2)), fr, pgp, ugp);
         tile_tflux(ql, fl, pgm, ugm);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, il, jl, kl));
+        const double gamc = WA(x.Q, I, NFQ, FQ_G, widx(I, il, jl, kl));
         const QStateH o = trans1_hydro(lq, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt);
-        rho[s] = lq.rho;
-        rrnew[s] = lq.rho - cdt * (fr[URHO] - fl[URHO]);
         side[s] = to_face(o, t);
     }
     RiemannH o;
     face_riemann_h(x, I, t, i, j, k, side[0], side[1], o);
-    double *F = x.FT[combo], *FDd = x.FD[d];
-    store_tflux_h(F, I, e, t, o);
-    // only the side(s) with a nonzero Riemann weight are corrected and read;
-    // species go in pairs (SP2)
-    const bool useL = o.fpl != 0.0, useR = o.fmr != 0.0;
-    const SpeciesPairs XL = species_pairs(x.SM[t], I, NFS, FS_X), XR = species_pairs(x.SP[t], I, NFS, FS_X),
-                       XD = species_pairs(FDd, I, NFF, FF_X), XF = species_pairs(F, I, NFF, FF_X);
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const bool two = 2 * pr + 1 < NSPEC;  // the last pair holds one species
-        double x0[2] = {0.0, 0.0}, x1[2] = {0.0, 0.0};
-        if (useL) {
-            const dbl2 s = SP2(XL, pr, e), fr = SP2(XD, pr, er[0]), fl = SP2(XD, pr, el[0]);
-            x0[0] = trans1_species(rho[0], s.x, fr.x, fl.x, cdt, rrnew[0]);
-            if (two) x0[1] = trans1_species(rho[0], s.y, fr.y, fl.y, cdt, rrnew[0]);
-        }
-        if (useR) {
-            const dbl2 s = SP2(XR, pr, e), fr = SP2(XD, pr, er[1]), fl = SP2(XD, pr, el[1]);
-            x1[0] = trans1_species(rho[1], s.x, fr.x, fl.x, cdt, rrnew[1]);
-            if (two) x1[1] = trans1_species(rho[1], s.y, fr.y, fl.y, cdt, rrnew[1]);
-        }
-        SP2(XF, pr, e) = dbl2{o.f_rho * (o.fpl * x0[0] + o.fmr * x1[0]),
-                                            two ? o.f_rho * (o.fpl * x0[1] + o.fmr * x1[1]) : 0.0};
-    }
+    store_tflux_h(x.FT[combo], I, e, t, o);
 }
 
 // K_trans1 by cells: the thread of cell c (bricks elongated along the
@@ -624,20 +531,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void K
 // of t-face c + 1, with the d-fluxes on its cell's two d-faces, which it
 // reads once for both (K_trans1 reads them once per face side).  The minus
 // side goes through LDS to the thread above, which solves the Riemann
-// problem on its t-face as K_trans1 does.  Species: a face's weights decide
-// which sides it reads (the minus side's thread learns it through LDS), and
-// the corrected minus-side species follow pair by pair through LDS.
+// problem on its t-face as K_trans1 does.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K_trans1c(Plan3 p3, Ctx x)
 {
-    // the minus sides' hydro part, then (after the barrier that ends its
-    // reads) their species in the same memory
-    __shared__ union {
-        FaceH h[256];
-        dbl2 s[NSPEC_PAIRS][256];
-    } lds;
-    __shared__ unsigned char lds_f[256];
-    FaceH(&lds_h)[256] = lds.h;
-    dbl2(&lds_s)[NSPEC_PAIRS][256] = lds.s;
+    __shared__ FaceH lds_h[256];  // the minus sides
     int lb = logical_block(), combo;
     if (gridDim.y > 1) {
         combo = blockIdx.y;
@@ -666,151 +563,68 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
     const double cdtdx = x.dt_cur[m] / I.dx[d];
     const double cdt = cdtdx / 3.0;
     double *F = x.FT[combo], *FDd = x.FD[d];
-    const SpeciesPairs XL = species_pairs(x.SM[t], I, NFS, FS_X), XR = species_pairs(x.SP[t], I, NFS, FS_X),
-                       XD = species_pairs(FDd, I, NFF, FF_X), XF = species_pairs(F, I, NFF, FF_X);
     FaceH side_p;
-    double rho_p = 0.0, rrnew_p = 0.0, rho_m = 0.0, rrnew_m = 0.0;
     if (has_p || has_m) {
         double fr[UEDEN + 1], fl[UEDEN + 1], pgp, ugp, pgm, ugm;
         load_tflux_h(FDd, I, fr_i, fr, pgp, ugp);
         load_tflux_h(FDd, I, fl_i, fl, pgm, ugm);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, i, j, k));
+        const double gamc = WA(x.Q, I, NFQ, FQ_G, widx(I, i, j, k));
         if (has_m) {
             QInH lq;
             load_qin_h(x.SM[t], I, em, lq);
             const QStateH o = trans1_hydro(lq, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt);
-            rho_m = lq.rho;
-            rrnew_m = lq.rho - cdt * (fr[URHO] - fl[URHO]);
             lds_h[tid] = to_face(o, t);
         }
         if (has_p) {
             QInH lq;
             load_qin_h(x.SP[t], I, ep, lq);
             const QStateH o = trans1_hydro(lq, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt);
-            rho_p = lq.rho;
-            rrnew_p = lq.rho - cdt * (fr[URHO] - fl[URHO]);
             side_p = to_face(o, t);
         }
     }
     __syncthreads();
+    if (!has_p) return;
     RiemannH o;
-    bool useL = false, useR = false;
-    if (has_p) {
-        face_riemann_h(x, I, t, i, j, k, lds_h[below_of(tid, st)], side_p, o);
-        store_tflux_h(F, I, ep, t, o);
-        useL = o.fpl != 0.0;
-        useR = o.fmr != 0.0;
-    }
-    lds_f[tid] = useL;
-    __syncthreads();
-    const bool need_m = has_m && lds_f[tid + st];  // the face above reads this minus side
-    // every pair's corrected species first (the minus side to LDS, the plus
-    // side kept), so that their loads are in flight together; one barrier
-    dbl2 xpv[NSPEC_PAIRS];
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const bool two = 2 * pr + 1 < NSPEC;  // the last pair holds one species
-        double xm[2] = {0.0, 0.0}, xp[2] = {0.0, 0.0};
-        if (need_m || useR) {
-            const dbl2 fr = SP2(XD, pr, fr_i), fl = SP2(XD, pr, fl_i);
-            if (need_m) {
-                const dbl2 s = SP2(XL, pr, em);
-                xm[0] = trans1_species(rho_m, s.x, fr.x, fl.x, cdt, rrnew_m);
-                if (two) xm[1] = trans1_species(rho_m, s.y, fr.y, fl.y, cdt, rrnew_m);
-            }
-            if (useR) {
-                const dbl2 s = SP2(XR, pr, ep);
-                xp[0] = trans1_species(rho_p, s.x, fr.x, fl.x, cdt, rrnew_p);
-                if (two) xp[1] = trans1_species(rho_p, s.y, fr.y, fl.y, cdt, rrnew_p);
-            }
-        }
-        lds_s[pr][tid] = dbl2{xm[0], xm[1]};
-        xpv[pr] = dbl2{xp[0], xp[1]};
-    }
-    __syncthreads();
-    if (has_p) {
-#pragma unroll
-        for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-            const bool two = 2 * pr + 1 < NSPEC;
-            const dbl2 x0 = useL ? lds_s[pr][below_of(tid, st)] : dbl2{0.0, 0.0};
-            SP2(XF, pr, ep) = dbl2{o.f_rho * (o.fpl * x0.x + o.fmr * xpv[pr].x),
-                                   two ? o.f_rho * (o.fpl * x0.y + o.fmr * xpv[pr].y) : 0.0};
-        }
-    }
+    face_riemann_h(x, I, t, i, j, k, lds_h[below_of(tid, st)], side_p, o);
+    store_tflux_h(F, I, ep, t, o);
 }
 
 // The artificial viscosity of d-face (i,j,k) and the hydro part of its final
 // flux (apply_av, Source/Castro_hydro_nd.F90:174-245, with the reference's
-// corner-node pattern): stores the conserved fluxes and the Godunov p of
-// face e and returns what the species fluxes need.
-struct FinalAV {
-    double div1, dxd, frho;
-    idx_t cr, cl;
-};
-__device__ __forceinline__ FinalAV final_hydro(const Ctx &x, const FInst &I, int d, int i, int j, int k, idx_t e,
-                                               const RiemannH &o)
+// corner-node pattern): stores the conserved fluxes and Godunov p, u of face
+// e and what the species fluxes need (K_species).
+__device__ __forceinline__ void final_hydro(const Ctx &x, const FInst &I, int d, int i, int j, int k, idx_t e,
+                                            const RiemannH &o)
 {
-    FinalAV v;
     double div1;
 #define DVN(a, b, cc) EA(x.DV, I, 1, 0, eidx(I, a, b, cc))
     if (d == 0) div1 = FOURTH * (DVN(i, j, k) + DVN(i, j + 1, k) + DVN(i, j, k + 1) + DVN(i, j + 1, k));
     else if (d == 1) div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j, k + 1) + DVN(i + 1, j, k));
     else div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j + 1, k) + DVN(i + 1, j + 1, k));
 #undef DVN
-    v.div1 = 0.1 * fmin(0.0, div1);
-    v.cr = cidx(I, i, j, k);
-    v.cl = cidx(I, i - (d == 0), j - (d == 1), k - (d == 2));
-    v.dxd = I.dx[d];
-#define AVN(n, fval) ((fval) + v.dxd * (v.div1 * (CA(x.U1, I, NU1, n, v.cr) - CA(x.U1, I, NU1, n, v.cl))))
+    div1 = 0.1 * fmin(0.0, div1);
+    const idx_t cr = widx(I, i, j, k), cl = widx(I, i - (d == 0), j - (d == 1), k - (d == 2));
+    const double dxd = I.dx[d];
+#define AVN(n, fval) ((fval) + dxd * (div1 * (WA(x.U1, I, NU1, n, cr) - WA(x.U1, I, NU1, n, cl))))
     const int mn = UMX + d, mt = d == 0 ? UMY : UMX, mtt = d == 2 ? UMY : UMZ;
     double *FN = x.FN[d];
-    v.frho = AVN(URHO, o.f_rho);
     // momenta back in absolute order (mn = UMX + d, mt, mtt as above)
     const double vmn = AVN(mn, o.f_mn), vmt = AVN(mt, o.f_mt), vmtt = AVN(mtt, o.f_mtt);
     const double mx = d == 0 ? vmn : vmt;
     const double my = d == 0 ? vmt : (d == 1 ? vmn : vmtt);
     const double mz = d == 2 ? vmn : vmtt;
-    EF2(FN, I, NFN, URHO, e) = dbl2{v.frho, mx};
+    EF2(FN, I, NFN, URHO, e) = dbl2{AVN(URHO, o.f_rho), mx};
     EF2(FN, I, NFN, UMY, e) = dbl2{my, mz};
     EF2(FN, I, NFN, UEDEN, e) = dbl2{AVN(UEDEN, o.f_E), AVN(UEINT, o.f_e)};
-    EF2(FN, I, NFN, UTEMP, e) = dbl2{0.0, o.g_p};  // UTEMP, FN_GP
+    EF2(FN, I, NFN, FN_GP, e) = dbl2{o.g_p, o.g_un};
+    EF2(FN, I, NFN, FN_FR, e) = dbl2{o.f_rho, o.fpl};
+    EA(FN, I, NFN, FN_DIV, e) = div1;
 #undef AVN
-    return v;
-}
-
-// species flux of species pair pr with its artificial viscosity (the
-// corrected species x0 of the minus side, x1 of the plus side), added to
-// the running sum in species order
-__device__ __forceinline__ void final_species_pair(const FinalAV &v, const RiemannH &o, const SpeciesPairs &XU,
-                                                   int pr, const double *x0, const double *x1, double *fs,
-                                                   double &sum)
-{
-    const dbl2 ur = SP2(XU, pr, v.cr), ul = SP2(XU, pr, v.cl);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int n = 2 * pr + h;
-        if (n >= NSPEC) break;
-        const double f = o.f_rho * (o.fpl * x0[h] + o.fmr * x1[h]);
-        fs[n] = f + v.dxd * (v.div1 * ((h == 0 ? ur.x : ur.y) - (h == 0 ? ul.x : ul.y)));
-        sum = sum + fs[n];
-    }
-}
-
-// normalize_species_fluxes (Source/Castro_hydro_nd.F90:248-297) and the
-// species and Godunov-u stores of face e
-__device__ __forceinline__ void final_species_store(const SpeciesPairs &XN, double *FN, const FInst &I, idx_t e,
-                                                    const double *fs, double sum, double frho, double g_un)
-{
-    const double fac = (sum != 0.0) ? frho / sum : 1.0;
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr)
-        SP2(XN, pr, e) = dbl2{fs[2 * pr] * fac, 2 * pr + 1 < NSPEC ? fs[2 * pr + 1] * fac : 0.0};
-    EF(FN, I, NFN, FN_GU, e) = g_un;
 }
 
 // trans2 (Source/trans.F90:250-505) + final flux + apply_av
-// (Source/Castro_hydro_nd.F90:174-245) + normalize_species_fluxes (:248-297)
-// on the d-faces of the valid region.
+// (Source/Castro_hydro_nd.F90:174-245) on the d-faces of the valid region,
+// without the species.
 __global__ __launch_bounds__(256) void K_final(Plan p, Ctx x)
 {
     int m, i, j, k, sub_;
@@ -829,61 +643,28 @@ __global__ __launch_bounds__(256) void K_final(Plan p, Ctx x)
     const idx_t e = eidx(I, i, j, k);
     double *F2 = x.FT[pair_index(t1, t2)], *F3 = x.FT[pair_index(t2, t1)];
     FaceH side[2];
-    idx_t l2[2], r2[2], r3[2];
-    double rho[2], rrnew[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const int sh = s - 1;
         const int il = i + sh * ed[0], jl = j + sh * ed[1], kl = k + sh * ed[2];
-        l2[s] = eidx(I, il, jl, kl);
-        r2[s] = eidx(I, il + e1[0], jl + e1[1], kl + e1[2]);
-        r3[s] = eidx(I, il + e2[0], jl + e2[1], kl + e2[2]);
+        const idx_t l2 = eidx(I, il, jl, kl), r2 = eidx(I, il + e1[0], jl + e1[1], kl + e1[2]),
+                    r3 = eidx(I, il + e2[0], jl + e2[1], kl + e2[2]);
         QInH lq;
         load_qin_h(s == 0 ? x.SM[d] : x.SP[d], I, e, lq);
         double f2r[UEDEN + 1], f2l[UEDEN + 1], f3r[UEDEN + 1], f3l[UEDEN + 1], pg2p, ug2p, pg2m, ug2m, pg3p, ug3p,
             pg3m, ug3m;
-        load_tflux_h(F2, I, r2[s], f2r, pg2p, ug2p);
-        load_tflux_h(F2, I, l2[s], f2l, pg2m, ug2m);
-        load_tflux_h(F3, I, r3[s], f3r, pg3p, ug3p);
-        load_tflux_h(F3, I, l2[s], f3l, pg3m, ug3m);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, il, jl, kl));
+        load_tflux_h(F2, I, r2, f2r, pg2p, ug2p);
+        load_tflux_h(F2, I, l2, f2l, pg2m, ug2m);
+        load_tflux_h(F3, I, r3, f3r, pg3p, ug3p);
+        load_tflux_h(F3, I, l2, f3l, pg3m, ug3m);
+        const double gamc = WA(x.Q, I, NFQ, FQ_G, widx(I, il, jl, kl));
         const QStateH o = trans2_hydro(lq, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m, gamc,
                                        h2, h3);
-        rho[s] = lq.rho;
-        rrnew[s] = lq.rho - h2 * (f2r[URHO] - f2l[URHO]) - h3 * (f3r[URHO] - f3l[URHO]);
         side[s] = to_face(o, d);
     }
     RiemannH o;
     face_riemann_h(x, I, d, i, j, k, side[0], side[1], o);
-    double *FN = x.FN[d];
-    const SpeciesPairs XL = species_pairs(x.SM[d], I, NFS, FS_X), XR = species_pairs(x.SP[d], I, NFS, FS_X),
-                       X2 = species_pairs(F2, I, NFF, FF_X), X3 = species_pairs(F3, I, NFF, FF_X),
-                       XN = species_pairs(FN, I, NFN, FN_X);
-    const SpeciesPairs XU = cell_species(x.U1X, I);
-    const FinalAV v = final_hydro(x, I, d, i, j, k, e, o);
-    double fs[NSPEC], sum = 0.0;
-    const bool useL = o.fpl != 0.0, useR = o.fmr != 0.0;
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const bool two = 2 * pr + 1 < NSPEC;  // the last pair holds one species
-        double x0[2] = {0.0, 0.0}, x1[2] = {0.0, 0.0};
-        if (useL) {
-            const dbl2 s = SP2(XL, pr, e);
-            const dbl2 a = SP2(X2, pr, r2[0]), b = SP2(X2, pr, l2[0]);
-            const dbl2 c3 = SP2(X3, pr, r3[0]), d3 = SP2(X3, pr, l2[0]);
-            x0[0] = trans2_species(rho[0], s.x, a.x, b.x, c3.x, d3.x, h2, h3, rrnew[0]);
-            if (two) x0[1] = trans2_species(rho[0], s.y, a.y, b.y, c3.y, d3.y, h2, h3, rrnew[0]);
-        }
-        if (useR) {
-            const dbl2 s = SP2(XR, pr, e);
-            const dbl2 a = SP2(X2, pr, r2[1]), b = SP2(X2, pr, l2[1]);
-            const dbl2 c3 = SP2(X3, pr, r3[1]), d3 = SP2(X3, pr, l2[1]);
-            x1[0] = trans2_species(rho[1], s.x, a.x, b.x, c3.x, d3.x, h2, h3, rrnew[1]);
-            if (two) x1[1] = trans2_species(rho[1], s.y, a.y, b.y, c3.y, d3.y, h2, h3, rrnew[1]);
-        }
-        final_species_pair(v, o, XU, pr, x0, x1, fs, sum);
-    }
-    final_species_store(XN, FN, I, e, fs, sum, v.frho, o.g_un);
+    final_hydro(x, I, d, i, j, k, e, o);
 }
 
 // K_final by cells: the thread of cell c (bricks elongated along d,
@@ -892,19 +673,11 @@ __global__ __launch_bounds__(256) void K_final(Plan p, Ctx x)
 // with the four transverse fluxes on its cell's t1- and t2-faces, which it
 // reads once for both (K_final reads them once per face side).  The minus
 // side goes through LDS to the thread above, which solves the Riemann
-// problem on its d-face and applies the artificial viscosity and the
-// species normalisation as K_final does; species sides as in K_trans1c.
+// problem on its d-face and applies the artificial viscosity as K_final
+// does.
 __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
 {
-    // the minus sides' hydro part, then (after the barrier that ends its
-    // reads) their species in the same memory
-    __shared__ union {
-        FaceH h[256];
-        dbl2 s[NSPEC_PAIRS][256];
-    } lds;
-    __shared__ unsigned char lds_f[256];
-    FaceH(&lds_h)[256] = lds.h;
-    dbl2(&lds_s)[NSPEC_PAIRS][256] = lds.s;
+    __shared__ FaceH lds_h[256];  // the minus sides
     int lb = logical_block(), d;
     if (gridDim.y > 1) {
         d = blockIdx.y;
@@ -932,13 +705,8 @@ __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
     const idx_t l2 = ep, r2 = eidx(I, i + (t1 == 0), j + (t1 == 1), k), r3 = eidx(I, i, j + (t2 == 1), k + (t2 == 2));
     const double dt = x.dt_cur[m];
     const double h2 = 0.5 * dt / I.dx[t1], h3 = 0.5 * dt / I.dx[t2];
-    double *F2 = x.FT[pair_index(t1, t2)], *F3 = x.FT[pair_index(t2, t1)], *FN = x.FN[d];
-    const SpeciesPairs XL = species_pairs(x.SM[d], I, NFS, FS_X), XR = species_pairs(x.SP[d], I, NFS, FS_X),
-                       X2 = species_pairs(F2, I, NFF, FF_X), X3 = species_pairs(F3, I, NFF, FF_X),
-                       XN = species_pairs(FN, I, NFN, FN_X);
-    const SpeciesPairs XU = cell_species(x.U1X, I);
+    double *F2 = x.FT[pair_index(t1, t2)], *F3 = x.FT[pair_index(t2, t1)];
     FaceH side_p;
-    double rho_p = 0.0, rrnew_p = 0.0, rho_m = 0.0, rrnew_m = 0.0;
     if (has_p || has_m) {
         double f2r[UEDEN + 1], f2l[UEDEN + 1], f3r[UEDEN + 1], f3l[UEDEN + 1], pg2p, ug2p, pg2m, ug2m, pg3p, ug3p,
             pg3m, ug3m;
@@ -946,14 +714,12 @@ __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
         load_tflux_h(F2, I, l2, f2l, pg2m, ug2m);
         load_tflux_h(F3, I, r3, f3r, pg3p, ug3p);
         load_tflux_h(F3, I, l2, f3l, pg3m, ug3m);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, i, j, k));
+        const double gamc = WA(x.Q, I, NFQ, FQ_G, widx(I, i, j, k));
         if (has_m) {
             QInH lq;
             load_qin_h(x.SM[d], I, em, lq);
             const QStateH o = trans2_hydro(lq, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m,
                                            gamc, h2, h3);
-            rho_m = lq.rho;
-            rrnew_m = lq.rho - h2 * (f2r[URHO] - f2l[URHO]) - h3 * (f3r[URHO] - f3l[URHO]);
             lds_h[tid] = to_face(o, d);
         }
         if (has_p) {
@@ -961,59 +727,14 @@ __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
             load_qin_h(x.SP[d], I, ep, lq);
             const QStateH o = trans2_hydro(lq, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m,
                                            gamc, h2, h3);
-            rho_p = lq.rho;
-            rrnew_p = lq.rho - h2 * (f2r[URHO] - f2l[URHO]) - h3 * (f3r[URHO] - f3l[URHO]);
             side_p = to_face(o, d);
         }
     }
     __syncthreads();
+    if (!has_p) return;
     RiemannH o;
-    FinalAV v;
-    bool useL = false, useR = false;
-    if (has_p) {
-        face_riemann_h(x, I, d, i, j, k, lds_h[below_of(tid, st)], side_p, o);
-        v = final_hydro(x, I, d, i, j, k, ep, o);
-        useL = o.fpl != 0.0;
-        useR = o.fmr != 0.0;
-    }
-    lds_f[tid] = useL;
-    __syncthreads();
-    const bool need_m = has_m && lds_f[tid + st];  // the face above reads this minus side
-    // every pair's corrected species first (the minus side to LDS, the plus
-    // side kept), so that their loads are in flight together; one barrier
-    dbl2 xpv[NSPEC_PAIRS];
-#pragma unroll
-    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-        const bool two = 2 * pr + 1 < NSPEC;  // the last pair holds one species
-        double xm[2] = {0.0, 0.0}, xp[2] = {0.0, 0.0};
-        if (need_m || useR) {
-            const dbl2 a = SP2(X2, pr, r2), b = SP2(X2, pr, l2);
-            const dbl2 c3 = SP2(X3, pr, r3), d3 = SP2(X3, pr, l2);
-            if (need_m) {
-                const dbl2 s = SP2(XL, pr, em);
-                xm[0] = trans2_species(rho_m, s.x, a.x, b.x, c3.x, d3.x, h2, h3, rrnew_m);
-                if (two) xm[1] = trans2_species(rho_m, s.y, a.y, b.y, c3.y, d3.y, h2, h3, rrnew_m);
-            }
-            if (useR) {
-                const dbl2 s = SP2(XR, pr, ep);
-                xp[0] = trans2_species(rho_p, s.x, a.x, b.x, c3.x, d3.x, h2, h3, rrnew_p);
-                if (two) xp[1] = trans2_species(rho_p, s.y, a.y, b.y, c3.y, d3.y, h2, h3, rrnew_p);
-            }
-        }
-        lds_s[pr][tid] = dbl2{xm[0], xm[1]};
-        xpv[pr] = dbl2{xp[0], xp[1]};
-    }
-    __syncthreads();
-    if (has_p) {
-        double fs[NSPEC], sum = 0.0;
-#pragma unroll
-        for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-            const dbl2 x0v = useL ? lds_s[pr][below_of(tid, st)] : dbl2{0.0, 0.0};
-            const double x0[2] = {x0v.x, x0v.y}, x1[2] = {xpv[pr].x, xpv[pr].y};
-            final_species_pair(v, o, XU, pr, x0, x1, fs, sum);
-        }
-        final_species_store(XN, FN, I, ep, fs, sum, v.frho, o.g_un);
-    }
+    face_riemann_h(x, I, d, i, j, k, lds_h[below_of(tid, st)], side_p, o);
+    final_hydro(x, I, d, i, j, k, ep, o);
 }
 
 // fill_hydro_source (Source/Castro_hydro_nd.F90:344-441), Saxpy and the two
@@ -1047,25 +768,51 @@ __device__ __forceinline__ void update_cells(Plan p, Ctx x)
         double u[NVAR];
 #pragma unroll
         for (int n = 0; n < NVAR; ++n) u[n] = CA(x.U, I, NVAR, n, c);  // clean(S_old), stored by K_prim
+        // the species fluxes of the six faces with their normalisation
+        // (Source/Castro_hydro_nd.F90:248-297)
+        {
+            const SpeciesPairs P[3] = {P0, P1, P2};
+            double *FN[3] = {F0, F1, F2};
+            const idx_t eh[3] = {ex, ey, ez};
+            dbl2 f[3][2][NSPEC_PAIRS];
 #pragma unroll
-        for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-            const dbl2 f0 = SP2(P0, pr, e), f0x = SP2(P0, pr, ex), f1 = SP2(P1, pr, e), f1y = SP2(P1, pr, ey),
-                       f2 = SP2(P2, pr, e), f2z = SP2(P2, pr, ez);
-            const int n = UFS + 2 * pr;
-            u[n] = u[n] + dt * flux_div(f0.x, f0x.x, f1.x, f1y.x, f2.x, f2z.x, a0, a1, a2, volinv);
-            if (n + 1 < NVAR) u[n + 1] = u[n + 1] + dt * flux_div(f0.y, f0x.y, f1.y, f1y.y, f2.y, f2z.y, a0, a1, a2, volinv);
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int hi = 0; hi < 2; ++hi) {
+                    const idx_t ee = hi ? eh[d] : e;
+                    double sum = 0.0;
+#pragma unroll
+                    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+                        f[d][hi][pr] = SP2(P[d], pr, ee);
+                        sum = sum + f[d][hi][pr].x;
+                        if (2 * pr + 1 < NSPEC) sum = sum + f[d][hi][pr].y;
+                    }
+                    const double fac = (sum != 0.0) ? EF(FN[d], I, NFN, URHO, ee) / sum : 1.0;
+#pragma unroll
+                    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+                        f[d][hi][pr].x = f[d][hi][pr].x * fac;
+                        f[d][hi][pr].y = f[d][hi][pr].y * fac;
+                    }
+                }
+#pragma unroll
+            for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+                const int n = UFS + 2 * pr;
+                u[n] = u[n] + dt * flux_div(f[0][0][pr].x, f[0][1][pr].x, f[1][0][pr].x, f[1][1][pr].x, f[2][0][pr].x,
+                                            f[2][1][pr].x, a0, a1, a2, volinv);
+                if (n + 1 < NVAR)
+                    u[n + 1] = u[n + 1] + dt * flux_div(f[0][0][pr].y, f[0][1][pr].y, f[1][0][pr].y, f[1][1][pr].y,
+                                                        f[2][0][pr].y, f[2][1][pr].y, a0, a1, a2, volinv);
+            }
         }
-        // URHO..UTEMP and FN_GP as the four pairs (0,1) (2,3) (4,5) (6,7) of
-        // the six faces; the last pair (UTEMP, Godunov p) first, for p div u
+        // URHO..UEINT as the three pairs (0,1) (2,3) (4,5) of the six faces,
+        // and the pair of Godunov p and u for p div u; UTEMP has no flux
         double pdivu;
         {
-            const dbl2 g0 = EF2(F0, I, NFN, UTEMP, e), g0x = EF2(F0, I, NFN, UTEMP, ex), g1 = EF2(F1, I, NFN, UTEMP, e),
-                       g1y = EF2(F1, I, NFN, UTEMP, ey), g2 = EF2(F2, I, NFN, UTEMP, e),
-                       g2z = EF2(F2, I, NFN, UTEMP, ez);
-            u[UTEMP] = u[UTEMP] + dt * flux_div(g0.x, g0x.x, g1.x, g1y.x, g2.x, g2z.x, a0, a1, a2, volinv);
-            pdivu = HALF * (g0x.y + g0.y) * (EF(F0, I, NFN, FN_GU, ex) - EF(F0, I, NFN, FN_GU, e)) / dx0 +
-                    HALF * (g1y.y + g1.y) * (EF(F1, I, NFN, FN_GU, ey) - EF(F1, I, NFN, FN_GU, e)) / dx1 +
-                    HALF * (g2z.y + g2.y) * (EF(F2, I, NFN, FN_GU, ez) - EF(F2, I, NFN, FN_GU, e)) / dx2;
+            const dbl2 g0 = EF2(F0, I, NFN, FN_GP, e), g0x = EF2(F0, I, NFN, FN_GP, ex), g1 = EF2(F1, I, NFN, FN_GP, e),
+                       g1y = EF2(F1, I, NFN, FN_GP, ey), g2 = EF2(F2, I, NFN, FN_GP, e),
+                       g2z = EF2(F2, I, NFN, FN_GP, ez);
+            pdivu = HALF * (g0x.x + g0.x) * (g0x.y - g0.y) / dx0 + HALF * (g1y.x + g1.x) * (g1y.y - g1.y) / dx1 +
+                    HALF * (g2z.x + g2.x) * (g2z.y - g2.y) / dx2;
         }
 #pragma unroll
         for (int n = 0; n < UTEMP; n += 2) {
@@ -1180,10 +927,8 @@ static std::vector<int> step_stages(const FusedLevel *F)
     return v;
 }
 
-// the cell stages before and after the face stages of a step (estdt,
-// K_prim) run over whole instances; the face stages and K_update run slab
-// by slab
-static bool whole_instance_stage(int stage) { return stage == ST_EST || stage == ST_PRIM; }
+// estdt runs over whole instances, every other stage slab by slab
+static bool whole_instance_stage(int stage) { return stage == ST_EST; }
 
 // brick of an overlapping stage's direction d for its tiling (W, L, X)
 static KernelTiling ovl_brick(const KernelTiling &t, int d)
@@ -1203,12 +948,12 @@ static bool ovl_tiling_ok(const KernelTiling &t)
 
 // block table of a brick tiling t over the range (shift, add) of a slab;
 // ovl >= 0: the bricks overlap along that direction (plan_cell_ovl)
-static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int slab, int ovl)
+static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int slab, int ovl, bool prim = false)
 {
-    const FInst *tab = slab < 0 ? F->inst : F->sinst[slab];
+    const FInst *tab = slab < 0 ? F->inst : (prim ? F->pinst[slab] : F->sinst[slab]);
     for (auto &pb : F->plans)
         if (pb.t.bx == t.bx && pb.t.by == t.by && pb.t.bz == t.bz && pb.t.zg == t.zg && pb.shift == sh &&
-            pb.add == add && pb.slab == slab && pb.ovl == ovl)
+            pb.add == add && pb.slab == slab && pb.ovl == ovl && pb.prim == prim)
             return Plan{tab, pb.blk0, F->ninst, t.bx, t.by, t.bz, sh, add, t.zg};
     FusedLevel::PlanBuf pb;
     pb.t = t;
@@ -1216,7 +961,8 @@ static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int 
     pb.add = add;
     pb.slab = slab;
     pb.ovl = ovl;
-    const std::vector<FInst> &hs = slab < 0 ? F->hinst : F->hsinst[slab];
+    pb.prim = prim;
+    const std::vector<FInst> &hs = slab < 0 ? F->hinst : (prim ? F->hpinst[slab] : F->hsinst[slab]);
     std::vector<int> b0(F->ninst + 1);
     const int bb[3] = {t.bx, t.by, t.bz};
     int acc = 0;
@@ -1245,7 +991,7 @@ static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int 
 Plan get_plan(FusedLevel *F, int stage, int slab)
 {
     if (whole_instance_stage(stage)) slab = -1;
-    return plan_for(F, F->tiling[stage], stage_shift[stage], stage_add[stage], slab, -1);
+    return plan_for(F, F->tiling[stage], stage_shift[stage], stage_add[stage], slab, -1, stage == ST_PRIM);
 }
 
 // K_trans1's LDS for a brick: its d-flux tile (the brick widened by one cell
@@ -1274,6 +1020,70 @@ static Plan3 get_plan3(FusedLevel *F, int stage, int slab)
     return q;
 }
 
+#ifndef SPEC_LZMAX
+#define SPEC_LZMAX 64
+#endif
+// tiles of the species stage over an instance's columns, times the pairs
+static int spec_tiles(const FInst &I)
+{
+    return ((I.n[0] + SPEC_TX - 3) / (SPEC_TX - 2)) * ((I.n[1] + SPEC_TY - 3) / (SPEC_TY - 2)) * NSPEC_PAIRS;
+}
+
+// Planes per chunk of the species stage: a chunk marches through its planes
+// and two more, so long chunks waste least, but a launch takes as many rounds
+// of a chunk as its blocks need of the chip's CUs.  Two blocks share a CU and
+// take 1.4 times as long as one alone (256^3: 3.5 us a plane of each CU with
+// two, 5 us with one); the candidate with the least total is taken.
+static int spec_chunk(const std::vector<FInst> &inst)
+{
+    constexpr double cus = 256.0;
+    int zmax = 0, best = 1;
+    for (const FInst &I : inst) zmax = std::max(zmax, I.zn);
+    double tbest = 1e300;
+    for (int lz = 1; lz <= std::min(zmax, SPEC_LZMAX); ++lz) {
+        long blocks = 0;
+        for (const FInst &I : inst)
+            if (I.zn > 0) blocks += (long)spec_tiles(I) * ((I.zn + lz - 1) / lz);
+        const double rounds = blocks <= cus ? 1.4 : (double)std::max(2.0, ceil(blocks / cus));
+        const double t = rounds * (lz + 2.5);
+        if (t < tbest) {
+            tbest = t;
+            best = lz;
+        }
+    }
+    return best;
+}
+
+// block table of the species stage over a slab
+static SpecPlan spec_plan(FusedLevel *F, int slab, int &nblocks)
+{
+    const FInst *tab = F->sinst[slab];
+    for (auto &sb : F->specs)
+        if (sb.slab == slab) {
+            nblocks = sb.nblocks;
+            return SpecPlan{tab, sb.blk0, F->ninst, sb.lz};
+        }
+    FusedLevel::SpecBuf sb;
+    sb.slab = slab;
+    sb.lz = spec_chunk(F->hsinst[slab]);
+    std::vector<int> b0(F->ninst + 1);
+    int acc = 0;
+    for (int m = 0; m < F->ninst; ++m) {
+        b0[m] = acc;
+        const FInst &I = F->hsinst[slab][m];
+        if (I.zn > 0) acc += spec_tiles(I) * ((I.zn + sb.lz - 1) / sb.lz);
+    }
+    b0[F->ninst] = acc;
+    nblocks = sb.nblocks = acc;
+    if (check_hip(hipMalloc(&sb.blk0, sizeof(int) * (F->ninst + 1)), "hipMalloc(species plan)") ||
+        check_hip(hipMemcpy(sb.blk0, b0.data(), sizeof(int) * (F->ninst + 1), hipMemcpyHostToDevice), "plan h2d")) {
+        nblocks = 0;
+        return SpecPlan{nullptr, nullptr, 0, 0};
+    }
+    F->specs.push_back(sb);
+    return SpecPlan{tab, sb.blk0, F->ninst, sb.lz};
+}
+
 int plan_blocks(FusedLevel *F, const Plan &p)
 {
     for (auto &pb : F->plans)
@@ -1287,6 +1097,14 @@ using namespace mc;
 
 namespace mc {
 
+static void launch_species(FusedLevel *F, hipStream_t s, int slab)
+{
+    int nb = 0;
+    const SpecPlan p = spec_plan(F, slab, nb);
+    if (nb > 0)
+        hipLaunchKernelGGL(K_species, dim3(nb), dim3(SPEC_TX * SPEC_TY), 0, s, p, F->ctx);
+}
+
 static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, int slab = 0)
 {
     F->ctx.tab = eos_table();
@@ -1299,7 +1117,10 @@ static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, in
         const KernelTiling &t = F->tiling[stage];
         if (stage == ST_TFLUX) hipLaunchKernelGGL(K_tflux, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
         else if (stage == ST_TRANS1C) hipLaunchKernelGGL(K_trans1c, dim3(6 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
-        else hipLaunchKernelGGL(K_finalc, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
+        else {
+            hipLaunchKernelGGL(K_finalc, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
+            launch_species(F, s, slab);
+        }
         return;
     }
     Plan p = get_plan(F, stage, slab);
@@ -1314,12 +1135,24 @@ static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, in
     dim3 g(interleave ? nb * ny : nb, interleave ? 1 : ny), b(nt);
     switch (stage) {
     case ST_EST: hipLaunchKernelGGL(K_est, g, b, 0, s, p, F->ctx); break;
-    case ST_PRIM: hipLaunchKernelGGL(K_prim, g, b, 0, s, p, F->ctx); break;
+    case ST_PRIM:
+        if (F->slab) {
+            if (slab == 0)  // the boundary planes the step's images are made from
+                hipLaunchKernelGGL(K_save_planes, dim3((unsigned)((F->totP + 255) / 256)), dim3(256), 0, s, F->inst,
+                                   F->ninst, F->totP, F->ctx);
+            hipLaunchKernelGGL(K_prim<true>, g, b, 0, s, p, F->ctx);
+        } else {
+            hipLaunchKernelGGL(K_prim<false>, g, b, 0, s, p, F->ctx);
+        }
+        break;
     case ST_FLAT: hipLaunchKernelGGL(K_flat, g, b, 0, s, p, F->ctx); break;
     case ST_TRACE: hipLaunchKernelGGL(K_trace, g, b, 0, s, p, F->ctx); break;
     case ST_FLUX1: hipLaunchKernelGGL(K_flux1, g, b, 0, s, p, F->ctx); break;
     case ST_TRANS1: hipLaunchKernelGGL(K_trans1, g, b, trans1_tile_bytes(p.bx, p.by, p.bz), s, p, F->ctx); break;
-    case ST_FINAL: hipLaunchKernelGGL(K_final, g, b, 0, s, p, F->ctx); break;
+    case ST_FINAL:
+        hipLaunchKernelGGL(K_final, g, b, 0, s, p, F->ctx);
+        launch_species(F, s, slab);
+        break;
     case ST_UPDATE:
         if (F->defer_post) hipLaunchKernelGGL(K_update_adv, g, b, 0, s, p, F->ctx);
         else hipLaunchKernelGGL(K_update, g, b, 0, s, p, F->ctx);
@@ -1342,7 +1175,7 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     // face stages over whole instances
     F->slab = (slab > 0 && slab < nzmax) ? slab : 0;
     F->nslab = F->slab ? (nzmax + F->slab - 1) / F->slab : 1;
-    long offD = 0, offE = 0, offQ = 0;
+    long offD = 0, offE = 0, offQ = 0, offW = 0, offP = 0;
     for (const auto &sp : spec) {
         FInst I;
         for (int d = 0; d < 3; ++d) {
@@ -1367,13 +1200,32 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
             delete F;
             return nullptr;
         }
-        I.nQ = I.nD + (I.nD & 1);  // even, like nE
+        const int wR = F->slab ? std::min(F->slab, sp.n[2]) + 2 * WHALO : sp.n[2];
+        I.nW = (long)I.n[0] * I.n[1] * wR;
+        I.nQ = I.nW + (I.nW & 1);  // even, like nE
+        I.offW = offW;
+        I.offP = offP;
+        I.wwrap = I.periodic;
+        I.wlo = 0;
+        I.whi = sp.n[2] - 1;
+        I.wz = 0;
+        I.wR = 1 << 30;
+        if (F->slab) {  // images of a periodic instance have planes of their own
+            I.wwrap = 0;
+            if (I.periodic) {
+                I.wlo = -(1 << 29);
+                I.whi = 1 << 29;
+            }
+            I.wR = wR;
+            offP += (long)I.n[0] * I.n[1] * 2 * WHALO;
+        }
         I.offD = offD;
         I.offE = offE;
         I.offQ = offQ;
         offD += I.nD;
         offE += I.nE;
         offQ += I.nQ;
+        offW += I.nW;
         F->hinst.push_back(I);
     }
     // one instance table per slab: cells [s * slab, (s + 1) * slab) in z,
@@ -1383,23 +1235,47 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
         for (FInst &I : F->hsinst[sl]) {
             I.zlo = sl * F->slab;
             I.zn = std::max(0, std::min(F->slab, I.n[2] - I.zlo));
+            // the ring holds planes [zlo - WHALO, zlo + zn + WHALO), plane k in
+            // slot k mod wR
+            const int first = I.zlo - WHALO;
+            I.wz = first - ((first % I.wR) + I.wR) % I.wR;
+        }
+    // K_prim of slab sl adds the planes up to WHALO above it
+    F->hpinst = F->hsinst;
+    if (F->slab)
+        for (int m = 0; m < F->ninst; ++m) {
+            const FInst &H = F->hinst[m];
+            int k0 = H.periodic ? -WHALO : 0;
+            const int top = H.periodic ? H.n[2] + WHALO : H.n[2];
+            for (int sl = 0; sl < F->nslab; ++sl) {
+                FInst &I = F->hpinst[sl][m];
+                const int k1 = I.zn > 0 ? std::min(I.zlo + I.zn + WHALO, top) : k0;
+                I.zlo = k0;
+                I.zn = std::max(0, k1 - k0);
+                k0 = std::max(k0, k1);
+            }
         }
     F->totD = offD;
     F->totE = offE;
     F->totQ = offQ;
+    F->totW = offW;
+    F->totP = offP;
     for (int s = 0; s < NSTAGE; ++s) F->tiling[s] = KernelTiling{64, 2, 2};
     F->tiling[ST_EST] = F->tiling[ST_PRIM] = F->tiling[ST_UPDATE] = KernelTiling{64, 4, 1};
     F->tiling[ST_TFLUX] = F->tiling[ST_TRANS1C] = F->tiling[ST_FINALC] = KernelTiling{16, 16, 64};
     bool ok = !check_hip(hipMalloc(&F->inst, sizeof(FInst) * F->ninst), "hipMalloc(inst)") &&
               !check_hip(hipMemcpy(F->inst, F->hinst.data(), sizeof(FInst) * F->ninst, hipMemcpyHostToDevice), "h2d");
     F->sinst.assign(F->nslab, nullptr);
+    F->pinst.assign(F->nslab, nullptr);
     if (!F->slab) {
-        F->sinst[0] = F->inst;
+        F->sinst[0] = F->pinst[0] = F->inst;
     } else {
+        auto table = [&](FInst *&d, const std::vector<FInst> &h) {
+            return !check_hip(hipMalloc(&d, sizeof(FInst) * F->ninst), "hipMalloc(slab inst)") &&
+                   !check_hip(hipMemcpy(d, h.data(), sizeof(FInst) * F->ninst, hipMemcpyHostToDevice), "h2d");
+        };
         for (int sl = 0; sl < F->nslab && ok; ++sl)
-            ok = !check_hip(hipMalloc(&F->sinst[sl], sizeof(FInst) * F->ninst), "hipMalloc(slab inst)") &&
-                 !check_hip(hipMemcpy(F->sinst[sl], F->hsinst[sl].data(), sizeof(FInst) * F->ninst,
-                                      hipMemcpyHostToDevice), "h2d");
+            ok = table(F->sinst[sl], F->hsinst[sl]) && table(F->pinst[sl], F->hpinst[sl]);
     }
     auto A = [&](double *&p, long n) {
         if (ok && check_hip(hipMalloc(&p, sizeof(double) * std::max(n, 1L)), "hipMalloc(fused)")) ok = false;
@@ -1408,11 +1284,12 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     memset(&x, 0, sizeof(x));
     x.inst = F->inst;
     A(x.U, NVAR * offD);
-    A(x.U1, NU1 * offD);
+    A(x.U1, NU1 * offW);
     A(x.U1X, 2L * NSPEC_PAIRS * offQ);
-    A(x.Q, NFQ * offD);
-    A(x.QX, 2L * NSPEC_PAIRS * offQ);
+    A(x.Q, NFQ * offW);
+    if (F->slab) A(x.UB, NVAR * offP);
     A(x.FL, offE);
+    A(x.RW, 6 * offE);
     A(x.DV, offE);
     for (int d = 0; d < 3; ++d) {
         A(x.SM[d], NFS * offE);
@@ -1485,7 +1362,7 @@ void fused_destroy(FusedLevel *F)
     if (F->gexec) (void)hipGraphExecDestroy(F->gexec);
     if (F->graph) (void)hipGraphDestroy(F->graph);
     Ctx &x = F->ctx;
-    double *ps[] = {x.U, x.U1, x.U1X, x.Q, x.QX, x.FL, x.DV, x.dt_cur, x.dt_est, x.time};
+    double *ps[] = {x.U, x.U1, x.U1X, x.Q, x.FL, x.DV, x.RW, x.UB, x.dt_cur, x.dt_est, x.time};
     for (double *p : ps)
         if (p) (void)hipFree(p);
     for (int d = 0; d < 3; ++d) {
@@ -1498,9 +1375,14 @@ void fused_destroy(FusedLevel *F)
     if (x.steps) (void)hipFree(x.steps);
     for (auto &pb : F->plans)
         if (pb.blk0) (void)hipFree(pb.blk0);
-    if (F->slab)
+    for (auto &sb : F->specs)
+        if (sb.blk0) (void)hipFree(sb.blk0);
+    if (F->slab) {
         for (FInst *p : F->sinst)
             if (p) (void)hipFree(p);
+        for (FInst *p : F->pinst)
+            if (p) (void)hipFree(p);
+    }
     if (F->inst) (void)hipFree(F->inst);
     if (F->abox) (void)hipFree(F->abox);
     if (F->abstart) (void)hipFree(F->abstart);
@@ -1525,12 +1407,11 @@ int fused_export(FusedLevel *F, double *arena, hipStream_t s)
 
 // ---- intermediate sets
 template <class Fn>
-static void for_each_intermediate(FusedArrays &S, long totD, long totE, long totQ, Fn f)
+static void for_each_intermediate(FusedArrays &S, long totW, long totE, long totQ, Fn f)
 {
-    f(S.U1, NU1 * totD);
+    f(S.U1, NU1 * totW);
     f(S.U1X, 2L * NSPEC_PAIRS * totQ);
-    f(S.Q, NFQ * totD);
-    f(S.QX, 2L * NSPEC_PAIRS * totQ);
+    f(S.Q, NFQ * totW);
     f(S.FL, totE);
     f(S.DV, totE);
     for (int d = 0; d < 3; ++d) {
@@ -1542,23 +1423,29 @@ static void for_each_intermediate(FusedArrays &S, long totD, long totE, long tot
     for (int c = 0; c < 6; ++c) f(S.FT[c], NFF * totE);
 }
 
-// device bytes of an engine for these instances: the state, the cell arrays
-// and the face arrays (one slab deep in z when slab > 0)
+// device bytes of an engine for these instances: the state, the primitives
+// and the face arrays (a ring of planes and one slab deep in z when slab > 0)
 size_t fused_bytes_for(const std::vector<FusedInstanceSpec> &spec, int slab)
 {
-    size_t cells = 0, ext = 0, q = 0;
+    size_t cells = 0, win = 0, ext = 0, q = 0, planes = 0;
+    int nzmax = 0;
+    for (const auto &sp : spec) nzmax = std::max(nzmax, sp.n[2]);
+    if (slab >= nzmax) slab = 0;
     for (const auto &sp : spec) {
-        const long nD = (long)sp.n[0] * sp.n[1] * sp.n[2];
+        const long nxy = (long)sp.n[0] * sp.n[1], nD = nxy * sp.n[2];
         const int ez = (slab > 0 ? std::min(slab, sp.n[2]) : sp.n[2]) + 2;
+        const long nW = slab > 0 ? nxy * (ez - 2 + 2 * WHALO) : nD;
         long nE = (long)(sp.n[0] + 2) * (sp.n[1] + 2) * ez;
         nE += nE & 1;
         cells += nD;
+        win += nW;
         ext += nE;
-        q += nD + (nD & 1);
+        q += nW + (nW & 1);
+        if (slab > 0) planes += nxy * 2 * WHALO;
     }
-    const size_t per_cell = NVAR + NU1 + NFQ, per_q = 2 * 2 * NSPEC_PAIRS;
-    const size_t per_ext = 2 + 3 * (2 * NFS + NFF + NFN) + 6 * NFF;
-    return sizeof(double) * (per_cell * cells + per_q * q + per_ext * ext);
+    const size_t per_ext = 2 + 6 + 3 * (2 * NFS + NFF + NFN) + 6 * NFF;
+    return sizeof(double) *
+           (NVAR * (cells + planes) + (NU1 + NFQ) * win + 2 * NSPEC_PAIRS * q + per_ext * ext);
 }
 
 // Whole instances when their arrays take at most half the free device
@@ -1586,7 +1473,7 @@ size_t fused_intermediate_bytes(const FusedLevel *F)
 {
     FusedArrays S{};
     size_t n = 0;
-    for_each_intermediate(S, F->totD, F->totE, F->totQ, [&](double *&, long c) { n += sizeof(double) * std::max(c, 1L); });
+    for_each_intermediate(S, F->totW, F->totE, F->totQ, [&](double *&, long c) { n += sizeof(double) * std::max(c, 1L); });
     return n;
 }
 
@@ -1594,7 +1481,7 @@ int fused_alloc_intermediates(const FusedLevel *F, FusedArrays &S)
 {
     S = FusedArrays{};
     bool ok = true;
-    for_each_intermediate(S, F->totD, F->totE, F->totQ, [&](double *&p, long c) {
+    for_each_intermediate(S, F->totW, F->totE, F->totQ, [&](double *&p, long c) {
         if (ok && check_hip(hipMalloc(&p, sizeof(double) * std::max(c, 1L)), "hipMalloc(intermediates)")) ok = false;
     });
     if (!ok) fused_free_intermediates(S);
@@ -1618,7 +1505,6 @@ FusedArrays fused_get_intermediates(const FusedLevel *F)
     S.U1 = x.U1;
     S.U1X = x.U1X;
     S.Q = x.Q;
-    S.QX = x.QX;
     S.FL = x.FL;
     S.DV = x.DV;
     for (int d = 0; d < 3; ++d) {
@@ -1637,7 +1523,6 @@ void fused_set_intermediates(FusedLevel *F, const FusedArrays &S)
     x.U1 = S.U1;
     x.U1X = S.U1X;
     x.Q = S.Q;
-    x.QX = S.QX;
     x.FL = S.FL;
     x.DV = S.DV;
     for (int d = 0; d < 3; ++d) {
@@ -1672,22 +1557,21 @@ int fused_estimate(FusedLevel *F, hipStream_t s)
     return check_hip(hipGetLastError(), "fused_estimate");
 }
 
-// the face stages and the update of one z-slab
+// the primitives, the face stages and the update of one z-slab
 static void enqueue_slab(FusedLevel *F, int sl, hipStream_t s)
 {
+    launch_stage(F, ST_PRIM, s, 1, sl);
     for (int st : step_stages(F)) launch_stage(F, st, s, stage_ny[st], sl);
 }
 
-// enqueue one coarse step of every instance.  K_prim runs over whole
-// instances; then, slab after slab, the face stages and K_update: a slab's
-// update rewrites only its own cells of the state, which no later stage of
-// the step reads (the face stages read the primitives and the cleaned
-// state K_prim stored).
+// enqueue one coarse step of every instance, slab after slab: K_prim on the
+// planes the slab's face stages are the first to read, the face stages, and
+// K_update.  A slab's update rewrites only its own cells of the state, whose
+// primitives are made already and which no later stage of the step reads.
 static void enqueue_step(FusedLevel *F, double stop_time, hipStream_t s)
 {
     F->ctx.tab = eos_table();
     hipLaunchKernelGGL(K_dt, dim3(1), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
-    launch_stage(F, ST_PRIM, s);
     for (int sl = 0; sl < F->nslab; ++sl) enqueue_slab(F, sl, s);
     hipLaunchKernelGGL(K_tick, dim3(1), dim3(256), 0, s, F->ctx, F->ninst);
 }
@@ -1695,7 +1579,7 @@ static void enqueue_step(FusedLevel *F, double stop_time, hipStream_t s)
 // Eager steps with a HIP event pair around every stage launch on stream s;
 // stage_ms[st] receives the summed duration of stage st (over its slabs),
 // launches[st] the number of launches (the dt kernels are counted under
-// FST_N).
+// FST_N; K_prim counts once a step).
 int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s, double *stage_ms, int *launches)
 {
     if (!eos_ready()) {
@@ -1708,9 +1592,10 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
     const int *ny = stage_ny;
     std::vector<int> stage_of;  // stage of each timed launch of one step (NSTAGE: dt control)
     stage_of.push_back(NSTAGE);
-    stage_of.push_back(ST_PRIM);
-    for (int sl = 0; sl < F->nslab; ++sl)
+    for (int sl = 0; sl < F->nslab; ++sl) {
+        stage_of.push_back(ST_PRIM);
         for (int q = 0; q < nso; ++q) stage_of.push_back(slab_order[q]);
+    }
     const size_t per = stage_of.size();
     std::vector<hipEvent_t> ev(2 * per * (size_t)nsteps, nullptr);
     int rc = 0;
@@ -1724,14 +1609,11 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
         hipLaunchKernelGGL(K_dt, dim3(1), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
         (void)hipEventRecord(E[2 * q + 1], s);
         ++q;
-        (void)hipEventRecord(E[2 * q], s);
-        launch_stage(F, ST_PRIM, s);
-        (void)hipEventRecord(E[2 * q + 1], s);
-        ++q;
         for (int sl = 0; sl < F->nslab; ++sl)
-            for (int k = 0; k < nso; ++k, ++q) {
+            for (int k = -1; k < nso; ++k, ++q) {
+                const int st = k < 0 ? (int)ST_PRIM : slab_order[k];
                 (void)hipEventRecord(E[2 * q], s);
-                launch_stage(F, slab_order[k], s, ny[slab_order[k]], sl);
+                launch_stage(F, st, s, ny[st], sl);
                 (void)hipEventRecord(E[2 * q + 1], s);
             }
         hipLaunchKernelGGL(K_tick, dim3(1), dim3(256), 0, s, F->ctx, F->ninst);
@@ -1747,7 +1629,8 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
             float ms = 0.f;
             if (check_hip(hipEventElapsedTime(&ms, E[2 * q], E[2 * q + 1]), "hipEventElapsedTime")) rc = -1;
             stage_ms[stage_of[q]] += ms;
-            launches[stage_of[q]] += 1;
+            // K_prim's share of every slab makes one pass over the instances
+            if (stage_of[q] != ST_PRIM || q == 1) launches[stage_of[q]] += 1;
         }
     }
     for (auto &e : ev)
@@ -1777,8 +1660,10 @@ int fused_steps(FusedLevel *F, int nsteps, double stop_time, hipStream_t s, bool
         // make sure every plan table exists before capture
         for (int sl = 0; sl < F->nslab; ++sl)
             for (int st = 0; st < NSTAGE; ++st) {
+                int nb;
                 if (overlap_stage(st)) (void)get_plan3(F, st, sl);
                 else (void)get_plan(F, st, sl);
+                if (st == ST_FINAL) (void)spec_plan(F, sl, nb);
             }
         if (check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture")) return -1;
         enqueue_step(F, stop_time, s);
@@ -1801,7 +1686,6 @@ int fused_advance_dt(FusedLevel *F, double dt, hipStream_t s)
     }
     fill(F->ctx.dt_cur, F->ninst, dt, s);
     fill(F->ctx.dt_est, F->ninst, DBL_MAX, s);
-    launch_stage(F, ST_PRIM, s);
     for (int sl = 0; sl < F->nslab; ++sl) enqueue_slab(F, sl, s);
     F->have_est = true;
     return check_hip(hipGetLastError(), "fused_advance_dt");
@@ -2016,6 +1900,12 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
     auto restore_state = [&]() {
         return check_hip(hipMemcpyAsync(x.U, saveU, nU, hipMemcpyDeviceToDevice, s), "autotune restore");
     };
+    if (!rc && F->slab) {  // of the first slab, which the stages are timed on
+        rc = restore_state();
+        launch_stage(F, ST_PRIM, s);
+        for (int st : step_stages(F))
+            if (st != ST_UPDATE) launch_stage(F, st, s, ny[st]);
+    }
     // every stage of every kernel variant; the faster kernel of each
     // alternative is chosen below
     const std::vector<int> tuned = {ST_PRIM,   ST_FLAT,  ST_TRACE,  ST_FLUX1,  ST_TFLUX,

@@ -14,26 +14,33 @@ namespace mc {
 // the cleaned state U1 holds the NU1 components before the species in the
 // cell layout, its species live in their own array of pairs (Ctx::U1X)
 constexpr int NU1 = UFS;
-// primitive components of the fused path; the species of q live in their
-// own array of pairs (Ctx::QX)
-enum { FQ_RHO = 0, FQ_U, FQ_V, FQ_W, FQ_P, FQ_RE, FQ_C, FQ_G, NFQ };
+// primitive components of the fused path, and 1/rho: the species of q are
+// those of U1 times 1/rho, formed where they are read
+enum { FQ_RHO = 0, FQ_U, FQ_V, FQ_W, FQ_P, FQ_RE, FQ_C, FQ_G, FQ_RI, NFQ };
 // The face arrays below store their components in interleaved pairs (EF,
 // EF2): 2 * NSPEC_PAIRS component slots for NSPEC species, every pair
 // starting at an even component and every component count even.
 constexpr int NSPEC_PAIRS = (NSPEC + 1) / 2;
-// traced / corrected interface states (velocities in absolute order)
-enum { FS_RHO = 0, FS_U, FS_V, FS_W, FS_P, FS_RE, FS_X, NFS = FS_X + 2 * NSPEC_PAIRS };
-// transverse-stage fluxes: conserved URHO..UEDEN, Godunov p, species,
-// Godunov normal u (and a padding slot)
-enum { FF_RHO = 0, FF_MX, FF_MY, FF_MZ, FF_E, FF_GP, FF_X, FF_GU = FF_X + 2 * NSPEC_PAIRS, NFF = FF_GU + 2 };
-// final fluxes: conserved URHO..UTEMP, Godunov p, species, Godunov normal u
-// (and a padding slot)
+// traced interface states without species (velocities in absolute order)
+enum { FS_RHO = 0, FS_U, FS_V, FS_W, FS_P, FS_RE, NFS };
+// First-stage and transverse-stage fluxes without species: mass flux with
+// the Riemann weight fpl of the minus side (0, 1/2 or 1; the plus side's is
+// 1 - fpl), momenta, energy, Godunov p and normal u.  The species stage
+// needs the first pair alone.
+enum { FF_RHO = 0, FF_W, FF_MX, FF_MY, FF_MZ, FF_E, FF_GP, FF_GU, NFF };
+// final fluxes: conserved URHO..UEINT (UTEMP's flux is zero and not stored),
+// Godunov p and normal u; the mass flux before the artificial viscosity and
+// its weight; the viscosity's coefficient (doubles, in the first half of its
+// pair's region); the species fluxes before their normalisation (species_fac)
 static_assert(UFS + NSPEC == NVAR, "the species are the last conserved components");
-enum { FN_GP = UFS, FN_X, FN_GU = FN_X + 2 * NSPEC_PAIRS, NFN = FN_GU + 2 };
+enum { FN_GP = UTEMP, FN_GU, FN_FR, FN_W, FN_DIV, FN_X = FN_DIV + 2, NFN = FN_X + 2 * NSPEC_PAIRS };
 static_assert(NFS % 2 == 0 && NFF % 2 == 0 && NFN % 2 == 0, "face arrays hold whole pairs");
-static_assert(FS_X % 2 == 0 && FF_X % 2 == 0 && FN_X % 2 == 0, "species pairs start at even components");
+static_assert(FN_X % 2 == 0 && FN_FR % 2 == 0 && FN_DIV % 2 == 0 && FN_GP % 2 == 0, "pairs start at even components");
 static_assert(FS_RHO == 0 && FS_U == 1 && FS_V == 2 && FS_W == 3 && FS_P == 4 && FS_RE == 5, "state pairs");
-static_assert(FF_E == UEDEN && FF_GP == FF_E + 1 && FN_GP == UTEMP + 1, "flux pairs");
+
+// planes of primitives a slab's face stages read beyond its cells (the
+// flattening of its ring cells reaches three cells further)
+constexpr int WHALO = 4;
 
 struct FInst {
     int n[3];
@@ -41,7 +48,15 @@ struct FInst {
     double dx[3];
     long offD, offE;  // cell offsets in the cell / extended index spaces
     long nD, nE;      // cell counts
-    long offQ, nQ;    // species pairs of q: offset and cell count, both even
+    // The primitives and the cleaned state (Q, U1, U1X) cover the whole
+    // instance, or in slabs a ring buffer of the slab's planes and WHALO
+    // more on either side: cell offset and count, and the same made even
+    // (U1X's pairs).
+    long offW, nW, offQ, nQ;
+    // plane k of these arrays is plane_w(I, k): wrapped or clamped to [wlo,
+    // whi], less wz, in a ring of wR planes
+    int wwrap, wlo, whi, wz, wR;
+    long offP;        // offset of the saved boundary planes (Ctx::UB)
     int ext[3];       // n + 2 in x and y; in z the planes of one slab + 2
     // The face stages work on a z-slab of cells [zlo, zlo + zn) (the whole
     // instance unless the engine runs in slabs): the extended arrays hold the
@@ -62,7 +77,9 @@ struct Plan {
 
 struct Ctx {
     const FInst *inst;
-    double *U, *U1, *U1X, *Q, *QX, *FL, *DV;
+    double *U, *U1, *U1X, *Q, *FL, *DV;
+    double *UB;  // slabs: the state's first and last WHALO planes as the step found them
+    double *RW;  // per ring cell and direction: the densities of its plus and minus states (3 pairs)
     double *SM[3], *SP[3], *FD[3], *FT[6], *FN[3];
     double *dt_cur, *dt_est, *time;
     int *steps;
@@ -170,9 +187,14 @@ struct Plan3 {
     int nb[3];
 };
 
+// Domain cell behind index i: periodic image, or the nearest cell.  An index
+// within one period of the domain (all of them unless the instance is
+// smaller than a stencil or a tile) wraps without a division.
 __device__ __forceinline__ int bmap(int i, int n, int periodic)
 {
-    return periodic ? ((i % n) + n) % n : min(max(i, 0), n - 1);
+    if (!periodic) return min(max(i, 0), n - 1);
+    if ((unsigned)(i + n) < 3u * (unsigned)n) return i < 0 ? i + n : (i >= n ? i - n : i);
+    return ((i % n) + n) % n;
 }
 
 // Cell and face indices within one instance are 32-bit and so are the byte
@@ -233,7 +255,7 @@ __device__ __forceinline__ gdbl2 &EF2(double *a, const FInst &I, int C, int c, i
 
 // The species of a face array (species block at the even component cX) as
 // NSPEC_PAIRS pairs, and the species kept apart in pairs of a cell array
-// (q, U1; count nQ).  The base and pair stride are taken once, before a
+// (U1; count nQ).  The base and pair stride are taken once, before a
 // kernel's species loop, so that the loop's stores (which may alias the
 // instance table as far as the compiler knows) do not force the instance
 // fields to be loaded again in every pass.
@@ -245,11 +267,11 @@ __device__ __forceinline__ SpeciesPairs species_pairs(double *a, const FInst &I,
 {
     return SpeciesPairs{a + ((long)C * I.offE + (long)cX * I.nE), 2 * I.nE};
 }
-// the species of a cell array kept apart in pairs (q, U1), over the
-// instance's cells
-__device__ __forceinline__ SpeciesPairs cell_species(double *QX, const FInst &I)
+// the species of a cell array kept apart in pairs (U1), over the instance's
+// cells
+__device__ __forceinline__ SpeciesPairs cell_species(double *UX, const FInst &I)
 {
-    return SpeciesPairs{QX + 2L * NSPEC_PAIRS * I.offQ, 2 * I.nQ};
+    return SpeciesPairs{UX + 2L * NSPEC_PAIRS * I.offQ, 2 * I.nQ};
 }
 // pair p at element idx (idx < 2^28)
 __device__ __forceinline__ gdbl2 &SP2(const SpeciesPairs &S, int p, idx_t idx)
@@ -273,6 +295,18 @@ __device__ __forceinline__ idx_t cidx(const FInst &I, int i, int j, int k)
     return (idx_t)bmap(i, I.n[0], I.periodic) +
            (idx_t)I.n[0] * ((idx_t)bmap(j, I.n[1], I.periodic) + (idx_t)I.n[1] * (idx_t)bmap(k, I.n[2], I.periodic));
 }
+// plane of Q, U1, U1X that holds cell plane k, and the index of a
+// (boundary-mapped) cell in them
+__device__ __forceinline__ int plane_w(const FInst &I, int k)
+{
+    const int d = (I.wwrap ? bmap(k, I.n[2], 1) : min(max(k, I.wlo), I.whi)) - I.wz;
+    return d >= I.wR ? d - I.wR : d;
+}
+__device__ __forceinline__ idx_t widx(const FInst &I, int i, int j, int k)
+{
+    return (idx_t)bmap(i, I.n[0], I.periodic) +
+           (idx_t)I.n[0] * ((idx_t)bmap(j, I.n[1], I.periodic) + (idx_t)I.n[1] * (idx_t)plane_w(I, k));
+}
 // index of an extended cell / face (i, j in [-1, n], k in the slab's ring
 // [zlo - 1, zlo + zn])
 __device__ __forceinline__ idx_t eidx(const FInst &I, int i, int j, int k)
@@ -287,6 +321,11 @@ __device__ __forceinline__ int hi_cell(const FInst &I, int a) { return a == 2 ? 
 __device__ __forceinline__ gdouble &CA(double *a, const FInst &I, int C, int c, idx_t idx)
 {
     return at(uniform_ptr(a + ((long)C * I.offD + (long)c * I.nD)), idx);
+}
+// component c of Q or U1 (index widx)
+__device__ __forceinline__ gdouble &WA(double *a, const FInst &I, int C, int c, idx_t idx)
+{
+    return at(uniform_ptr(a + ((long)C * I.offW + (long)c * I.nW)), idx);
 }
 // component c chosen per lane (c not uniform across the wavefront)
 __device__ __forceinline__ double CA_lane(const double *a, const FInst &I, int C, int c, idx_t idx)
@@ -350,33 +389,48 @@ __device__ __forceinline__ void store_tflux_h(double *F, const FInst &I, idx_t e
     const double mx = d == 0 ? o.f_mn : o.f_mt;
     const double my = d == 0 ? o.f_mt : (d == 1 ? o.f_mn : o.f_mtt);
     const double mz = d == 2 ? o.f_mn : o.f_mtt;
-    EF2(F, I, NFF, FF_RHO, e) = dbl2{o.f_rho, mx};
-    EF2(F, I, NFF, FF_MY, e) = dbl2{my, mz};
-    EF2(F, I, NFF, FF_E, e) = dbl2{o.f_E, o.g_p};
-    EF(F, I, NFF, FF_GU, e) = o.g_un;
+    EF2(F, I, NFF, FF_RHO, e) = dbl2{o.f_rho, o.fpl};
+    EF2(F, I, NFF, FF_MX, e) = dbl2{mx, my};
+    EF2(F, I, NFF, FF_MZ, e) = dbl2{mz, o.f_E};
+    EF2(F, I, NFF, FF_GP, e) = dbl2{o.g_p, o.g_un};
 }
 
 // Riemann problem on face (i,j,k) of direction d (cells i-e_d and i)
 __device__ __forceinline__ void face_riemann_h(const Ctx &x, const FInst &I, int d, int i, int j, int k,
                                                const FaceH &L, const FaceH &R, RiemannH &o)
 {
-    const idx_t cr = cidx(I, i, j, k);
-    const idx_t cl = cidx(I, i - (d == 0), j - (d == 1), k - (d == 2));
-    riemann_hydro(L, R, CA(x.Q, I, NFQ, FQ_C, cl), CA(x.Q, I, NFQ, FQ_C, cr), CA(x.Q, I, NFQ, FQ_G, cl),
-                  CA(x.Q, I, NFQ, FQ_G, cr), o);
+    const idx_t cr = widx(I, i, j, k);
+    const idx_t cl = widx(I, i - (d == 0), j - (d == 1), k - (d == 2));
+    riemann_hydro(L, R, WA(x.Q, I, NFQ, FQ_C, cl), WA(x.Q, I, NFQ, FQ_C, cr), WA(x.Q, I, NFQ, FQ_G, cl),
+                  WA(x.Q, I, NFQ, FQ_G, cr), o);
 }
 
 // URHO..UEDEN of a transverse-stage flux and its Godunov p, u
 __device__ __forceinline__ void load_tflux_h(double *F, const FInst &I, idx_t e, double *v, double &gp, double &gu)
 {
-    const dbl2 a = EF2(F, I, NFF, FF_RHO, e), b = EF2(F, I, NFF, FF_MY, e), c = EF2(F, I, NFF, FF_E, e);
-    v[URHO] = a.x;
-    v[UMX] = a.y;
-    v[UMY] = b.x;
-    v[UMZ] = b.y;
-    v[UEDEN] = c.x;
-    gp = c.y;
-    gu = EF(F, I, NFF, FF_GU, e);
+    const dbl2 a = EF2(F, I, NFF, FF_MX, e), b = EF2(F, I, NFF, FF_MZ, e), c = EF2(F, I, NFF, FF_GP, e);
+    v[URHO] = EF(F, I, NFF, FF_RHO, e);
+    v[UMX] = a.x;
+    v[UMY] = a.y;
+    v[UMZ] = b.x;
+    v[UEDEN] = b.y;
+    gp = c.x;
+    gu = c.y;
+}
+
+// normalize_species_fluxes (Source/Castro_hydro_nd.F90:248-297): the factor
+// of face e's species fluxes, from their sum in species order and the mass
+// flux frho of the face
+__device__ __forceinline__ double species_fac(const SpeciesPairs &XN, idx_t e, double frho)
+{
+    double sum = 0.0;
+#pragma unroll
+    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+        const dbl2 f = SP2(XN, pr, e);
+        sum = sum + f.x;
+        if (2 * pr + 1 < NSPEC) sum = sum + f.y;
+    }
+    return (sum != 0.0) ? frho / sum : 1.0;
 }
 
 static __constant__ int c_pair_t[6] = {1, 2, 0, 2, 0, 1};   // state (face) direction
@@ -411,12 +465,19 @@ struct FusedLevel {
     // plans: one block table per (tiling, ghost) pair
     struct PlanBuf {
         KernelTiling t;
-        int shift, add, slab;  // slab -1: the whole instance (cell stages)
+        int shift, add, slab;  // slab -1: the whole instance (estdt)
+        bool prim;             // K_prim's plane ranges (pinst)
         int ovl;               // direction along which bricks overlap by one cell, -1 none
         int *blk0 = nullptr;
         int nblocks = 0;
     };
     std::vector<PlanBuf> plans;
+    // block tables of the species stage, one per slab
+    struct SpecBuf {
+        int slab, lz, nblocks = 0;
+        int *blk0 = nullptr;
+    };
+    std::vector<SpecBuf> specs;
     // per stage: est prim flat trace flux1 trans1 final update tflux
     // trans1c finalc; the last three are (W, L, X): bricks (W, L, 1) along
     // y, (W, 1, L) along z and (X, W*L/X, 1) along x, each overlapping its
@@ -432,6 +493,11 @@ struct FusedLevel {
     int slab = 0, nslab = 1;
     std::vector<FInst *> sinst;
     std::vector<std::vector<FInst>> hsinst;
+    // and one per slab for K_prim, whose planes run ahead of the slab's
+    // (zlo, zn: the planes not yet in the ring, unwrapped)
+    std::vector<FInst *> pinst;
+    std::vector<std::vector<FInst>> hpinst;
+    long totW = 0, totP = 0;
     bool have_est = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
