@@ -9,15 +9,19 @@
 //  * the density-side quantities (iat, xd and all density basis weights)
 //    depend only on ye*rho, which is fixed during a Newton solve, so they are
 //    computed once per call;
-//  * Newton iterations evaluate only e and de/dT (the three h5 sums that feed
-//    them); the full set (p, dp/drho, dp/dT, gamma_1, ...) is evaluated once,
-//    at the temperature the reference's final pass uses.  Every quantity that
-//    is computed is computed with the reference's expression, so results are
-//    bit-identical to the reference arithmetic when built without FMA
-//    contraction;
-//  * the h5 sums of one evaluation run together, two table columns at a
-//    time (each sum keeps its own term order), so the four nodes' columns
-//    are not all held in registers at once.
+//  * Newton iterations evaluate only e and de/dT (eos_energy: the three h5
+//    sums that feed them); the rest (eos_pressure: p, dp/drho, dp/dT, gamma_1,
+//    ...) is evaluated once, at the temperature the reference's final pass
+//    uses, with weights of its own.  Every quantity that is computed is
+//    computed with the reference's expression, so results are bit-identical
+//    to the reference arithmetic when built without FMA contraction;
+//  * table cells are found with a single-precision logarithm except near grid
+//    lines, and a convergence test divides only near its tolerance.
+// With both halves of an evaluation in one loop a kernel took 256 registers
+// and spilled or ran one wavefront per SIMD; apart they take at most 251 with
+// a cell's state (256^3: K_prim 3.55 -> 2.95 ms, K_update 4.5 -> 4.1, K_est 2.0 ->
+// 1.4; a 64^3 box: estdt 81 -> 25 us, compute_temp on its grown 72^3 31 -> 17;
+// 1,000,000 unordered (rho, e) solves 436 -> 342 us).
 // The electron chemical potential and number density tables (ef*, xf*) and
 // the entropy terms feed nothing on the hydro path and are not evaluated.
 #pragma once
@@ -105,47 +109,6 @@ __device__ __forceinline__ void load_node(const double *p, double *o, int ncol)
     }
 }
 
-// One column q of the biquintic sum in the reference's term order:
-// fi(4q+1)*wd*wt + fi(4q+2)*wmd*wt + fi(4q+3)*wd*wmt + fi(4q+4)*wmd*wmt
-#define MC_H5_TERMS(acc, N, q, wd, wmd, wt, wmt)                                \
-    acc = acc + N.a[q] * wd * wt;                                               \
-    acc = acc + N.b[q] * wmd * wt;                                              \
-    acc = acc + N.c[q] * wd * wmt;                                              \
-    acc = acc + N.d[q] * wmd * wmt;
-
-// Source/eos.F90:915-950; t-weights T, d-weights D.
-__device__ __forceinline__ double h5(const Nodes &N, const W6 &T, const W6 &D)
-{
-    double acc = N.a[NF] * D.w0 * T.w0;
-    acc = acc + N.b[NF] * D.w0m * T.w0;
-    acc = acc + N.c[NF] * D.w0 * T.w0m;
-    acc = acc + N.d[NF] * D.w0m * T.w0m;
-    MC_H5_TERMS(acc, N, NFT, D.w0, D.w0m, T.w1, T.w1m)
-    MC_H5_TERMS(acc, N, NFTT, D.w0, D.w0m, T.w2, T.w2m)
-    MC_H5_TERMS(acc, N, NFD, D.w1, D.w1m, T.w0, T.w0m)
-    MC_H5_TERMS(acc, N, NFDD, D.w2, D.w2m, T.w0, T.w0m)
-    MC_H5_TERMS(acc, N, NFDT, D.w1, D.w1m, T.w1, T.w1m)
-    MC_H5_TERMS(acc, N, NFDDT, D.w2, D.w2m, T.w1, T.w1m)
-    MC_H5_TERMS(acc, N, NFDTT, D.w1, D.w1m, T.w2, T.w2m)
-    MC_H5_TERMS(acc, N, NFDDTT, D.w2, D.w2m, T.w2, T.w2m)
-    return acc;
-}
-
-// Source/eos.F90:1034-1059 over the dpdf columns; w = (w0, w1, w0m, w1m).
-__device__ __forceinline__ double h3_dpdf(const Nodes &N, double t0, double t1, double t0m, double t1m,
-                                          double d0, double d1, double d0m, double d1m)
-{
-    double acc = N.a[NDPDF] * d0 * t0;
-    acc = acc + N.b[NDPDF] * d0m * t0;
-    acc = acc + N.c[NDPDF] * d0 * t0m;
-    acc = acc + N.d[NDPDF] * d0m * t0m;
-    MC_H5_TERMS(acc, N, NDPDFT, d0, d0m, t1, t1m)
-    MC_H5_TERMS(acc, N, NDPDFD, d1, d1m, t0, t0m)
-    MC_H5_TERMS(acc, N, NDPDFDT, d1, d1m, t1, t1m)
-    return acc;
-}
-#undef MC_H5_TERMS
-
 // One column of a biquintic or bicubic sum: the four nodes' values a b c d
 // (nodes (i,j) (i+1,j) (i,j+1) (i+1,j+1)) with the density weights (wd, wmd)
 // and temperature weights (wt, wmt), added to acc in h5's term order (the
@@ -163,13 +126,28 @@ __device__ __forceinline__ void hcol(double &acc, bool first, double a, double b
 __device__ __forceinline__ double wsel(const W6 &w, int k) { return k == 0 ? w.w0 : (k == 1 ? w.w1 : w.w2); }
 __device__ __forceinline__ double wselm(const W6 &w, int k) { return k == 0 ? w.w0m : (k == 1 ? w.w1m : w.w2m); }
 
+// Table cell of x on a logarithmic axis: (int)((log10(x) - lo) * stpi) + 1,
+// clamped to 1..n (Source/eos.F90:229-244).  Except within 1/256 of a grid
+// line the single-precision logarithm decides it (its error is below 1e-4
+// cells over the table); there, and for anything but a positive normal number,
+// log10 does.
+__device__ __forceinline__ int eos_cell(double x, double lo, double stpi, int n)
+{
+    const int h = __double2hiint(x);
+    const int ex = (h >> 20) - 1023;
+    const float m = __int_as_float(0x3f800000 | ((h & 0xfffff) << 3) | (int)((unsigned)__double2loint(x) >> 29));
+    const float f = (((float)ex + __builtin_amdgcn_logf(m)) * 0.301029996f - (float)lo) * (float)stpi;
+    const float r = f - floorf(f);
+    int c = (int)f + 1;
+    if (!(r > 0.00390625f && r < 0.99609375f && ex > -500 && ex < 500)) c = (int)((log10(x) - lo) * stpi) + 1;
+    return c < 1 ? 1 : (c > n ? n : c);
+}
+
 // Density-side data of one EOS call (constant through the Newton solve).
 struct EosDen {
-    double den, deni, ytot1, ye, din;
+    double den, deni, ytot1, ye, din, xd;
     int iat;
-    W6 D;     // quintic weights (value)
-    W6 dD;    // quintic weights (d/d din)
-    double x0, x1, x0m, x1m;  // cubic weights (value)
+    W6 D;  // quintic weights (value)
 };
 
 __device__ __forceinline__ void eos_density(const EosTable &tab, double rho, double abar, double zbar,
@@ -180,72 +158,95 @@ __device__ __forceinline__ void eos_density(const EosTable &tab, double rho, dou
     s.ye = zbar / abar;
     s.din = s.ye * s.den;
     s.deni = 1.0 / s.den;
-    int iat = (int)((log10(s.din) - eosc::dlo) * eosc::dstpi) + 1;
-    iat = iat < 1 ? 1 : (iat > EOS_IMAX - 1 ? EOS_IMAX - 1 : iat);
-    s.iat = iat;
-    const double *g = tab.dg + (long)(iat - 1) * EOS_GRID;
+    s.iat = eos_cell(s.din, eosc::dlo, eosc::dstpi, EOS_IMAX - 1);
+    const double *g = tab.dg + (long)(s.iat - 1) * EOS_GRID;
     const double dI = g[G_X], dd = g[G_D], dd2 = g[G_D2], ddi = g[G_DI];
-    double xd = fmax((s.din - dI) * ddi, 0.0);
-    double mxd = 1.0 - xd;
+    const double xd = fmax((s.din - dI) * ddi, 0.0);
+    const double mxd = 1.0 - xd;
+    s.xd = xd;
     s.D.w0 = psi0(xd);
     s.D.w1 = psi1(xd) * dd;
     s.D.w2 = psi2(xd) * dd2;
     s.D.w0m = psi0(mxd);
     s.D.w1m = -psi1(mxd) * dd;
     s.D.w2m = psi2(mxd) * dd2;
-    s.dD.w0 = dpsi0(xd) * ddi;
-    s.dD.w1 = dpsi1(xd);
-    s.dD.w2 = dpsi2(xd) * dd;
-    s.dD.w0m = -dpsi0(mxd) * ddi;
-    s.dD.w1m = dpsi1(mxd);
-    s.dD.w2m = -dpsi2(mxd) * dd;
-    s.x0 = xpsi0(xd);
-    s.x1 = xpsi1(xd) * dd;
-    s.x0m = xpsi0(mxd);
-    s.x1m = -xpsi1(mxd) * dd;
 }
 
-// Full thermodynamic output of one evaluation.
+// Thermodynamic output of one evaluation.
 struct EosFull {
     double p, e, dpdT, dpdr, dedT, dedr, gam1, dpde, dpdr_e;
 };
 
-// One evaluation at temperature temp (Source/eos.F90:195-518).  FULL=false
-// computes only e and de/dT; FULL=true computes everything the path uses.
-template <bool FULL>
-__device__ __forceinline__ void eos_eval(const EosTable &tab, const EosDen &s, double temp, int &jat_out,
-                                         EosFull &o)
+// The four table rows of a cell, two columns (c2 = 0: columns 0 and 1, ...) at
+// a time.
+struct EosCols {
+    double2 a, b, c, d;  // nodes (i,j) (i+1,j) (i,j+1) (i+1,j+1)
+};
+struct EosRows {
+    const char *base;
+    unsigned off;
+    __device__ __forceinline__ EosCols load(int c2) const
+    {
+        const char *q = base + off + 16 * c2;
+        return EosCols{*(const double2 *)q, *(const double2 *)(q + 8 * EOS_NODE),
+                       *(const double2 *)(q + 8L * EOS_IMAX * EOS_NODE),
+                       *(const double2 *)(q + 8L * EOS_IMAX * EOS_NODE + 8 * EOS_NODE)};
+    }
+};
+// Pairs of columns loaded together.  A row is one cache line, and a
+// wavefront's rows (4 per lane) can fill the vector L1: where lanes share no
+// rows (mc_eos_eval_batch over unordered points) every group fetches the lines
+// again.  1,000,000 such (rho, e) solves took 531, 508, 489 and 342 us with
+// groups of 1 (one ahead), 2, 3 and 5; cells of a flow are indifferent
+// (K_prim 2.9 ms, K_update 3.8 to 4.1 at 256^3), as are three wavefronts per
+// SIMD, which groups of 1 allow.
+constexpr int EOS_CHUNK = 5;
+__device__ __forceinline__ EosRows eos_rows(const EosTable &tab, int iat, int jat)
+{
+    EosRows r;
+    r.base = (const char *)tab.node;
+    r.off = ((unsigned)(iat - 1) + (unsigned)EOS_IMAX * (unsigned)(jat - 1)) * (8u * EOS_NODE);
+    return r;
+}
+// The next columns' address waits for the sums so far: without the tie the
+// compiler gathers every column of every sum first (104 registers of table
+// values, and one wavefront per SIMD or spills).
+#define MC_EOS_STEP(r, s0, s1, s2) asm volatile("" : "+v"((r).off), "+v"(s0), "+v"(s1), "+v"(s2))
+
+// columns' weights in the order of the node slots: density weight dsel,
+// temperature weight tsel
+__device__ constexpr int eos_dsel[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
+__device__ constexpr int eos_tsel[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
+
+// e and de/dT at temperature temp (Source/eos.F90:195-518): what a Newton
+// iteration needs.
+// The biquintic sums (Source/eos.F90:915-950) of the free energy and its
+// derivatives run column by column: every sum adds the reference's terms in
+// its order, EOS_CHUNK pairs of columns of the four nodes at a time.
+__device__ __forceinline__ void eos_energy(const EosTable &tab, const EosDen &s, double temp, int &jat_out,
+                                           EosFull &o)
 {
     using namespace eosc;
     const double den = s.den, deni = s.deni, ytot1 = s.ytot1, ye = s.ye;
-    const double tempi = 1.0 / temp;
+    const int jat = eos_cell(temp, tlo, tstpi, EOS_JMAX - 1);
+    jat_out = jat;
+    EosRows rows = eos_rows(tab, s.iat, jat);
+    EosCols col[5];
+    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
+    const double tJ = g[G_X], dt = g[G_D], dt2 = g[G_D2], dti = g[G_DI], dt2i = g[G_D2I];
 
+    const double tempi = 1.0 / temp;
     const double prad = asoli3 * temp * temp * temp * temp;
     const double dpraddt = 4.0 * prad * tempi;
     const double erad = 3.0 * prad * deni;
     const double deraddt = 3.0 * dpraddt * deni;
-
     const double pion = kergavo * ytot1 * den * temp;
-    const double dpiondd = kergavo * ytot1 * temp;
     const double dpiondt = kergavo * ytot1 * den;
     const double eion = 1.5 * pion * deni;
     const double deiondt = 1.5 * dpiondt * deni;
 
-    int jat = (int)((log10(temp) - tlo) * tstpi) + 1;
-    jat = jat < 1 ? 1 : (jat > EOS_JMAX - 1 ? EOS_JMAX - 1 : jat);
-    jat_out = jat;
-
-    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
-    const double tJ = g[G_X], dt = g[G_D], dt2 = g[G_D2], dti = g[G_DI], dt2i = g[G_D2I];
-
-    const double *n0 = tab.node + ((long)(s.iat - 1) + (long)EOS_IMAX * (jat - 1)) * EOS_NODE;
-    const double2 *qa = reinterpret_cast<const double2 *>(n0), *qb = reinterpret_cast<const double2 *>(n0 + EOS_NODE),
-                  *qc = reinterpret_cast<const double2 *>(n0 + (long)EOS_IMAX * EOS_NODE),
-                  *qd = reinterpret_cast<const double2 *>(n0 + (long)EOS_IMAX * EOS_NODE + EOS_NODE);
-
     const double xt = fmax((temp - tJ) * dti, 0.0);
     const double mxt = 1.0 - xt;
-
     W6 T, dT, ddT;
     T.w0 = psi0(xt);
     T.w1 = psi1(xt) * dt;
@@ -266,30 +267,25 @@ __device__ __forceinline__ void eos_eval(const EosTable &tab, const EosDen &s, d
     ddT.w1m = -ddpsi1(mxt) * dti;
     ddT.w2m = ddpsi2(mxt);
 
-    // The biquintic sums (Source/eos.F90:915-950) of the free energy and its
-    // derivatives, column by column: every sum adds the same terms in the
-    // same order as h5, but only two columns of the four nodes are live at a
-    // time.  Column q takes density weight dsel and temperature weight tsel.
-    constexpr int dsel[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
-    constexpr int tsel[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
-    double free = 0.0, df_t = 0.0, df_tt = 0.0, df_d = 0.0, df_dt = 0.0;
+    double free = 0.0, df_t = 0.0, df_tt = 0.0;
 #pragma unroll
     for (int c2 = 0; c2 < 5; ++c2) {
-        const double2 va = qa[c2], vb = qb[c2], vc = qc[c2], vd = qd[c2];
+        if (c2 % EOS_CHUNK == 0) {
+            if (c2) MC_EOS_STEP(rows, free, df_t, df_tt);
+#pragma unroll
+            for (int l = c2; l < c2 + EOS_CHUNK && l < 5; ++l) col[l] = rows.load(l);
+        }
+        const EosCols cur = col[c2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int q = 2 * c2 + h;
             if (q >= 9) break;
-            const double a = h ? va.y : va.x, b = h ? vb.y : vb.x, c = h ? vc.y : vc.x, d = h ? vd.y : vd.x;
-            const double wd = wsel(s.D, dsel[q]), wmd = wselm(s.D, dsel[q]);
-            hcol(free, q == 0, a, b, c, d, wd, wmd, wsel(T, tsel[q]), wselm(T, tsel[q]));
-            hcol(df_t, q == 0, a, b, c, d, wd, wmd, wsel(dT, tsel[q]), wselm(dT, tsel[q]));
-            hcol(df_tt, q == 0, a, b, c, d, wd, wmd, wsel(ddT, tsel[q]), wselm(ddT, tsel[q]));
-            if (FULL) {
-                const double ed = wsel(s.dD, dsel[q]), emd = wselm(s.dD, dsel[q]);
-                hcol(df_d, q == 0, a, b, c, d, ed, emd, wsel(T, tsel[q]), wselm(T, tsel[q]));
-                hcol(df_dt, q == 0, a, b, c, d, ed, emd, wsel(dT, tsel[q]), wselm(dT, tsel[q]));
-            }
+            const double a = h ? cur.a.y : cur.a.x, b = h ? cur.b.y : cur.b.x, c = h ? cur.c.y : cur.c.x,
+                         d = h ? cur.d.y : cur.d.x;
+            const double wd = wsel(s.D, eos_dsel[q]), wmd = wselm(s.D, eos_dsel[q]);
+            hcol(free, q == 0, a, b, c, d, wd, wmd, wsel(T, eos_tsel[q]), wselm(T, eos_tsel[q]));
+            hcol(df_t, q == 0, a, b, c, d, wd, wmd, wsel(dT, eos_tsel[q]), wselm(dT, eos_tsel[q]));
+            hcol(df_tt, q == 0, a, b, c, d, wd, wmd, wsel(ddT, eos_tsel[q]), wselm(ddT, eos_tsel[q]));
         }
     }
 
@@ -297,53 +293,119 @@ __device__ __forceinline__ void eos_eval(const EosTable &tab, const EosDen &s, d
     const double dsepdt = -df_tt * ye;
     const double eele = ye * free + temp * sele;
     const double deepdt = temp * dsepdt;
-
     o.e = erad + eion + eele;
     o.dedT = deraddt + deiondt + deepdt;
+}
 
-    if (FULL) {
-        const double xt0 = xpsi0(xt), xt1 = xpsi1(xt) * dt, xt0m = xpsi0(mxt), xt1m = -xpsi1(mxt) * dt;
-        // the bicubic dpdf sum (Source/eos.F90:1034-1059), columns 9..12 in
-        // h3_dpdf's order: (d0, t0), (d0, t1), (d1, t0), (d1, t1)
-        double dpepdd = 0.0;
-        {
-            const double2 a0 = qa[4], b0 = qb[4], c0 = qc[4], d0 = qd[4];  // column 9 in .y
-            hcol(dpepdd, true, a0.y, b0.y, c0.y, d0.y, s.x0, s.x0m, xt0, xt0m);
-            const double2 a1 = qa[5], b1 = qb[5], c1 = qc[5], d1 = qd[5];  // columns 10, 11
-            hcol(dpepdd, false, a1.x, b1.x, c1.x, d1.x, s.x0, s.x0m, xt1, xt1m);
-            hcol(dpepdd, false, a1.y, b1.y, c1.y, d1.y, s.x1, s.x1m, xt0, xt0m);
-            const double2 a2 = qa[6], b2 = qb[6], c2 = qc[6], d2 = qd[6];  // column 12 in .x
-            hcol(dpepdd, false, a2.x, b2.x, c2.x, d2.x, s.x1, s.x1m, xt1, xt1m);
+// The rest of an evaluation whose e and de/dT eos_energy left in o: pressure
+// and its derivatives, de/drho, gamma_1.
+__device__ __forceinline__ void eos_pressure(const EosTable &tab, const EosDen &s, double temp, int jat, EosFull &o)
+{
+    using namespace eosc;
+    const double den = s.den, deni = s.deni, ytot1 = s.ytot1, ye = s.ye;
+    EosRows rows = eos_rows(tab, s.iat, jat);
+    EosCols col[7];
+    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
+    const double tJ = g[G_X], dt = g[G_D], dt2 = g[G_D2], dti = g[G_DI];
+    const double *gd = tab.dg + (long)(s.iat - 1) * EOS_GRID;
+    const double dd = gd[G_D], ddi = gd[G_DI];
+    const double xt = fmax((temp - tJ) * dti, 0.0);
+    const double mxt = 1.0 - xt, xd = s.xd, mxd = 1.0 - s.xd;
+
+    W6 T, dT, dD;
+    T.w0 = psi0(xt);
+    T.w1 = psi1(xt) * dt;
+    T.w2 = psi2(xt) * dt2;
+    T.w0m = psi0(mxt);
+    T.w1m = -psi1(mxt) * dt;
+    T.w2m = psi2(mxt) * dt2;
+    dT.w0 = dpsi0(xt) * dti;
+    dT.w1 = dpsi1(xt);
+    dT.w2 = dpsi2(xt) * dt;
+    dT.w0m = -dpsi0(mxt) * dti;
+    dT.w1m = dpsi1(mxt);
+    dT.w2m = -dpsi2(mxt) * dt;
+    dD.w0 = dpsi0(xd) * ddi;
+    dD.w1 = dpsi1(xd);
+    dD.w2 = dpsi2(xd) * dd;
+    dD.w0m = -dpsi0(mxd) * ddi;
+    dD.w1m = dpsi1(mxd);
+    dD.w2m = -dpsi2(mxd) * dd;
+
+    // df_d, df_dt over the quintic columns, then the bicubic dpdf sum
+    // (Source/eos.F90:1034-1059) over columns 9..12, in its order (d0, t0),
+    // (d0, t1), (d1, t0), (d1, t1)
+    double df_d = 0.0, df_dt = 0.0, dpepdd = 0.0;
+#pragma unroll
+    for (int c2 = 0; c2 < 7; ++c2) {
+        if (c2 % EOS_CHUNK == 0) {
+            if (c2) MC_EOS_STEP(rows, df_d, df_dt, dpepdd);
+#pragma unroll
+            for (int l = c2; l < c2 + EOS_CHUNK && l < 7; ++l) col[l] = rows.load(l);
         }
-        dpepdd = fmax(ye * dpepdd, 0.0);
-
-        const double deraddd = -erad * deni;
-        const double deiondd = (1.5 * dpiondd - eion) * deni;
-        double x = s.din * s.din;
-        const double pele = x * df_d;
-        const double dpepdt = x * df_dt;
-        x = ye * ye;
-        const double dsepdd = -df_dt * x;
-        const double deepdd = x * df_d + temp * dsepdd;
-
-        const double pres = prad + pion + pele;
-        const double dpresdd = 0.0 + dpiondd + dpepdd;
-        const double dpresdt = dpraddt + dpiondt + dpepdt;
-        const double denerdd = deraddd + deiondd + deepdd;
-        const double denerdt = o.dedT;
-
-        const double zz = pres * deni;
-        const double zzi = den / pres;
-        const double chit = temp / pres * dpresdt;
-        const double chid = dpresdd * zzi;
-        o.gam1 = chit * zz * chit / (temp * denerdt) + chid;
-        o.p = pres;
-        o.dpdT = dpresdt;
-        o.dpdr = dpresdd;
-        o.dpde = dpresdt / denerdt;
-        o.dpdr_e = dpresdd - dpresdt * denerdd / denerdt;
-        o.dedr = denerdd;
+        const EosCols cur = col[c2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int q = 2 * c2 + h;
+            if (q >= 13) break;
+            const double a = h ? cur.a.y : cur.a.x, b = h ? cur.b.y : cur.b.x, c = h ? cur.c.y : cur.c.x,
+                         d = h ? cur.d.y : cur.d.x;
+            if (q < 9) {
+                const double ed = wsel(dD, eos_dsel[q]), emd = wselm(dD, eos_dsel[q]);
+                hcol(df_d, q == 0, a, b, c, d, ed, emd, wsel(T, eos_tsel[q]), wselm(T, eos_tsel[q]));
+                hcol(df_dt, q == 0, a, b, c, d, ed, emd, wsel(dT, eos_tsel[q]), wselm(dT, eos_tsel[q]));
+            } else {
+                const bool d1 = q >= 11, t1 = q == 10 || q == 12;
+                hcol(dpepdd, q == 9, a, b, c, d, d1 ? xpsi1(xd) * dd : xpsi0(xd), d1 ? -xpsi1(mxd) * dd : xpsi0(mxd),
+                     t1 ? xpsi1(xt) * dt : xpsi0(xt), t1 ? -xpsi1(mxt) * dt : xpsi0(mxt));
+            }
+        }
     }
+    dpepdd = fmax(ye * dpepdd, 0.0);
+
+    const double tempi = 1.0 / temp;
+    const double prad = asoli3 * temp * temp * temp * temp;
+    const double dpraddt = 4.0 * prad * tempi;
+    const double erad = 3.0 * prad * deni;
+    const double pion = kergavo * ytot1 * den * temp;
+    const double dpiondd = kergavo * ytot1 * temp;
+    const double dpiondt = kergavo * ytot1 * den;
+    const double eion = 1.5 * pion * deni;
+    const double deraddd = -erad * deni;
+    const double deiondd = (1.5 * dpiondd - eion) * deni;
+    double x = s.din * s.din;
+    const double pele = x * df_d;
+    const double dpepdt = x * df_dt;
+    x = ye * ye;
+    const double dsepdd = -df_dt * x;
+    const double deepdd = x * df_d + temp * dsepdd;
+
+    const double pres = prad + pion + pele;
+    const double dpresdd = 0.0 + dpiondd + dpepdd;
+    const double dpresdt = dpraddt + dpiondt + dpepdt;
+    const double denerdd = deraddd + deiondd + deepdd;
+    const double denerdt = o.dedT;
+
+    const double zz = pres * deni;
+    const double zzi = den / pres;
+    const double chit = temp / pres * dpresdt;
+    const double chid = dpresdd * zzi;
+    o.gam1 = chit * zz * chit / (temp * denerdt) + chid;
+    o.p = pres;
+    o.dpdT = dpresdt;
+    o.dpdr = dpresdd;
+    o.dpde = dpresdt / denerdt;
+    o.dpdr_e = dpresdd - dpresdt * denerdd / denerdt;
+    o.dedr = denerdd;
+}
+#undef MC_EOS_STEP
+
+// One whole evaluation (FULL) or e and de/dT.
+template <bool FULL>
+__device__ __forceinline__ void eos_eval(const EosTable &tab, const EosDen &s, double temp, int &jat, EosFull &o)
+{
+    eos_energy(tab, s, temp, jat, o);
+    if (FULL) eos_pressure(tab, s, temp, jat, o);
 }
 
 // Result of a (rho, e) solve.
@@ -352,41 +414,50 @@ struct EosRE {
     int iat, jat, niter;
 };
 
-// eos(eos_input_re, ...): Newton on T with the reference's step clamps
-// (Source/eos.F90:524-550).  FULL=false when the caller only needs T
-// (compute_temp restores e and discards everything else).
+// One Newton step on T with the reference's clamps (Source/eos.F90:524-550);
+// true when it has converged.  |dT / T| < ttol is decided without the
+// division unless it is within rounding of the tolerance.
+__device__ __forceinline__ bool eos_newton(double &temp, double f, double want, double dfdT)
+{
+    const double temp_old = temp;
+    temp = temp - (f - want) / dfdT;
+    temp = fmax(0.5 * temp_old, fmin(temp, 2.0 * temp_old));
+    temp = fmax(eosc::mintemp, temp);
+    const double d = fabs(temp - temp_old), t = eosc::ttol * fabs(temp_old);
+    bool ok = d < t;
+    if (!(d < t * (1.0 - 1.0e-12) || d > t * (1.0 + 1.0e-12))) ok = fabs((temp - temp_old) / temp_old) < eosc::ttol;
+    return ok;
+}
+
+// eos(eos_input_re, ...): Newton on T for e.  FULL=false when the caller only
+// needs T (compute_temp restores e and discards everything else).  As in the
+// reference, the evaluation after convergence is the one the outputs come
+// from; only that one computes the pressure (the last of a solve that does
+// not converge steps on after it).
 template <bool FULL>
 __device__ __forceinline__ EosRE eos_re(const EosTable &tab, double rho, double T0, double e_want, double abar,
                                         double zbar)
 {
     EosDen s;
     eos_density(tab, rho, abar, zbar, s);
-    double temp = T0;
+    double temp = T0, teval = T0;
     bool converged = false;
     EosFull o;
     int jat = 0, iter;
     for (iter = 1; iter <= EOS_MAX_NEWTON; ++iter) {
-        const bool last = converged || iter == EOS_MAX_NEWTON;
-        if (FULL && last) {
-            eos_eval<true>(tab, s, temp, jat, o);
-        } else {
-            if (converged) break;
-            eos_eval<false>(tab, s, temp, jat, o);
-        }
+        if (!FULL && converged) break;
+        teval = temp;
+        eos_energy(tab, s, temp, jat, o);
         if (converged) break;
-        const double temp_old = temp;
-        temp = temp - (o.e - e_want) / o.dedT;
-        temp = fmax(0.5 * temp_old, fmin(temp, 2.0 * temp_old));
-        temp = fmax(eosc::mintemp, temp);
-        const double error = fabs((temp - temp_old) / temp_old);
-        if (error < eosc::ttol) converged = true;
+        converged = eos_newton(temp, o.e, e_want, o.dedT);
     }
     if (!converged) eos_note_newton_failure(tab);
+    if (FULL) eos_pressure(tab, s, teval, jat, o);
     EosRE r;
+    r.niter = iter > EOS_MAX_NEWTON ? EOS_MAX_NEWTON : iter;
     r.T = temp;
     r.iat = s.iat;
     r.jat = jat;
-    r.niter = iter > EOS_MAX_NEWTON ? EOS_MAX_NEWTON : iter;
     if (FULL) {
         r.p = o.p;
         r.gam1 = o.gam1;
@@ -421,12 +492,7 @@ __device__ __forceinline__ double eos_rp_e(const EosTable &tab, double rho, doub
     for (int iter = 1; iter <= EOS_MAX_NEWTON; ++iter) {
         eos_eval<true>(tab, s, temp, jat, o);
         if (converged) break;
-        const double temp_old = temp;
-        temp = temp - (o.p - p_want) / o.dpdT;
-        temp = fmax(0.5 * temp_old, fmin(temp, 2.0 * temp_old));
-        temp = fmax(eosc::mintemp, temp);
-        const double error = fabs((temp - temp_old) / temp_old);
-        if (error < eosc::ttol) converged = true;
+        converged = eos_newton(temp, o.p, p_want, o.dpdT);
     }
     if (!converged) eos_note_newton_failure(tab);
     if (T_out) *T_out = temp;

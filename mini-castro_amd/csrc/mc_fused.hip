@@ -63,12 +63,12 @@ namespace mc {
 
 // ------------------------------------------------------------------ stages
 // estdt on the current state (Castro::estTimeStep before the first step)
-__global__ __launch_bounds__(256) void K_est(Plan p, Ctx x)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void K_est(Plan p, Ctx x)
 {
     int m, i, j, k;
     double v = DBL_MAX;
     const bool ok = plan_cell(p, m, i, j, k);
-    const FInst &I = p.inst[m];
+    const FInst I = p.inst[m];
     if (ok) {
         const idx_t c = cidx(I, i, j, k);
         double u[NVAR];
@@ -81,7 +81,8 @@ __global__ __launch_bounds__(256) void K_est(Plan p, Ctx x)
 }
 
 // S_old clean (Castro_advance.cpp:51), Sborder clean (:66), ctoprim.
-// Held to 2 waves per SIMD like K_update (3.85 -> 3.65 ms at 256^3).
+// Held to 2 waves per SIMD (251 registers, no spills): 2.95 ms at 256^3, and
+// 3.6 at 3, which spills.
 // SLABS: the planes [zlo, zlo + zn) that a slab adds to the ring buffer of
 // primitives.  Planes outside a periodic instance are its images, made from
 // the saved boundary planes (Ctx::UB) and not stored back.
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void K
 {
     int m, i, j, k;
     if (!plan_cell(p, m, i, j, k)) return;
-    const FInst &I = p.inst[m];
+    const FInst I = p.inst[m];
     const bool own = !SLABS || (k >= 0 && k < I.n[2]);
     const idx_t c = cidx(I, i, j, k), cw = SLABS ? widx(I, i, j, k) : c;
     double u[NVAR];
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(256) void K_flat(Plan p, Ctx x)
 {
     int m, i, j, k;
     if (!plan_cell(p, m, i, j, k)) return;
-    const FInst &I = p.inst[m];
+    const FInst I = p.inst[m];
     const idx_t e = eidx(I, i, j, k);
     // rows and planes of the cells up to three away (offset s at s + 3)
     idx_t ix[7], iy[7], iz[7];
@@ -740,9 +741,6 @@ __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
 // fill_hydro_source (Source/Castro_hydro_nd.F90:344-441), Saxpy and the two
 // clean_state calls of Castro_advance.cpp:74-78 / Castro.cpp:369, then the
 // next step's estdt (Source/timestep.F90:12-72) min-reduced per instance.
-// Held to 256 registers (2 waves per SIMD): the few spilled values cost less
-// than the second wave gains on the EOS table gathers (6.1 -> 5.5 ms at 256^3;
-// the same limit slows K_prim, which spills more).
 // POST: post_timestep's clean_state and the estdt of the new state follow
 // the advance's clean (the step of a level that is not the coarse side of a
 // flux register); without it the state is left as Castro::advance leaves
@@ -753,76 +751,72 @@ __device__ __forceinline__ void update_cells(Plan p, Ctx x)
     int m, i, j, k;
     double v = DBL_MAX;
     const bool ok = plan_cell(p, m, i, j, k);
-    const FInst &I = p.inst[m];
+    const FInst I = p.inst[m];
     if (ok) {
         const idx_t c = cidx(I, i, j, k);
         const double dx0 = I.dx[0], dx1 = I.dx[1], dx2 = I.dx[2];
         const double a0 = dx1 * dx2, a1 = dx0 * dx2, a2 = dx0 * dx1;
         const double volinv = 1.0 / (dx0 * dx1 * dx2);
-        const idx_t e = eidx(I, i, j, k);
-        const idx_t ex = eidx(I, i + 1, j, k), ey = eidx(I, i, j + 1, k), ez = eidx(I, i, j, k + 1);
-        double *F0 = x.FN[0], *F1 = x.FN[1], *F2 = x.FN[2];
-        const SpeciesPairs P0 = species_pairs(F0, I, NFN, FN_X), P1 = species_pairs(F1, I, NFN, FN_X),
-                           P2 = species_pairs(F2, I, NFN, FN_X);
+        idx_t e = eidx(I, i, j, k);
         const double dt = x.dt_cur[m];
-        double u[NVAR];
+        // The flux divergence of every component (flux_div's sum, term by
+        // term), a direction at a time: its two faces' species fluxes with
+        // their normalisation (Source/Castro_hydro_nd.F90:248-297), the
+        // conserved fluxes as the pairs (0,1) (2,3) (4,5), and p div u from the
+        // pair of Godunov p and u.  UTEMP has no flux.
+        const idx_t up[3] = {1u, (idx_t)I.ext[0], (idx_t)I.ext[0] * (idx_t)I.ext[1]};
+        const double ad[3] = {a0, a1, a2}, dxd[3] = {dx0, dx1, dx2};
+        double s[NVAR], pdivu = 0.0;
+        idx_t cu = c;
 #pragma unroll
-        for (int n = 0; n < NVAR; ++n) u[n] = CA(x.U, I, NVAR, n, c);  // clean(S_old), stored by K_prim
-        // the species fluxes of the six faces with their normalisation
-        // (Source/Castro_hydro_nd.F90:248-297)
-        {
-            const SpeciesPairs P[3] = {P0, P1, P2};
-            double *FN[3] = {F0, F1, F2};
-            const idx_t eh[3] = {ex, ey, ez};
-            dbl2 f[3][2][NSPEC_PAIRS];
+        for (int d = 0; d < 3; ++d) {
+            const SpeciesPairs P = species_pairs(x.FN[d], I, NFN, FN_X);
+            dbl2 f[2][NSPEC_PAIRS];
+            double fac[2];
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
+            for (int hi = 0; hi < 2; ++hi) {
+                const idx_t ee = hi ? e + up[d] : e;
+                double sum = 0.0;
 #pragma unroll
-                for (int hi = 0; hi < 2; ++hi) {
-                    const idx_t ee = hi ? eh[d] : e;
-                    double sum = 0.0;
-#pragma unroll
-                    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-                        f[d][hi][pr] = SP2(P[d], pr, ee);
-                        sum = sum + f[d][hi][pr].x;
-                        if (2 * pr + 1 < NSPEC) sum = sum + f[d][hi][pr].y;
-                    }
-                    const double fac = (sum != 0.0) ? EF(FN[d], I, NFN, URHO, ee) / sum : 1.0;
-#pragma unroll
-                    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-                        f[d][hi][pr].x = f[d][hi][pr].x * fac;
-                        f[d][hi][pr].y = f[d][hi][pr].y * fac;
-                    }
+                for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+                    f[hi][pr] = SP2(P, pr, ee);
+                    sum = sum + f[hi][pr].x;
+                    if (2 * pr + 1 < NSPEC) sum = sum + f[hi][pr].y;
                 }
+                fac[hi] = (sum != 0.0) ? EF(x.FN[d], I, NFN, URHO, ee) / sum : 1.0;
+            }
+            auto add = [&](int n, double lo, double hi) {
+                s[n] = d == 0 ? lo * ad[d] - hi * ad[d] : s[n] + lo * ad[d] - hi * ad[d];
+            };
 #pragma unroll
             for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
-                const int n = UFS + 2 * pr;
-                u[n] = u[n] + dt * flux_div(f[0][0][pr].x, f[0][1][pr].x, f[1][0][pr].x, f[1][1][pr].x, f[2][0][pr].x,
-                                            f[2][1][pr].x, a0, a1, a2, volinv);
-                if (n + 1 < NVAR)
-                    u[n + 1] = u[n + 1] + dt * flux_div(f[0][0][pr].y, f[0][1][pr].y, f[1][0][pr].y, f[1][1][pr].y,
-                                                        f[2][0][pr].y, f[2][1][pr].y, a0, a1, a2, volinv);
+                add(UFS + 2 * pr, f[0][pr].x * fac[0], f[1][pr].x * fac[1]);
+                if (2 * pr + 1 < NSPEC) add(UFS + 2 * pr + 1, f[0][pr].y * fac[0], f[1][pr].y * fac[1]);
             }
-        }
-        // URHO..UEINT as the three pairs (0,1) (2,3) (4,5) of the six faces,
-        // and the pair of Godunov p and u for p div u; UTEMP has no flux
-        double pdivu;
-        {
-            const dbl2 g0 = EF2(F0, I, NFN, FN_GP, e), g0x = EF2(F0, I, NFN, FN_GP, ex), g1 = EF2(F1, I, NFN, FN_GP, e),
-                       g1y = EF2(F1, I, NFN, FN_GP, ey), g2 = EF2(F2, I, NFN, FN_GP, e),
-                       g2z = EF2(F2, I, NFN, FN_GP, ez);
-            pdivu = HALF * (g0x.x + g0.x) * (g0x.y - g0.y) / dx0 + HALF * (g1y.x + g1.x) * (g1y.y - g1.y) / dx1 +
-                    HALF * (g2z.x + g2.x) * (g2z.y - g2.y) / dx2;
-        }
 #pragma unroll
-        for (int n = 0; n < UTEMP; n += 2) {
-            const dbl2 f0 = EF2(F0, I, NFN, n, e), f0x = EF2(F0, I, NFN, n, ex), f1 = EF2(F1, I, NFN, n, e),
-                       f1y = EF2(F1, I, NFN, n, ey), f2 = EF2(F2, I, NFN, n, e), f2z = EF2(F2, I, NFN, n, ez);
-            const double s0 = flux_div(f0.x, f0x.x, f1.x, f1y.x, f2.x, f2z.x, a0, a1, a2, volinv);
-            double s1 = flux_div(f0.y, f0x.y, f1.y, f1y.y, f2.y, f2z.y, a0, a1, a2, volinv);
-            if (n + 1 == UEINT) s1 = s1 - pdivu;
-            u[n] = u[n] + dt * s0;
-            u[n + 1] = u[n + 1] + dt * s1;
+            for (int n = 0; n < UTEMP; n += 2) {
+                const dbl2 lo = EF2(x.FN[d], I, NFN, n, e), hi = EF2(x.FN[d], I, NFN, n, e + up[d]);
+                add(n, lo.x, hi.x);
+                add(n + 1, lo.y, hi.y);
+            }
+            const dbl2 g = EF2(x.FN[d], I, NFN, FN_GP, e), gh = EF2(x.FN[d], I, NFN, FN_GP, e + up[d]);
+            const double pd = HALF * (gh.x + g.x) * (gh.y - g.y) / dxd[d];
+            pdivu = d == 0 ? pd : pdivu + pd;
+            // one direction's loads at a time (all three would hold 200
+            // registers): the next addresses wait for this direction's sums
+#pragma unroll
+            for (int n = 0; n < NVAR; ++n)
+                if (n != UTEMP) asm volatile("" : "+v"(e), "+v"(cu), "+v"(s[n]));
+        }
+        double u[NVAR];
+#pragma unroll
+        for (int n = 0; n < NVAR; ++n) u[n] = CA(x.U, I, NVAR, n, cu);  // clean(S_old), stored by K_prim
+#pragma unroll
+        for (int n = 0; n < NVAR; ++n) {
+            if (n == UTEMP) continue;
+            double q = 0.0 + s[n] * volinv;
+            if (n == UEINT) q = q - pdivu;
+            u[n] = u[n] + dt * q;
         }
         clean_cell(u, x.tab); /* Castro_advance.cpp:78 */
         if (POST) clean_cell(u, x.tab); /* post_timestep, Castro.cpp:369 */
