@@ -809,6 +809,7 @@ mc_adjoint_t *mc_adjoint_create(const int *n_cell, const double *prob_lo, const 
         delete A;
         return nullptr;
     }
+    fused_set_keep_transverse(A->F, true);  // the reverse kernels read them
     A->nD = (long)n_cell[0] * n_cell[1] * n_cell[2];
     A->nE = fused_next(A->F, 0);  // the reverse kernels index with the engine's stride
     A->max_steps = max_steps;

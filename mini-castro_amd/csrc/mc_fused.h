@@ -73,6 +73,8 @@ void fused_set_variant(FusedLevel *F, int flags);
 // no estdt), for a coarse level whose post_timestep follows a reflux
 void fused_set_defer_post(FusedLevel *F, bool defer);
 int fused_variant(const FusedLevel *F);
+// true: every step leaves the transverse fluxes F^{t|d} in memory
+void fused_set_keep_transverse(FusedLevel *F, bool keep);
 
 // The arrays a step writes besides the state (primitives, flattening,
 // traces, fluxes).  A caller may give the engine another set to write into,

@@ -58,6 +58,7 @@
 #include "mc_hydro.h"
 #include "mc_internal.h"
 #include "mc_species.h"
+#include "mc_transverse.h"
 
 namespace mc {
 
@@ -590,39 +591,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
     store_tflux_h(F, I, ep, t, o);
 }
 
-// The artificial viscosity of d-face (i,j,k) and the hydro part of its final
-// flux (apply_av, Source/Castro_hydro_nd.F90:174-245, with the reference's
-// corner-node pattern): stores the conserved fluxes and Godunov p, u of face
-// e and what the species fluxes need (K_species).
-__device__ __forceinline__ void final_hydro(const Ctx &x, const FInst &I, int d, int i, int j, int k, idx_t e,
-                                            const RiemannH &o)
-{
-    double div1;
-#define DVN(a, b, cc) EA(x.DV, I, 1, 0, eidx(I, a, b, cc))
-    if (d == 0) div1 = FOURTH * (DVN(i, j, k) + DVN(i, j + 1, k) + DVN(i, j, k + 1) + DVN(i, j + 1, k));
-    else if (d == 1) div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j, k + 1) + DVN(i + 1, j, k));
-    else div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j + 1, k) + DVN(i + 1, j + 1, k));
-#undef DVN
-    div1 = 0.1 * fmin(0.0, div1);
-    const idx_t cr = widx(I, i, j, k), cl = widx(I, i - (d == 0), j - (d == 1), k - (d == 2));
-    const double dxd = I.dx[d];
-#define AVN(n, fval) ((fval) + dxd * (div1 * (WA(x.U1, I, NU1, n, cr) - WA(x.U1, I, NU1, n, cl))))
-    const int mn = UMX + d, mt = d == 0 ? UMY : UMX, mtt = d == 2 ? UMY : UMZ;
-    double *FN = x.FN[d];
-    // momenta back in absolute order (mn = UMX + d, mt, mtt as above)
-    const double vmn = AVN(mn, o.f_mn), vmt = AVN(mt, o.f_mt), vmtt = AVN(mtt, o.f_mtt);
-    const double mx = d == 0 ? vmn : vmt;
-    const double my = d == 0 ? vmt : (d == 1 ? vmn : vmtt);
-    const double mz = d == 2 ? vmn : vmtt;
-    EF2(FN, I, NFN, URHO, e) = dbl2{AVN(URHO, o.f_rho), mx};
-    EF2(FN, I, NFN, UMY, e) = dbl2{my, mz};
-    EF2(FN, I, NFN, UEDEN, e) = dbl2{AVN(UEDEN, o.f_E), AVN(UEINT, o.f_e)};
-    EF2(FN, I, NFN, FN_GP, e) = dbl2{o.g_p, o.g_un};
-    EF2(FN, I, NFN, FN_FR, e) = dbl2{o.f_rho, o.fpl};
-    EA(FN, I, NFN, FN_DIV, e) = div1;
-#undef AVN
-}
-
 // trans2 (Source/trans.F90:250-505) + final flux + apply_av
 // (Source/Castro_hydro_nd.F90:174-245) on the d-faces of the valid region,
 // without the species.
@@ -664,8 +632,10 @@ __global__ __launch_bounds__(256) void K_final(Plan p, Ctx x)
         side[s] = to_face(o, d);
     }
     RiemannH o;
+    FaceAv av;
+    face_av(x, I, d, i, j, k, av);
     face_riemann_h(x, I, d, i, j, k, side[0], side[1], o);
-    final_hydro(x, I, d, i, j, k, e, o);
+    final_hydro(x, I, d, e, o, av);
 }
 
 // K_final by cells: the thread of cell c (bricks elongated along d,
@@ -734,8 +704,10 @@ __global__ __launch_bounds__(256) void K_finalc(Plan3 p3, Ctx x)
     __syncthreads();
     if (!has_p) return;
     RiemannH o;
+    FaceAv av;
+    face_av(x, I, d, i, j, k, av);
     face_riemann_h(x, I, d, i, j, k, lds_h[below_of(tid, st)], side_p, o);
-    final_hydro(x, I, d, i, j, k, ep, o);
+    final_hydro(x, I, d, ep, o, av);
 }
 
 // fill_hydro_source (Source/Castro_hydro_nd.F90:344-441), Saxpy and the two
@@ -1014,31 +986,31 @@ static Plan3 get_plan3(FusedLevel *F, int stage, int slab)
     return q;
 }
 
-#ifndef SPEC_LZMAX
-#define SPEC_LZMAX 64
-#endif
-// tiles of the species stage over an instance's columns, times the pairs
-static int spec_tiles(const FInst &I)
+// tiles of columns of K_species and K_transfinal over an instance
+static int column_tiles(const FInst &I)
 {
-    return ((I.n[0] + SPEC_TX - 3) / (SPEC_TX - 2)) * ((I.n[1] + SPEC_TY - 3) / (SPEC_TY - 2)) * NSPEC_PAIRS;
+    return ((I.n[0] + SPEC_TX - 3) / (SPEC_TX - 2)) * ((I.n[1] + SPEC_TY - 3) / (SPEC_TY - 2));
 }
 
-// Planes per chunk of the species stage: a chunk marches through its planes
-// and two more, so long chunks waste least, but a launch takes as many rounds
-// of a chunk as its blocks need of the chip's CUs.  Two blocks share a CU and
-// take 1.4 times as long as one alone (256^3: 3.5 us a plane of each CU with
-// two, 5 us with one); the candidate with the least total is taken.
-static int spec_chunk(const std::vector<FInst> &inst)
+// Planes per chunk of a stage that marches through columns: a chunk marches
+// through its planes and two more, so long chunks waste least, but a launch
+// takes as many rounds of a chunk as its blocks need of the chip's CUs.  Two
+// blocks share a CU and take 1.4 times as long as one alone (K_species at
+// 256^3: 3.5 us a plane of each CU with two, 5 us with one); the candidate
+// with the least total is taken.  Above 64 planes nothing is gained (256^3:
+// 14.46 ms for K_final and K_species with chunks of at most 32 and 128 planes,
+// 14.42 with 64, 14.80 with 256).
+static int column_chunk(const std::vector<FInst> &inst, int per_tile)
 {
     constexpr double cus = 256.0;
     int zmax = 0, best = 1;
     for (const FInst &I : inst) zmax = std::max(zmax, I.zn);
     double tbest = 1e300;
-    for (int lz = 1; lz <= std::min(zmax, SPEC_LZMAX); ++lz) {
+    for (int lz = 1; lz <= std::min(zmax, 64); ++lz) {
         long blocks = 0;
         for (const FInst &I : inst)
-            if (I.zn > 0) blocks += (long)spec_tiles(I) * ((I.zn + lz - 1) / lz);
-        const double rounds = blocks <= cus ? 1.4 : (double)std::max(2.0, ceil(blocks / cus));
+            if (I.zn > 0) blocks += (long)column_tiles(I) * per_tile * ((I.zn + lz - 1) / lz);
+        const double rounds = blocks <= cus ? 1.4 : std::max(2.0, ceil(blocks / cus));
         const double t = rounds * (lz + 2.5);
         if (t < tbest) {
             tbest = t;
@@ -1048,34 +1020,53 @@ static int spec_chunk(const std::vector<FInst> &inst)
     return best;
 }
 
-// block table of the species stage over a slab
-static SpecPlan spec_plan(FusedLevel *F, int slab, int &nblocks)
+// block table of such a stage over a slab, with per_tile blocks for a tile's
+// chunk
+static SpecPlan column_plan(FusedLevel *F, int slab, int per_tile, int &nblocks)
 {
     const FInst *tab = F->sinst[slab];
     for (auto &sb : F->specs)
-        if (sb.slab == slab) {
+        if (sb.slab == slab && sb.per_tile == per_tile) {
             nblocks = sb.nblocks;
             return SpecPlan{tab, sb.blk0, F->ninst, sb.lz};
         }
     FusedLevel::SpecBuf sb;
     sb.slab = slab;
-    sb.lz = spec_chunk(F->hsinst[slab]);
+    sb.per_tile = per_tile;
+    sb.lz = column_chunk(F->hsinst[slab], per_tile);
     std::vector<int> b0(F->ninst + 1);
     int acc = 0;
     for (int m = 0; m < F->ninst; ++m) {
         b0[m] = acc;
         const FInst &I = F->hsinst[slab][m];
-        if (I.zn > 0) acc += spec_tiles(I) * ((I.zn + sb.lz - 1) / sb.lz);
+        if (I.zn > 0) acc += column_tiles(I) * per_tile * ((I.zn + sb.lz - 1) / sb.lz);
     }
     b0[F->ninst] = acc;
     nblocks = sb.nblocks = acc;
-    if (check_hip(hipMalloc(&sb.blk0, sizeof(int) * (F->ninst + 1)), "hipMalloc(species plan)") ||
+    if (check_hip(hipMalloc(&sb.blk0, sizeof(int) * (F->ninst + 1)), "hipMalloc(column plan)") ||
         check_hip(hipMemcpy(sb.blk0, b0.data(), sizeof(int) * (F->ninst + 1), hipMemcpyHostToDevice), "plan h2d")) {
         nblocks = 0;
         return SpecPlan{nullptr, nullptr, 0, 0};
     }
     F->specs.push_back(sb);
     return SpecPlan{tab, sb.blk0, F->ninst, sb.lz};
+}
+
+// Whether a step that runs the transverse stage by cells joins it with the
+// final fluxes (K_transfinal).  Its blocks march through few planes on a small
+// level and wait for memory with nothing else on their CU; from some 200,000
+// cells a launch it is the faster side, also for thin members (us, the stages
+// joined against K_trans1c, K_final and K_species: 40^3 121 : 107, 48^3
+// 184 : 172, 56^3 227 : 224, 30 x 30 x 200 331 : 328, 128 x 40 x 40 291 : 296,
+// 64^3 373 : 407, 80^3 570 : 682, 96^3 1001 : 1171, 256^3 15.7 : 19.0 ms;
+// a step of 1000 members of 4^3 17.6 : 17.8 ms).
+constexpr long JOINT_MIN = 200000;
+static bool joins_transverse(const FusedLevel *F, int slab)
+{
+    if ((F->variant & FV_FACE_TRANS1) || F->keep_transverse) return false;
+    long cells = 0;
+    for (const FInst &I : F->hsinst[slab]) cells += (long)I.n[0] * I.n[1] * I.zn;
+    return cells >= JOINT_MIN;
 }
 
 int plan_blocks(FusedLevel *F, const Plan &p)
@@ -1094,14 +1085,27 @@ namespace mc {
 static void launch_species(FusedLevel *F, hipStream_t s, int slab)
 {
     int nb = 0;
-    const SpecPlan p = spec_plan(F, slab, nb);
-    if (nb > 0)
-        hipLaunchKernelGGL(K_species, dim3(nb), dim3(SPEC_TX * SPEC_TY), 0, s, p, F->ctx);
+    const SpecPlan p = column_plan(F, slab, NSPEC_PAIRS, nb);
+    if (nb > 0) hipLaunchKernelGGL(K_species, dim3(nb), dim3(SPEC_TX * SPEC_TY), 0, s, p, F->ctx);
+}
+
+static void launch_transfinal(FusedLevel *F, hipStream_t s, int slab)
+{
+    int nb = 0;
+    const SpecPlan p = column_plan(F, slab, 1, nb);
+    if (nb > 0) hipLaunchKernelGGL(K_transfinal, dim3(nb), dim3(SPEC_TX * SPEC_TY), 0, s, p, F->ctx);
 }
 
 static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, int slab = 0)
 {
     F->ctx.tab = eos_table();
+    if (stage == ST_TRANS1C || stage == ST_FINAL || stage == ST_FINALC)
+        if (joins_transverse(F, slab)) {
+            // the transverse stage has made the final fluxes: the species are left
+            if (stage == ST_TRANS1C) launch_transfinal(F, s, slab);
+            else launch_species(F, s, slab);
+            return;
+        }
     if (overlap_stage(stage)) {
         // the directions / pairs interleaved block by block; one with fewer
         // bricks than the largest leaves its last blocks idle
@@ -1657,7 +1661,8 @@ int fused_steps(FusedLevel *F, int nsteps, double stop_time, hipStream_t s, bool
                 int nb;
                 if (overlap_stage(st)) (void)get_plan3(F, st, sl);
                 else (void)get_plan(F, st, sl);
-                if (st == ST_FINAL) (void)spec_plan(F, sl, nb);
+                if (st == ST_FINAL) (void)column_plan(F, sl, NSPEC_PAIRS, nb);
+                if (st == ST_TRANS1C && joins_transverse(F, sl)) (void)column_plan(F, sl, 1, nb);
             }
         if (check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture")) return -1;
         enqueue_step(F, stop_time, s);
@@ -1747,6 +1752,8 @@ void fused_set_variant(FusedLevel *F, int flags)
 }
 
 int fused_variant(const FusedLevel *F) { return F->variant; }
+
+void fused_set_keep_transverse(FusedLevel *F, bool keep) { F->keep_transverse = keep; }
 
 void fused_set_defer_post(FusedLevel *F, bool defer)
 {
@@ -1903,7 +1910,8 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
     // every stage of every kernel variant; the faster kernel of each
     // alternative is chosen below
     const std::vector<int> tuned = {ST_PRIM,   ST_FLAT,  ST_TRACE,  ST_FLUX1,  ST_TFLUX,
-                                    ST_TRANS1, ST_TRANS1C, ST_FINAL, ST_FINALC, ST_UPDATE};
+                                    ST_TRANS1, ST_FINAL, ST_FINALC, ST_TRANS1C, ST_UPDATE};
+    const int variant0 = F->variant;
     double tb[NSTAGE] = {0.0};
     if (bricks)
         for (int st = 0; st < NSTAGE; ++st) fused_get_tiling(F, st, bricks + 3 * st);
@@ -1912,6 +1920,10 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
     for (int st : tuned) {
         if (rc) break;
         const bool writes_state = st == ST_PRIM || st == ST_UPDATE;
+        // the final stages by themselves follow the face-by-face transverse
+        // stage; the one by cells may have joined them (below)
+        F->variant = st == ST_TRANS1C ? 0 : (int)FV_FACE_TRANS1;
+        const bool joined = st == ST_TRANS1C && joins_transverse(F, 0);
         KernelTiling best = F->tiling[st];
         double tbest = 1e300;
         std::vector<KernelTiling> cands(std::begin(tune_cand), std::end(tune_cand));
@@ -1964,6 +1976,7 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
         };
         for (const KernelTiling &c : cands) {
             if (!fused_tiling_ok(st, c.bx, c.by, c.bz)) continue;
+            if (joined && tbest < 1e300) break;  // its tiles are its own
             const double t = time_tiling(c);
             if (t < 0) break;
             if (t < tbest) {
@@ -1973,7 +1986,7 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
         }
         // then the brick order of the best brick: groups of brick planes in z
         for (int zg : {2, 4, 8}) {
-            if (rc) break;
+            if (rc || joined) break;
             KernelTiling c = best;
             c.zg = zg;
             const double t = time_tiling(c);
@@ -1983,6 +1996,21 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
             }
         }
         F->tiling[st] = best;
+        if (joined && !rc) {
+            // its share: the launch and the species that are left, less the
+            // faster final stage it replaces
+            float one = 0.f;
+            double sp = 0.0;
+            for (int r = 0; r < reps && !rc; ++r) {
+                (void)hipEventRecord(e0, s);
+                launch_stage(F, ST_FINAL, s);
+                (void)hipEventRecord(e1, s);
+                rc = check_hip(hipEventSynchronize(e1), "autotune sync") ||
+                     check_hip(hipEventElapsedTime(&one, e0, e1), "hipEventElapsedTime");
+                sp += one;
+            }
+            tbest = std::max(tbest + sp / reps - std::min(tb[ST_FINAL], tb[ST_FINALC]), 1e-6);
+        }
         tb[st] = tbest;
         if (bricks) {
             bricks[3 * st] = best.bx;
@@ -1991,6 +2019,7 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
         }
         if (best_ms) best_ms[st] = tbest;
     }
+    F->variant = variant0;
     if (!rc) {
         int v = 0;
         if (tb[ST_TRACE] + tb[ST_FLUX1] < tb[ST_TFLUX]) v |= FV_SPLIT_TRACE;

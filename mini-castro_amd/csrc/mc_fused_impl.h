@@ -433,6 +433,44 @@ __device__ __forceinline__ double species_fac(const SpeciesPairs &XN, idx_t e, d
     return (sum != 0.0) ? frho / sum : 1.0;
 }
 
+// What apply_av (Source/Castro_hydro_nd.F90:174-245, with the reference's
+// corner-node pattern) needs of the zones at d-face (i,j,k): the divergence
+// and the differences of the conserved state, read together
+struct FaceAv {
+    double div1, d[UEINT + 1];
+};
+__device__ __forceinline__ void face_av(const Ctx &x, const FInst &I, int d, int i, int j, int k, FaceAv &v)
+{
+    double div1;
+#define DVN(a, b, cc) EA(x.DV, I, 1, 0, eidx(I, a, b, cc))
+    if (d == 0) div1 = FOURTH * (DVN(i, j, k) + DVN(i, j + 1, k) + DVN(i, j, k + 1) + DVN(i, j + 1, k));
+    else if (d == 1) div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j, k + 1) + DVN(i + 1, j, k));
+    else div1 = FOURTH * (DVN(i, j, k) + DVN(i + 1, j, k) + DVN(i, j + 1, k) + DVN(i + 1, j + 1, k));
+#undef DVN
+    v.div1 = 0.1 * fmin(0.0, div1);
+    const idx_t cr = widx(I, i, j, k), cl = widx(I, i - (d == 0), j - (d == 1), k - (d == 2));
+#pragma unroll
+    for (int n = 0; n <= UEINT; ++n) v.d[n] = WA(x.U1, I, NU1, n, cr) - WA(x.U1, I, NU1, n, cl);
+}
+// The hydro part of d-face e's final flux: stores the conserved fluxes and
+// Godunov p, u, and what the species fluxes need (K_species).
+__device__ __forceinline__ void final_hydro(const Ctx &x, const FInst &I, int d, idx_t e, const RiemannH &o,
+                                            const FaceAv &v)
+{
+    const double dxd = I.dx[d];
+#define AVN(n, fval) ((fval) + dxd * (v.div1 * v.d[n]))
+    const double fx = d == 0 ? o.f_mn : o.f_mt, fy = d == 0 ? o.f_mt : (d == 1 ? o.f_mn : o.f_mtt),
+                 fz = d == 2 ? o.f_mn : o.f_mtt;
+    double *FN = x.FN[d];
+    EF2(FN, I, NFN, URHO, e) = dbl2{AVN(URHO, o.f_rho), AVN(UMX, fx)};
+    EF2(FN, I, NFN, UMY, e) = dbl2{AVN(UMY, fy), AVN(UMZ, fz)};
+    EF2(FN, I, NFN, UEDEN, e) = dbl2{AVN(UEDEN, o.f_E), AVN(UEINT, o.f_e)};
+    EF2(FN, I, NFN, FN_GP, e) = dbl2{o.g_p, o.g_un};
+    EF2(FN, I, NFN, FN_FR, e) = dbl2{o.f_rho, o.fpl};
+    EA(FN, I, NFN, FN_DIV, e) = v.div1;
+#undef AVN
+}
+
 static __constant__ int c_pair_t[6] = {1, 2, 0, 2, 0, 1};   // state (face) direction
 static __constant__ int c_pair_d[6] = {0, 0, 1, 1, 2, 2};   // flux direction
 
@@ -472,9 +510,10 @@ struct FusedLevel {
         int nblocks = 0;
     };
     std::vector<PlanBuf> plans;
-    // block tables of the species stage, one per slab
+    // block tables of the stages that march through columns (K_species,
+    // K_transfinal: per tile one block of each species pair, or one), per slab
     struct SpecBuf {
-        int slab, lz, nblocks = 0;
+        int slab, per_tile, lz, nblocks = 0;
         int *blk0 = nullptr;
     };
     std::vector<SpecBuf> specs;
@@ -487,6 +526,9 @@ struct FusedLevel {
     // K_update without post_timestep's clean and estdt (a coarse level of a
     // flux register, whose post_timestep runs after the reflux)
     bool defer_post = false;
+    // the transverse fluxes are read after the step (the adjoint's engine):
+    // K_transfinal, which keeps them on the chip, is not used
+    bool keep_transverse = false;
     // z-slabs of the face stages: planes per slab (0: the whole instance),
     // slab count, and one instance table per slab (zlo, zn set; slab 0 of a
     // whole-instance engine is `inst` itself)
