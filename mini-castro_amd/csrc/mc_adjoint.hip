@@ -14,9 +14,11 @@
 //   A_flat    cells+1 flattening, node-centred div(u)
 //   A_prim    cells   ctoprim, clean_state x2
 //
-// Each thread re-evaluates its forward stencil point and scatters the input
-// adjoints with hardware FP64 atomic adds (the forward reads through the
-// boundary map, so the adjoint accumulates into the mapped cells).  The
+// Each thread re-evaluates its forward stencil point.  What a stage owes the
+// fluxes it read is stored zone by zone and gathered by the stage that made
+// them, and states and zones are written by their one owner; what is left,
+// the zones a trace, the viscosity or the boundary map reaches, is scattered
+// with hardware FP64 atomic adds.  The
 // adjoint carries the hydro components of the state (rho, rho u, rho v,
 // rho w, rho E, rho e); see mc_adjoint.h for why T and the species are
 // constants of the differentiated map.
@@ -24,6 +26,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/mc_castro.h"
@@ -40,15 +43,20 @@ namespace mc {
 
 // adjoint component layouts
 enum { SB_RHO = 0, SB_U, SB_V, SB_W, SB_P, SB_RE, NSB };            // interface states
-enum { FB_RHO = 0, FB_MX, FB_MY, FB_MZ, FB_E, FB_GP, FB_GU, NFB };  // F^d, F^{t|d}
+enum { ZB_PGP = UEDEN + 1, ZB_PGM, ZB_UGP, ZB_UGM, NZB };  // fluxes across a zone
 enum { NB_RHO = 0, NB_MX, NB_MY, NB_MZ, NB_E, NB_EI, NB_GP, NB_GU, NNB };  // final fluxes
 
 struct ACtx {
     const double *Uold;  // checkpoint of the step (NVAR, cell layout)
     double *Ub;          // adjoint of the step's output state (NHB, cell layout)
     double *Ubo;         // adjoint of the step's input state (NHB, cell layout)
-    double *U1b, *Qb, *FLb, *DVb;
-    double *SMb[3], *SPb[3], *FDb[3], *FTb[6], *FNb[3];
+    double *Sb;          // adjoint of the update's sources, dt times (NHB, cell layout)
+    double *U1b, *Qb, *DVb;
+    double *QD[3];       // the primitives' share of direction d's traces (NQB, cell layout)
+    double *FLb[3], *SMb[3], *SPb[3];
+    double *ZF[6], *ZT[6];  // of F^{t|d} and of F^d (pair t, d), by the zone between the two faces
+    double *CG[3];          // c and Gamma_1, by the zone, from the states of direction d ..
+    double *CGF[3];         // .. and from F^d's faces: left c, Gamma_1, right c, Gamma_1
 };
 
 // device-scope FP64 atomic add (the hardware global_atomic_add_f64)
@@ -60,19 +68,6 @@ __device__ __forceinline__ void aadd(gdouble *p, double v)
         }
     }
 }
-// plain read-add-write, for an entry no other thread of the launch touches
-__device__ __forceinline__ void radd(gdouble *p, double v)
-{
-    if (v != 0.0) *p = *p + v;
-}
-// add into an adjoint entry: SOLE = this thread is the entry's only writer
-// in the launch (no atomic needed)
-template <bool SOLE>
-__device__ __forceinline__ void badd(gdouble *p, double v)
-{
-    if (SOLE) radd(p, v);
-    else aadd(p, v);
-}
 __device__ __forceinline__ gdouble *EAp(double *a, const FInst &I, int C, int c, idx_t idx)
 {
     return &at(a + ((long)C * I.offE + (long)c * I.nE), idx);
@@ -81,9 +76,6 @@ __device__ __forceinline__ gdouble *CAp(double *a, const FInst &I, int C, int c,
 {
     return &at(a + ((long)C * I.offD + (long)c * I.nD), idx);
 }
-
-// conserved-state adjoint component h -> flux component in the FN array
-__device__ __forceinline__ int fn_comp(int h) { return hb_comp(h); }
 
 // ------------------------------------------------------------------ A_update
 __global__ __launch_bounds__(256) void A_update(Plan p, Ctx x, ACtx a)
@@ -151,46 +143,28 @@ __global__ __launch_bounds__(256) void A_update(Plan p, Ctx x, ACtx a)
 #pragma unroll
     for (int h = 0; h < NHB; ++h) CA(a.Ubo, I, NHB, h, c) = ub[h];
 
-    const double ad[3] = {a0, a1, a2};
-    const idx_t ep[3] = {ex, ey, ez};
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        double *FB = a.FNb[d];
-#pragma unroll
-        for (int h = 0; h < NHB; ++h) {
-            const double g = sb[h] * ad[d] * volinv;
-            aadd(EAp(FB, I, NNB, h, e), g);
-            aadd(EAp(FB, I, NNB, h, ep[d]), -g);
-        }
-        // pdivu term of rho e: s -= 0.5 (GP+ + GP-) (GU+ - GU-) / dx_d
-        double *F = x.FN[d];
-        const double gpp = EF(F, I, NFN, FN_GP, ep[d]), gpm = EF(F, I, NFN, FN_GP, e);
-        const double gup = EF(F, I, NFN, FN_GU, ep[d]), gum = EF(F, I, NFN, FN_GU, e);
-        const double b = -sb[HB_EI] / I.dx[d];
-        aadd(EAp(FB, I, NNB, NB_GP, ep[d]), b * HALF * (gup - gum));
-        aadd(EAp(FB, I, NNB, NB_GP, e), b * HALF * (gup - gum));
-        aadd(EAp(FB, I, NNB, NB_GU, ep[d]), b * HALF * (gpp + gpm));
-        aadd(EAp(FB, I, NNB, NB_GU, e), -b * HALF * (gpp + gpm));
-    }
+    for (int h = 0; h < NHB; ++h) CA(a.Sb, I, NHB, h, c) = sb[h];
 }
 
 // ------------------------------------------------------------------ helpers
-// Riemann adjoint at face (i,j,k) of direction d; the c / gamma_c adjoints go
-// to the two cells of the face.
-__device__ __forceinline__ void face_riemann_hb(const Ctx &x, const ACtx &a, const FInst &I, int d, int i, int j,
-                                                int k, const FaceH &L, const FaceH &R, const RiemannHB &rb,
-                                                FaceHB &Lb, FaceHB &Rb)
+// Riemann adjoint at face (i,j,k) of direction d; the c / gamma_c adjoints of
+// its two cells in cg: left c, right c, left gamma_c, right gamma_c.
+__device__ __forceinline__ void face_riemann_hb(const Ctx &x, const FInst &I, int d, int i, int j, int k,
+                                                const FaceH &L, const FaceH &R, const RiemannHB &rb, FaceHB &Lb,
+                                                FaceHB &Rb, double *cg)
 {
     const idx_t cr = cidx(I, i, j, k);
     const idx_t cl = cidx(I, i - (d == 0), j - (d == 1), k - (d == 2));
-    double cLb = 0.0, cRb = 0.0, glb = 0.0, grb = 0.0;
+    Lb = Rb = FaceHB{0, 0, 0, 0, 0, 0};
+    cg[0] = cg[1] = cg[2] = cg[3] = 0.0;
     riemann_hydro_b(L, R, CA(x.Q, I, NFQ, FQ_C, cl), CA(x.Q, I, NFQ, FQ_C, cr), CA(x.Q, I, NFQ, FQ_G, cl),
-                    CA(x.Q, I, NFQ, FQ_G, cr), rb, Lb, Rb, cLb, cRb, glb, grb);
-    aadd(CAp(a.Qb, I, NQB, QB_C, cl), cLb);
-    aadd(CAp(a.Qb, I, NQB, QB_C, cr), cRb);
-    aadd(CAp(a.Qb, I, NQB, QB_G, cl), glb);
-    aadd(CAp(a.Qb, I, NQB, QB_G, cr), grb);
+                    CA(x.Q, I, NFQ, FQ_G, cr), rb, Lb, Rb, cg[0], cg[1], cg[2], cg[3]);
 }
+
+// a value by direction (of values: a choice between members would keep their
+// structure in memory)
+__device__ __forceinline__ double pick(int d, double x, double y, double z) { return d == 0 ? +x : (d == 1 ? +y : +z); }
 
 // FaceHB (velocities permuted to direction d) -> absolute-order state adjoint
 __device__ __forceinline__ QStateHB from_faceb(const FaceHB &f, int d)
@@ -200,247 +174,423 @@ __device__ __forceinline__ QStateHB from_faceb(const FaceHB &f, int d)
     o.p = f.p;
     o.rhoe = f.rhoe;
     // to_face: un = (u,v,w)[d]; ut = d==0 ? v : u; utt = d==2 ? v : w
-    double uvw[3] = {0.0, 0.0, 0.0};
-    uvw[d] += f.un;
-    uvw[d == 0 ? 1 : 0] += f.ut;
-    uvw[d == 2 ? 1 : 2] += f.utt;
-    o.u = uvw[0];
-    o.v = uvw[1];
-    o.w = uvw[2];
+    o.u = pick(d, f.un, f.ut, f.ut);
+    o.v = pick(d, f.ut, f.un, f.utt);
+    o.w = pick(d, f.utt, f.utt, f.un);
     return o;
 }
 
-template <bool SOLE = false>
-__device__ __forceinline__ void add_stateb(double *S, const FInst &I, idx_t e, const QInHB &b)
+// The adjoints of states and of zones' fluxes lie in pairs as the face arrays
+// do (EF2): one access moves two components (A_flux1 at 64^3: 133 us, by single
+// components 168).
+__device__ __forceinline__ void load_stateb(double *S, const FInst &I, idx_t e, QInHB &b)
 {
-    badd<SOLE>(EAp(S, I, NSB, SB_RHO, e), b.rho);
-    badd<SOLE>(EAp(S, I, NSB, SB_U, e), b.u);
-    badd<SOLE>(EAp(S, I, NSB, SB_V, e), b.v);
-    badd<SOLE>(EAp(S, I, NSB, SB_W, e), b.w);
-    badd<SOLE>(EAp(S, I, NSB, SB_P, e), b.p);
-    badd<SOLE>(EAp(S, I, NSB, SB_RE, e), b.rhoe);
+    const dbl2 ru = EF2(S, I, NSB, SB_RHO, e), vw = EF2(S, I, NSB, SB_V, e), pe = EF2(S, I, NSB, SB_P, e);
+    b = QInHB{ru.x, ru.y, vw.x, vw.y, pe.x, pe.y};
+}
+__device__ __forceinline__ void store_stateb(double *S, const FInst &I, idx_t e, const QInHB &b)
+{
+    EF2(S, I, NSB, SB_RHO, e) = dbl2{b.rho, b.u};
+    EF2(S, I, NSB, SB_V, e) = dbl2{b.v, b.w};
+    EF2(S, I, NSB, SB_P, e) = dbl2{b.p, b.rhoe};
 }
 
-template <bool SOLE = false>
+// into a d-face state that this thread alone has in the launch
 __device__ __forceinline__ void add_faceb(double *S, const FInst &I, idx_t e, int d, const FaceHB &f)
 {
-    const int un = SB_U + d, ut = d == 0 ? SB_V : SB_U, utt = d == 2 ? SB_V : SB_W;
-    badd<SOLE>(EAp(S, I, NSB, SB_RHO, e), f.rho);
-    badd<SOLE>(EAp(S, I, NSB, un, e), f.un);
-    badd<SOLE>(EAp(S, I, NSB, ut, e), f.ut);
-    badd<SOLE>(EAp(S, I, NSB, utt, e), f.utt);
-    badd<SOLE>(EAp(S, I, NSB, SB_P, e), f.p);
-    badd<SOLE>(EAp(S, I, NSB, SB_RE, e), f.rhoe);
+    const QStateHB o = from_faceb(f, d);
+    QInHB b;
+    load_stateb(S, I, e, b);
+    store_stateb(S, I, e, QInHB{b.rho + o.rho, b.u + o.u, b.v + o.v, b.w + o.w, b.p + o.p, b.rhoe + o.rhoe});
 }
 
-// adjoint of a transverse-stage flux entry (URHO..UEDEN + Godunov p, u)
-__device__ __forceinline__ void add_tfluxb(double *FB, const FInst &I, idx_t e, const double *vb, double gpb,
-                                           double gub)
+// Adjoint of the fluxes across a zone (ZB_*): the conserved fluxes enter as
+// right less left, so one set serves both faces; Godunov p and u each side.
+// (in pairs: two of momenta and rho, p and u of the high face, of the low; E)
+__device__ __forceinline__ void store_zoneb(double *Z, const FInst &I, idx_t e, const double (&v)[NZB])
 {
-#pragma unroll
-    for (int n = 0; n <= UEDEN; ++n) aadd(EAp(FB, I, NFB, n, e), vb[n]);
-    aadd(EAp(FB, I, NFB, FB_GP, e), gpb);
-    aadd(EAp(FB, I, NFB, FB_GU, e), gub);
+    EF2(Z, I, NZB, 0, e) = dbl2{v[URHO], v[UMX]};
+    EF2(Z, I, NZB, 2, e) = dbl2{v[UMY], v[UMZ]};
+    EA(Z, I, NZB, 8, e) = v[UEDEN];
+    EF2(Z, I, NZB, 4, e) = dbl2{v[ZB_PGP], v[ZB_UGP]};
+    EF2(Z, I, NZB, 6, e) = dbl2{v[ZB_PGM], v[ZB_UGM]};
 }
-
-// Riemann output adjoints stored in a transverse-flux adjoint entry
-__device__ __forceinline__ RiemannHB load_tfluxb(double *FB, const FInst &I, idx_t e, int d)
+struct FluxB {
+    double rho, mx, my, mz, E, gp, gu;
+};
+// added to v: what face e owes the zones on its two sides, el and e; has_l,
+// has_r: which of them had it
+__device__ __forceinline__ void gather_zoneb(double *Z, const FInst &I, idx_t el, idx_t e, bool has_l, bool has_r,
+                                             FluxB &v)
 {
-    const int mn = FB_MX + d, mt = d == 0 ? FB_MY : FB_MX, mtt = d == 2 ? FB_MY : FB_MZ;
+    if (has_l) {
+        const dbl2 f = EF2(Z, I, NZB, 0, el), g = EF2(Z, I, NZB, 2, el), h = EF2(Z, I, NZB, 4, el);
+        v.rho += f.x;
+        v.mx += f.y;
+        v.my += g.x;
+        v.mz += g.y;
+        v.E += EA(Z, I, NZB, 8, el);
+        v.gp += h.x;
+        v.gu += h.y;
+    }
+    if (has_r) {
+        const dbl2 f = EF2(Z, I, NZB, 0, e), g = EF2(Z, I, NZB, 2, e), h = EF2(Z, I, NZB, 6, e);
+        v.rho -= f.x;
+        v.mx -= f.y;
+        v.my -= g.x;
+        v.mz -= g.y;
+        v.E -= EA(Z, I, NZB, 8, e);
+        v.gp += h.x;
+        v.gu += h.y;
+    }
+}
+// as the adjoint of a Riemann problem's outputs on a d-face
+__device__ __forceinline__ RiemannHB riemannb_of(const FluxB &v, int d)
+{
     RiemannHB r;
-    r.f_rho = EA(FB, I, NFB, FB_RHO, e);
-    r.f_mn = EA(FB, I, NFB, mn, e);
-    r.f_mt = EA(FB, I, NFB, mt, e);
-    r.f_mtt = EA(FB, I, NFB, mtt, e);
-    r.f_E = EA(FB, I, NFB, FB_E, e);
+    r.f_rho = v.rho;
+    r.f_mn = pick(d, v.mx, v.my, v.mz);
+    r.f_mt = pick(d, v.my, v.mx, v.mx);
+    r.f_mtt = pick(d, v.mz, v.mz, v.my);
+    r.f_E = v.E;
     r.f_e = 0.0;
-    r.g_p = EA(FB, I, NFB, FB_GP, e);
-    r.g_un = EA(FB, I, NFB, FB_GU, e);
+    r.g_p = v.gp;
+    r.g_un = v.gu;
     return r;
 }
 
-// ------------------------------------------------------------------ A_final
-__global__ __launch_bounds__(256) void A_final(Plan p, Ctx x, ACtx a)
+// What follows is addressed through e, which waits for f: the forward values
+// are read again behind the Riemann problem instead of being kept across it.
+__device__ __forceinline__ void behind(idx_t &e, FaceHB &f)
 {
-    int m, i, j, k;
-    int sub_;
-    if (!plan_cell_sub(p, 3, sub_, m, i, j, k)) return;
-    const int d = sub_;
-    const FInst &I = p.inst[m];
-    const int c[3] = {i, j, k};
-    for (int q = 0; q < 3; ++q) {
-        if (c[q] < 0) return;
-        if (q != d && c[q] > I.n[q] - 1) return;
-    }
-    const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-    const int ed[3] = {d == 0, d == 1, d == 2}, e1[3] = {t1 == 0, t1 == 1, t1 == 2}, e2[3] = {t2 == 0, t2 == 1, t2 == 2};
-    const double dt = x.dt_cur[m];
-    const double h2 = 0.5 * dt / I.dx[t1], h3 = 0.5 * dt / I.dx[t2];
-    const idx_t e = eidx(I, i, j, k);
-    const int p2 = pair_index(t1, t2), p3 = pair_index(t2, t1);
-    double *F2 = x.FT[p2], *F3 = x.FT[p3];
-    FaceH side[2];
-    idx_t l2[2], r2[2], r3[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int sh = s - 1;
-        const int il = i + sh * ed[0], jl = j + sh * ed[1], kl = k + sh * ed[2];
-        l2[s] = eidx(I, il, jl, kl);
-        r2[s] = eidx(I, il + e1[0], jl + e1[1], kl + e1[2]);
-        r3[s] = eidx(I, il + e2[0], jl + e2[1], kl + e2[2]);
-        QInH lq;
-        load_qin_h(s == 0 ? x.SM[d] : x.SP[d], I, e, lq);
-        double f2r[UEDEN + 1], f2l[UEDEN + 1], f3r[UEDEN + 1], f3l[UEDEN + 1], pg2p, ug2p, pg2m, ug2m, pg3p, ug3p,
-            pg3m, ug3m;
-        load_tflux_h(F2, I, r2[s], f2r, pg2p, ug2p);
-        load_tflux_h(F2, I, l2[s], f2l, pg2m, ug2m);
-        load_tflux_h(F3, I, r3[s], f3r, pg3p, ug3p);
-        load_tflux_h(F3, I, l2[s], f3l, pg3m, ug3m);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, il, jl, kl));
-        const QStateH o = trans2_hydro(lq, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m, gamc,
-                                       h2, h3);
-        side[s] = to_face(o, d);
-    }
-    // artificial viscosity (forward: Source/Castro_hydro_nd.F90:174-245)
-    idx_t nodes[4];
+    asm volatile("" : "+v"(e), "+v"(f.rho), "+v"(f.un), "+v"(f.ut), "+v"(f.utt), "+v"(f.p), "+v"(f.rhoe));
+}
+__device__ __forceinline__ void behind(idx_t &e, QInHB &f)
+{
+    asm volatile("" : "+v"(e), "+v"(f.rho), "+v"(f.u), "+v"(f.v), "+v"(f.w), "+v"(f.p), "+v"(f.rhoe));
+}
+
+// Bricks of L zones along a direction d, W across (256 threads: (L, W, 1) for
+// x, (W, L, 1) for y, (W, 1, L) for z), over the zones -1..n along d and
+// -ring..n-1+ring across; consecutive bricks share ovl zones along d.
+struct Lines {
+    int ring, ovl;
+    int L[3], W[3], nb0[3], nb1[3], nb[3];
+};
+__device__ __forceinline__ bool line_cell(const Lines &q, int d, int lb, const FInst &I, int &i, int &j, int &k, int &l)
+{
+    const int L = q.L[d], W = q.W[d], t = threadIdx.x, r = q.ring;
+    const int b0 = lb % q.nb0[d], b1 = (lb / q.nb0[d]) % q.nb1[d], b2 = lb / (q.nb0[d] * q.nb1[d]);
+    const int s = L - q.ovl;
     if (d == 0) {
-        nodes[0] = eidx(I, i, j, k);
-        nodes[1] = eidx(I, i, j + 1, k);
-        nodes[2] = eidx(I, i, j, k + 1);
-        nodes[3] = eidx(I, i, j + 1, k);
-    } else if (d == 1) {
-        nodes[0] = eidx(I, i, j, k);
-        nodes[1] = eidx(I, i + 1, j, k);
-        nodes[2] = eidx(I, i, j, k + 1);
-        nodes[3] = eidx(I, i + 1, j, k);
+        l = t % L;
+        i = b0 * s + l - 1;
+        j = b1 * W + t / L - r;
+        k = b2 - r;
     } else {
-        nodes[0] = eidx(I, i, j, k);
-        nodes[1] = eidx(I, i + 1, j, k);
-        nodes[2] = eidx(I, i, j + 1, k);
-        nodes[3] = eidx(I, i + 1, j + 1, k);
+        l = t / W;
+        i = b0 * W + t % W - r;
+        j = d == 1 ? b1 * s + l - 1 : b1 - r;
+        k = d == 1 ? b2 - r : b2 * s + l - 1;
     }
-    const double draw = FOURTH * (EA(x.DV, I, 1, 0, nodes[0]) + EA(x.DV, I, 1, 0, nodes[1]) +
-                                  EA(x.DV, I, 1, 0, nodes[2]) + EA(x.DV, I, 1, 0, nodes[3]));
-    const double div1 = 0.1 * fmin(0.0, draw);
-    const idx_t cr = cidx(I, i, j, k), cl = cidx(I, i - ed[0], j - ed[1], k - ed[2]);
-    const double dxd = I.dx[d];
-    double fnb[NNB];
-#pragma unroll
-    for (int q = 0; q < NNB; ++q) fnb[q] = EA(a.FNb[d], I, NNB, q, e);
-    double div1_b = 0.0;
-#pragma unroll
-    for (int h = 0; h < NHB; ++h) {
-        const int n = hb_comp(h);
-        const double ur = CA(x.U1, I, NU1, n, cr), ul = CA(x.U1, I, NU1, n, cl);
-        div1_b += fnb[h] * dxd * (ur - ul);
-        const double g = fnb[h] * dxd * div1;
-        aadd(CAp(a.U1b, I, NHB, h, cr), g);
-        aadd(CAp(a.U1b, I, NHB, h, cl), -g);
+    const int h0 = I.n[0] + (d == 0 ? 1 : r), h1 = I.n[1] + (d == 1 ? 1 : r), h2 = I.n[2] + (d == 2 ? 1 : r);
+    return i < h0 && j < h1 && k < h2;
+}
+
+// ------------------------------------------------------------------ A_final
+// Final fluxes of direction d: apply_av, the Riemann problem, trans2.  The
+// thread of zone c re-evaluates its two d-states (the plus state of d-face c,
+// the minus state of d-face c + 1) from the zone's transverse fluxes, read
+// once; the minus side goes up through LDS, the thread of a face reverses its
+// Riemann problem and its viscosity, and the minus side's share comes back
+// down.  Bricks share two zones along d, so that one thread has both faces of
+// every zone and owns what the zone gives.  64^3: 250 us; by faces, with an
+// atomic add for each of the 74 adjoints a face gives, 603 (atomics come at 92
+// to 97 a nanosecond).  Two waves a SIMD wait for memory now: without the
+// stores it takes 181, without the Riemann problem 216.
+__global__ __launch_bounds__(256) void A_final(Lines q, const FInst *inst, Ctx x, ACtx a)
+{
+    __shared__ double ls[6][256], lr[14][256];
+    int lb = logical_block();
+    const int d = lb % 3;
+    lb /= 3;
+    if (lb >= q.nb[d]) return;  // the whole block
+    const FInst &I = inst[0];
+    int i, j, k, l;
+    const bool ok = line_cell(q, d, lb, I, i, j, k, l);
+    const int tid = threadIdx.x, st = d == 0 ? 1 : q.W[d], top = q.L[d] - 1, nd = I.n[d];
+    const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
+    const int cd = d == 0 ? i : (d == 1 ? j : k);
+    const int ei = d == 0, ej = d == 1, ek = d == 2;
+    const bool has_p = ok && cd >= 0, has_m = ok && cd + 1 <= nd;  // the zone's plus and minus states
+    const idx_t ep = eidx(I, i, j, k), em = eidx(I, i + ei, j + ej, k + ek);
+    const idx_t r2 = eidx(I, i + (t1 == 0), j + (t1 == 1), k), r3 = eidx(I, i, j + (t2 == 1), k + (t2 == 2));
+    const double dt = x.dt_cur[0];
+    const double h2 = 0.5 * dt / I.dx[t1], h3 = 0.5 * dt / I.dx[t2];
+    const int p2 = pair_index(t1, t2), p3 = pair_index(t2, t1);
+    double f2r[UEDEN + 1], f2l[UEDEN + 1], f3r[UEDEN + 1], f3l[UEDEN + 1], pg2p, ug2p, pg2m, ug2m, pg3p, ug3p, pg3m,
+        ug3m, gamc = 0.0;
+    QInH qm, qp;
+    FaceH side_p{};
+    if (ok) {
+        load_tflux_h(x.FT[p2], I, r2, f2r, pg2p, ug2p);
+        load_tflux_h(x.FT[p2], I, ep, f2l, pg2m, ug2m);
+        load_tflux_h(x.FT[p3], I, r3, f3r, pg3p, ug3p);
+        load_tflux_h(x.FT[p3], I, ep, f3l, pg3m, ug3m);
+        gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, i, j, k));
+        if (has_m) {
+            load_qin_h(x.SM[d], I, em, qm);
+            const FaceH f = to_face(trans2_hydro(qm, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p,
+                                                 ug3m, gamc, h2, h3), d);
+            ls[0][tid] = f.rho;
+            ls[1][tid] = f.un;
+            ls[2][tid] = f.ut;
+            ls[3][tid] = f.utt;
+            ls[4][tid] = f.p;
+            ls[5][tid] = f.rhoe;
+        }
+        if (has_p) {
+            load_qin_h(x.SP[d], I, ep, qp);
+            side_p = to_face(trans2_hydro(qp, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m,
+                                          gamc, h2, h3), d);
+        }
     }
-    if (draw < 0.0) {
-        const double nb = 0.1 * FOURTH * div1_b;
+    __syncthreads();
+    FaceHB Lb{}, Rb{};
+    double cg[4] = {0.0, 0.0, 0.0, 0.0}, g[NHB] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (has_p && l > 0) {
+        const int tb = tid - st;
+        const FaceH side_m{ls[0][tb], ls[1][tb], ls[2][tb], ls[3][tb], ls[4][tb], ls[5][tb]};
+        // the update: a face is the low face of zone cd, the high face of cd - 1
+        const idx_t cr = cidx(I, i, j, k), cl = cidx(I, i - ei, j - ej, k - ek);
+        const bool in_r = cd < nd, in_l = cd > 0;
+        const double dx0 = I.dx[0], dx1 = I.dx[1], dx2 = I.dx[2], dxd = I.dx[d];
+        const double av = (d == 0 ? dx1 * dx2 : (d == 1 ? dx0 * dx2 : dx0 * dx1)) * (1.0 / (dx0 * dx1 * dx2));
+        double fnb[NNB];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) aadd(EAp(a.DVb, I, 1, 0, nodes[q]), nb);
-    }
-    // final Riemann
-    const int mn = NB_MX + d, mt = d == 0 ? NB_MY : NB_MX, mtt = d == 2 ? NB_MY : NB_MZ;
-    RiemannHB rb;
-    rb.f_rho = fnb[NB_RHO];
-    rb.f_mn = fnb[mn];
-    rb.f_mt = fnb[mt];
-    rb.f_mtt = fnb[mtt];
-    rb.f_E = fnb[NB_E];
-    rb.f_e = fnb[NB_EI];
-    rb.g_p = fnb[NB_GP];
-    rb.g_un = fnb[NB_GU];
-    FaceHB sb[2] = {{0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0}};
-    face_riemann_hb(x, a, I, d, i, j, k, side[0], side[1], rb, sb[0], sb[1]);
-    // trans2
+        for (int h = 0; h < NHB; ++h) {
+            double v = 0.0;
+            if (in_r) v += CA(a.Sb, I, NHB, h, cr) * av;
+            if (in_l) v -= CA(a.Sb, I, NHB, h, cl) * av;
+            fnb[h] = v;
+        }
+        // pdivu term of rho e: s -= 0.5 (GP+ + GP-) (GU+ - GU-) / dx_d
+        double *F = x.FN[d];
+        const dbl2 g0 = EF2(F, I, NFN, FN_GP, ep);
+        fnb[NB_GP] = fnb[NB_GU] = 0.0;
+        if (in_r) {
+            const dbl2 gp = EF2(F, I, NFN, FN_GP, em);
+            const double b = -CA(a.Sb, I, NHB, HB_EI, cr) / dxd;
+            fnb[NB_GP] += b * HALF * (gp.y - g0.y);
+            fnb[NB_GU] -= b * HALF * (gp.x + g0.x);
+        }
+        if (in_l) {
+            const dbl2 gm = EF2(F, I, NFN, FN_GP, eidx(I, i - ei, j - ej, k - ek));
+            const double b = -CA(a.Sb, I, NHB, HB_EI, cl) / dxd;
+            fnb[NB_GP] += b * HALF * (g0.y - gm.y);
+            fnb[NB_GU] += b * HALF * (g0.x + gm.x);
+        }
+        // artificial viscosity (forward: Source/Castro_hydro_nd.F90:174-245)
+        const idx_t na = eidx(I, i + (d != 0), j + (d == 0), k);
+        const idx_t nb = d == 2 ? eidx(I, i, j + 1, k) : eidx(I, i, j, k + 1);
+        const idx_t nc = d == 2 ? eidx(I, i + 1, j + 1, k) : na;
+        const double draw = FOURTH * (EA(x.DV, I, 1, 0, ep) + EA(x.DV, I, 1, 0, na) + EA(x.DV, I, 1, 0, nb) +
+                                      EA(x.DV, I, 1, 0, nc));
+        const double div1 = 0.1 * fmin(0.0, draw);
+        double div1_b = 0.0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int sh = s - 1;
-        const int il = i + sh * ed[0], jl = j + sh * ed[1], kl = k + sh * ed[2];
-        QInH lq;
-        load_qin_h(s == 0 ? x.SM[d] : x.SP[d], I, e, lq);
-        double f2r[UEDEN + 1], f2l[UEDEN + 1], f3r[UEDEN + 1], f3l[UEDEN + 1], pg2p, ug2p, pg2m, ug2m, pg3p, ug3p,
-            pg3m, ug3m;
-        load_tflux_h(F2, I, r2[s], f2r, pg2p, ug2p);
-        load_tflux_h(F2, I, l2[s], f2l, pg2m, ug2m);
-        load_tflux_h(F3, I, r3[s], f3r, pg3p, ug3p);
-        load_tflux_h(F3, I, l2[s], f3l, pg3m, ug3m);
-        const idx_t cg = cidx(I, il, jl, kl);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cg);
-        const QStateHB ob = from_faceb(sb[s], d);
-        QInHB lqb = {0, 0, 0, 0, 0, 0};
-        double f2rb[5] = {0, 0, 0, 0, 0}, f2lb[5] = {0, 0, 0, 0, 0}, f3rb[5] = {0, 0, 0, 0, 0},
-               f3lb[5] = {0, 0, 0, 0, 0}, gb[8] = {0, 0, 0, 0, 0, 0, 0, 0}, gamcb = 0.0;
-        trans2_hydro_b(lq, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m, gamc, h2, h3, ob, lqb,
-                       f2rb, f2lb, f3rb, f3lb, gb, gamcb);
-        // the d-face states at e are this thread's alone in A_final
-        add_stateb<true>(s == 0 ? a.SMb[d] : a.SPb[d], I, e, lqb);
-        add_tfluxb(a.FTb[p2], I, r2[s], f2rb, gb[0], gb[2]);
-        add_tfluxb(a.FTb[p2], I, l2[s], f2lb, gb[1], gb[3]);
-        add_tfluxb(a.FTb[p3], I, r3[s], f3rb, gb[4], gb[6]);
-        add_tfluxb(a.FTb[p3], I, l2[s], f3lb, gb[5], gb[7]);
-        aadd(CAp(a.Qb, I, NQB, QB_G, cg), gamcb);
+        for (int h = 0; h < NHB; ++h) {
+            const int n = hb_comp(h);
+            div1_b += fnb[h] * dxd * (CA(x.U1, I, NU1, n, cr) - CA(x.U1, I, NU1, n, cl));
+            g[h] = fnb[h] * dxd * div1;
+        }
+        // a face that two bricks have is counted in the lower one
+        if (draw < 0.0 && (l < top || cd == nd)) {
+            const double v = 0.1 * FOURTH * div1_b;
+            aadd(EAp(a.DVb, I, 1, 0, ep), v);
+            aadd(EAp(a.DVb, I, 1, 0, na), v);
+            aadd(EAp(a.DVb, I, 1, 0, nb), v);
+            aadd(EAp(a.DVb, I, 1, 0, nc), v);
+        }
+        RiemannHB rb;
+        rb.f_rho = fnb[NB_RHO];
+        rb.f_mn = pick(d, fnb[NB_MX], fnb[NB_MY], fnb[NB_MZ]);
+        rb.f_mt = pick(d, fnb[NB_MY], fnb[NB_MX], fnb[NB_MX]);
+        rb.f_mtt = pick(d, fnb[NB_MZ], fnb[NB_MZ], fnb[NB_MY]);
+        rb.f_E = fnb[NB_E];
+        rb.f_e = fnb[NB_EI];
+        rb.g_p = fnb[NB_GP];
+        rb.g_un = fnb[NB_GU];
+        face_riemann_hb(x, I, d, i, j, k, side_m, side_p, rb, Lb, Rb, cg);
     }
+    lr[0][tid] = Lb.rho;
+    lr[1][tid] = Lb.un;
+    lr[2][tid] = Lb.ut;
+    lr[3][tid] = Lb.utt;
+    lr[4][tid] = Lb.p;
+    lr[5][tid] = Lb.rhoe;
+    lr[6][tid] = cg[0];
+    lr[7][tid] = cg[2];
+#pragma unroll
+    for (int h = 0; h < NHB; ++h) lr[8 + h][tid] = g[h];
+    __syncthreads();
+    // the zone's owner has both its faces (its one face at the domain's ends)
+    if (!ok || !(l > 0 || cd < 0) || !(l < top || cd == nd)) return;
+    double z2[NZB] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, z3[NZB] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, dummy[UEDEN + 1] = {0, 0, 0, 0, 0};
+    double gb[8] = {0, 0, 0, 0, 0, 0, 0, 0}, gamcb = has_p ? cg[3] : 0.0, cb = has_p ? cg[1] : 0.0;
+    double f2b[5] = {0, 0, 0, 0, 0}, f3b[5] = {0, 0, 0, 0, 0};
+    const idx_t c = cidx(I, i, j, k);
+    if (has_p) {
+        QInHB o{0, 0, 0, 0, 0, 0};
+        trans2_hydro_b(qp, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m, gamc, h2, h3,
+                       from_faceb(Rb, d), o, f2b, dummy, f3b, dummy, gb, gamcb);
+        store_stateb(a.SPb[d], I, ep, o);
+    }
+    if (has_m) {
+        const int ta = tid + st;
+        QInHB o{0, 0, 0, 0, 0, 0};
+        const FaceHB m{lr[0][ta], lr[1][ta], lr[2][ta], lr[3][ta], lr[4][ta], lr[5][ta]};
+        trans2_hydro_b(qm, f2r, f2l, f3r, f3l, pg2p, pg2m, ug2p, ug2m, pg3p, pg3m, ug3p, ug3m, gamc, h2, h3,
+                       from_faceb(m, d), o, f2b, dummy, f3b, dummy, gb, gamcb);
+        store_stateb(a.SMb[d], I, em, o);
+        cb += lr[6][ta];
+        gamcb += lr[7][ta];
+#pragma unroll
+        for (int h = 0; h < NHB; ++h) g[h] -= lr[8 + h][ta];
+    }
+#pragma unroll
+    for (int n = 0; n <= UEDEN; ++n) {
+        z2[n] = f2b[n];
+        z3[n] = f3b[n];
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        z2[ZB_PGP + n] = gb[n];
+        z3[ZB_PGP + n] = gb[4 + n];
+    }
+    store_zoneb(a.ZF[p2], I, ep, z2);
+    store_zoneb(a.ZF[p3], I, ep, z3);
+    EF2(a.CG[d], I, 2, 0, ep) = dbl2{cb, gamcb};
+#pragma unroll
+    for (int h = 0; h < NHB; ++h) aadd(CAp(a.U1b, I, NHB, h, c), g[h]);
 }
 
 // ------------------------------------------------------------------ A_trans1
-__global__ __launch_bounds__(256) void A_trans1(Plan p, Ctx x, ACtx a)
+// F^{t|d} of both d: the Riemann problem and trans1, by zones along t as in
+// A_final; the fluxes' adjoints are gathered from the zones of the third
+// direction's A_final.  64^3: 352 us; by faces with atomic adds 787, with the
+// forward values kept across the Riemann problem (spilled) 370.
+__global__ __launch_bounds__(256) void A_trans1(Lines q, const FInst *inst, Ctx x, ACtx a)
 {
-    int m, i, j, k;
-    int sub_;
-    if (!plan_cell_sub(p, 6, sub_, m, i, j, k)) return;
-    const int combo = sub_;
-    const int t = c_pair_t[combo], d = c_pair_d[combo];
-    const FInst &I = p.inst[m];
-    const int c[3] = {i, j, k};
-    if (c[t] < 0 || c[d] < 0 || c[d] > I.n[d] - 1) return;
-    const idx_t e = eidx(I, i, j, k);
-    const int et[3] = {t == 0, t == 1, t == 2}, ed[3] = {d == 0, d == 1, d == 2};
-    const double cdtdx = x.dt_cur[m] / I.dx[d];
-    const double cdt = cdtdx / 3.0;
-    FaceH side[2];
-    idx_t el[2], er[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int sh = s - 1;
-        const int il = i + sh * et[0], jl = j + sh * et[1], kl = k + sh * et[2];
-        el[s] = eidx(I, il, jl, kl);
-        er[s] = eidx(I, il + ed[0], jl + ed[1], kl + ed[2]);
-        QInH lq;
-        load_qin_h(s == 0 ? x.SM[t] : x.SP[t], I, e, lq);
-        double fr[UEDEN + 1], fl[UEDEN + 1], pgp, ugp, pgm, ugm;
-        load_tflux_h(x.FD[d], I, er[s], fr, pgp, ugp);
-        load_tflux_h(x.FD[d], I, el[s], fl, pgm, ugm);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, il, jl, kl));
-        const QStateH o = trans1_hydro(lq, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt);
-        side[s] = to_face(o, t);
+    __shared__ double ls[6][256], lr[8][256];
+    int lb = logical_block();
+    const int t = lb % 3;
+    lb /= 3;
+    if (lb >= q.nb[t]) return;  // the whole block
+    const FInst &I = inst[0];
+    int i, j, k, l;
+    const bool ok = line_cell(q, t, lb, I, i, j, k, l);
+    const int tid = threadIdx.x, st = t == 0 ? 1 : q.W[t], top = q.L[t] - 1, nt = I.n[t];
+    const int ct = t == 0 ? i : (t == 1 ? j : k);
+    const int ei = t == 0, ej = t == 1, ek = t == 2;
+    const bool has_p = ok && ct >= 0, has_m = ok && ct + 1 <= nt;
+    const bool own = ok && (l > 0 || ct < 0) && (l < top || ct == nt);
+    const idx_t ep = eidx(I, i, j, k), em = eidx(I, i + ei, j + ej, k + ek);
+    // where A_final has been: across t the zones of the domain
+    const bool in0 = i >= 0 && i < I.n[0], in1 = j >= 0 && j < I.n[1], in2 = k >= 0 && k < I.n[2];
+    const bool fin = (t == 0 || in0) && (t == 1 || in1) && (t == 2 || in2);
+    QInHB ob_p{0, 0, 0, 0, 0, 0}, ob_m{0, 0, 0, 0, 0, 0};
+    double cb = 0.0, gamcb = 0.0, gamc = 0.0;
+    if (ok) gamc = CA(x.Q, I, NFQ, FQ_G, cidx(I, i, j, k));
+    if (own && fin) {
+        if (has_p) load_stateb(a.SPb[t], I, ep, ob_p);
+        if (has_m) load_stateb(a.SMb[t], I, em, ob_m);
+        const dbl2 v = EF2(a.CG[t], I, 2, 0, ep);
+        cb = v.x;
+        gamcb = v.y;
     }
-    const RiemannHB rb = load_tfluxb(a.FTb[combo], I, e, t);
-    FaceHB sb[2] = {{0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0}};
-    face_riemann_hb(x, a, I, t, i, j, k, side[0], side[1], rb, sb[0], sb[1]);
-#pragma unroll
     for (int s = 0; s < 2; ++s) {
-        const int sh = s - 1;
-        const int il = i + sh * et[0], jl = j + sh * et[1], kl = k + sh * et[2];
-        QInH lq;
-        load_qin_h(s == 0 ? x.SM[t] : x.SP[t], I, e, lq);
+        const int d = t == 0 ? 1 + s : (t == 1 ? 2 * s : s);
+        const bool act = ok && (d == 0 ? in0 : (d == 1 ? in1 : in2));
+        const int combo = pair_index(t, d);
+        const double cdtdx = x.dt_cur[0] / I.dx[d];
+        const double cdt = cdtdx / 3.0;
         double fr[UEDEN + 1], fl[UEDEN + 1], pgp, ugp, pgm, ugm;
-        load_tflux_h(x.FD[d], I, er[s], fr, pgp, ugp);
-        load_tflux_h(x.FD[d], I, el[s], fl, pgm, ugm);
-        const idx_t cg = cidx(I, il, jl, kl);
-        const double gamc = CA(x.Q, I, NFQ, FQ_G, cg);
-        const QStateHB ob = from_faceb(sb[s], t);
-        QInHB lqb = {0, 0, 0, 0, 0, 0};
-        double frb[5] = {0, 0, 0, 0, 0}, flb[5] = {0, 0, 0, 0, 0}, pgpb = 0, pgmb = 0, ugpb = 0, ugmb = 0, gamcb = 0;
-        trans1_hydro_b(lq, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt, ob, lqb, frb, flb, pgpb, pgmb, ugpb, ugmb, gamcb);
-        add_stateb(s == 0 ? a.SMb[t] : a.SPb[t], I, e, lqb);
-        add_tfluxb(a.FDb[d], I, er[s], frb, pgpb, ugpb);
-        add_tfluxb(a.FDb[d], I, el[s], flb, pgmb, ugmb);
-        aadd(CAp(a.Qb, I, NQB, QB_G, cg), gamcb);
+        const idx_t dr = eidx(I, i + (d == 0), j + (d == 1), k + (d == 2)) - ep;
+        FaceH side_p{};
+        idx_t er = ep;
+        behind(er, ob_m);
+        if (act) {
+            load_tflux_h(x.FD[d], I, er + dr, fr, pgp, ugp);
+            load_tflux_h(x.FD[d], I, er, fl, pgm, ugm);
+            if (has_m) {
+                QInH qm;
+                load_qin_h(x.SM[t], I, er + (em - ep), qm);
+                const FaceH f = to_face(trans1_hydro(qm, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt), t);
+                ls[0][tid] = f.rho;
+                ls[1][tid] = f.un;
+                ls[2][tid] = f.ut;
+                ls[3][tid] = f.utt;
+                ls[4][tid] = f.p;
+                ls[5][tid] = f.rhoe;
+            }
+            if (has_p) {
+                QInH qp;
+                load_qin_h(x.SP[t], I, er, qp);
+                side_p = to_face(trans1_hydro(qp, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt), t);
+            }
+        }
+        __syncthreads();
+        FaceHB Lb{}, Rb{};
+        double cg[4] = {0.0, 0.0, 0.0, 0.0};
+        if (act && has_p && l > 0) {
+            const int tb = tid - st;
+            const FaceH side_m{ls[0][tb], ls[1][tb], ls[2][tb], ls[3][tb], ls[4][tb], ls[5][tb]};
+            FluxB v{};
+            gather_zoneb(a.ZF[combo], I, eidx(I, i - ei, j - ej, k - ek), ep, ct > 0, ct < nt, v);
+            face_riemann_hb(x, I, t, i, j, k, side_m, side_p, riemannb_of(v, t), Lb, Rb, cg);
+        }
+        lr[0][tid] = Lb.rho;
+        lr[1][tid] = Lb.un;
+        lr[2][tid] = Lb.ut;
+        lr[3][tid] = Lb.utt;
+        lr[4][tid] = Lb.p;
+        lr[5][tid] = Lb.rhoe;
+        lr[6][tid] = cg[0];
+        lr[7][tid] = cg[2];
+        __syncthreads();
+        if (!(act && own)) continue;
+        er = ep;
+        behind(er, Rb);
+        load_tflux_h(x.FD[d], I, er + dr, fr, pgp, ugp);
+        load_tflux_h(x.FD[d], I, er, fl, pgm, ugm);
+        double frb[5] = {0, 0, 0, 0, 0}, dummy[UEDEN + 1] = {0, 0, 0, 0, 0}, z[NZB] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        if (has_p) {
+            QInH qp;
+            load_qin_h(x.SP[t], I, er, qp);
+            cb += cg[1];
+            gamcb += cg[3];
+            trans1_hydro_b(qp, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt, from_faceb(Rb, t), ob_p, frb, dummy, z[ZB_PGP],
+                           z[ZB_PGM], z[ZB_UGP], z[ZB_UGM], gamcb);
+        }
+        if (has_m) {
+            const int ta = tid + st;
+            const FaceHB m{lr[0][ta], lr[1][ta], lr[2][ta], lr[3][ta], lr[4][ta], lr[5][ta]};
+            QInH qm;
+            load_qin_h(x.SM[t], I, er + (em - ep), qm);
+            cb += lr[6][ta];
+            gamcb += lr[7][ta];
+            trans1_hydro_b(qm, fr, fl, pgp, pgm, ugp, ugm, gamc, cdt, from_faceb(m, t), ob_m, frb, dummy, z[ZB_PGP],
+                           z[ZB_PGM], z[ZB_UGP], z[ZB_UGM], gamcb);
+        }
+#pragma unroll
+        for (int n = 0; n <= UEDEN; ++n) z[n] = frb[n];
+        store_zoneb(a.ZT[combo], I, ep, z);
     }
+    if (!own) return;
+    if (has_p) store_stateb(a.SPb[t], I, ep, ob_p);
+    if (has_m) store_stateb(a.SMb[t], I, em, ob_m);
+    EF2(a.CG[t], I, 2, 0, ep) = dbl2{cb, gamcb};
 }
 
 // ------------------------------------------------------------------ A_flux1
@@ -453,37 +603,54 @@ __global__ __launch_bounds__(256) void A_flux1(Plan p, Ctx x, ACtx a)
     const FInst &I = p.inst[m];
     const int pos = d == 0 ? i : (d == 1 ? j : k);
     if (pos < 0) return;
-    const idx_t e = eidx(I, i, j, k);
+    const idx_t e = eidx(I, i, j, k), el = eidx(I, i - (d == 0), j - (d == 1), k - (d == 2));
     FaceH L, R;
     load_fs_h(x.SM[d], I, e, d, L);
     load_fs_h(x.SP[d], I, e, d, R);
-    const RiemannHB rb = load_tfluxb(a.FDb[d], I, e, d);
-    FaceHB Lb = {0, 0, 0, 0, 0, 0}, Rb = {0, 0, 0, 0, 0, 0};
-    face_riemann_hb(x, a, I, d, i, j, k, L, R, rb, Lb, Rb);
-    // one thread per d-face: the states at e are this thread's alone here
-    add_faceb<true>(a.SMb[d], I, e, d, Lb);
-    add_faceb<true>(a.SPb[d], I, e, d, Rb);
+    FluxB v{};
+    double cg[4];
+    for (int s = 0; s < 2; ++s)  // the two pairs (t, d)
+        gather_zoneb(a.ZT[2 * d + s], I, el, e, pos > 0, pos < I.n[d], v);
+    FaceHB Lb, Rb;
+    face_riemann_hb(x, I, d, i, j, k, L, R, riemannb_of(v, d), Lb, Rb, cg);
+    add_faceb(a.SMb[d], I, e, d, Lb);
+    add_faceb(a.SPb[d], I, e, d, Rb);
+    EF2(a.CGF[d], I, 4, 0, e) = dbl2{cg[0], cg[2]};
+    EF2(a.CGF[d], I, 4, 2, e) = dbl2{cg[1], cg[3]};
 }
 
 // ------------------------------------------------------------------ A_trace
-__global__ __launch_bounds__(256) void A_trace(Plan p, Ctx x, ACtx a)
+// The thread of a zone reverses one direction's traces.  What it owes the five
+// zones of its stencil is summed along the brick through LDS, a variable at a
+// time, and stored; what leaves the brick or the range, or belongs to a zone
+// of the ring, is added by itself to the mapped zone.  64^3: 338 us against
+// 432 with 38 atomic adds a zone and direction; what is left is arithmetic at
+// two waves a SIMD (VALUs 42% busy; three waves spill and gain nothing).
+__global__ __launch_bounds__(256) void A_trace(Lines q, const FInst *inst, Ctx x, ACtx a)
 {
-    int m, i, j, k;
-    int sub_;
-    if (!plan_cell_sub(p, 3, sub_, m, i, j, k)) return;
-    const int d = sub_;
-    const FInst &I = p.inst[m];
+    __shared__ double ls[2][5][256];
+    int lb = logical_block();
+    const int d = lb % 3;
+    lb /= 3;
+    if (lb >= q.nb[d]) return;  // the whole block
+    const FInst &I = inst[0];
+    int i, j, k, l;
+    const bool ok = line_cell(q, d, lb, I, i, j, k, l);
+    i = min(i, I.n[0]);  // threads without a zone read the last one
+    j = min(j, I.n[1]);
+    k = min(k, I.n[2]);
+    const int tid = threadIdx.x, st = d == 0 ? 1 : q.W[d], top = q.L[d] - 1, nd = I.n[d];
     const int di = (d == 0), dj = (d == 1), dk = (d == 2);
     const int pos = d == 0 ? i : (d == 1 ? j : k);
     const bool do_p = pos >= 0;
-    const bool do_m = pos <= I.n[d] - 1;
+    const bool do_m = pos <= nd - 1;
     const int cun = FQ_U + d, cut = d == 0 ? FQ_V : (d == 1 ? FQ_W : FQ_U), cutt = d == 0 ? FQ_W : (d == 1 ? FQ_U : FQ_V);
     const idx_t c0 = cidx(I, i, j, k);
     const double cc = CA(x.Q, I, NFQ, FQ_C, c0);
     const double un = CA(x.Q, I, NFQ, cun, c0);
     const idx_t ec = eidx(I, i, j, k);
     const double flatn = EA(x.FL, I, 1, 0, ec);
-    const double dtdx = x.dt_cur[m] / I.dx[d];
+    const double dtdx = x.dt_cur[0] / I.dx[d];
     idx_t cs[5];
 #pragma unroll
     for (int s = -2; s <= 2; ++s) cs[s + 2] = cidx(I, i + s * di, j + s * dj, k + s * dk);
@@ -514,26 +681,43 @@ __global__ __launch_bounds__(256) void A_trace(Plan p, Ctx x, ACtx a)
     }
 
     const idx_t ep = ec, em = eidx(I, i + di, j + dj, k + dk);
-    const int sun = SB_U + d, sut = d == 0 ? SB_V : (d == 1 ? SB_W : SB_U), sutt = d == 0 ? SB_W : (d == 1 ? SB_U : SB_V);
     double Ipb[3][4] = {{0}}, Imb[3][4] = {{0}};
     double gam_mb = 0.0, gam_pb = 0.0, Ip_utb = 0.0, Im_utb = 0.0, Ip_uttb = 0.0, Im_uttb = 0.0;
     if (do_p) {
-        double *SB = a.SPb[d];
-        ppm_project_b<true>(Im, gam_m, un, cc, EA(SB, I, NSB, SB_RHO, ep), EA(SB, I, NSB, sun, ep),
-                            EA(SB, I, NSB, SB_RE, ep), EA(SB, I, NSB, SB_P, ep), Imb, gam_mb);
-        Im_utb = EA(SB, I, NSB, sut, ep);
-        Im_uttb = EA(SB, I, NSB, sutt, ep);
+        QInHB v;
+        load_stateb(a.SPb[d], I, ep, v);
+        ppm_project_b<true>(Im, gam_m, un, cc, v.rho, pick(d, v.u, v.v, v.w), v.rhoe, v.p, Imb, gam_mb);
+        Im_utb = pick(d, v.v, v.w, v.u);
+        Im_uttb = pick(d, v.w, v.u, v.v);
     }
     if (do_m) {
-        double *SB = a.SMb[d];
-        ppm_project_b<false>(Ip, gam_p, un, cc, EA(SB, I, NSB, SB_RHO, em), EA(SB, I, NSB, sun, em),
-                             EA(SB, I, NSB, SB_RE, em), EA(SB, I, NSB, SB_P, em), Ipb, gam_pb);
-        Ip_utb = EA(SB, I, NSB, sut, em);
-        Ip_uttb = EA(SB, I, NSB, sutt, em);
+        QInHB v;
+        load_stateb(a.SMb[d], I, em, v);
+        ppm_project_b<false>(Ip, gam_p, un, cc, v.rho, pick(d, v.u, v.v, v.w), v.rhoe, v.p, Ipb, gam_pb);
+        Ip_utb = pick(d, v.v, v.w, v.u);
+        Ip_uttb = pick(d, v.w, v.u, v.v);
     }
-    double unb = 0.0, ccb = 0.0, flatb = 0.0;
+    double unb = 0.0, flatb = 0.0;
+    // c and Gamma_1: from the states' corrections and the faces' Riemann problems
+    const dbl2 cgz = EF2(a.CG[d], I, 2, 0, ec);
+    double ccb = cgz.x, gcb = cgz.y;
+    if (do_p) {
+        const dbl2 v = EF2(a.CGF[d], I, 4, 2, ep);
+        ccb += v.x;
+        gcb += v.y;
+    }
+    if (do_m) {
+        const dbl2 v = EF2(a.CGF[d], I, 4, 0, em);
+        ccb += v.x;
+        gcb += v.y;
+    }
+    const bool inside = i >= 0 && i < I.n[0] && j >= 0 && j < I.n[1] && k >= 0 && k < I.n[2];
+    // which zones of the stencil the brick has
+    const bool b1 = l >= 1, b2 = l >= 2, a1 = l < top && pos < nd, a2 = l + 1 < top && pos + 1 < nd;
 #pragma unroll
-    for (int vv = 0; vv < 7; ++vv) {
+    for (int z = 0; z < 7; ++z) {
+        constexpr int order[7] = {0, 2, 3, 4, 5, 6, 1};  // the normal velocity last: unb goes to it
+        const int vv = order[z];
         double s5[5], SMv, SPv;
 #pragma unroll
         for (int q = 0; q < 5; ++q) s5[q] = CA(x.Q, I, NFQ, vars[vv], cs[q]);
@@ -570,12 +754,30 @@ __global__ __launch_bounds__(256) void A_trace(Plan p, Ctx x, ACtx a)
         smb -= 3.0 * s6b;
         spb -= 3.0 * s6b;
         ppm_reconstruct_b(s5, flatn, smb, spb, s5b, flatb);
+        if (vv == 1) s5b[2] += unb;
+        if (vv == 6) s5b[2] += gcb;
+        double(*S)[256] = ls[z & 1];
 #pragma unroll
-        for (int q = 0; q < 5; ++q) aadd(CAp(a.Qb, I, NQB, qbv[vv], cs[q]), s5b[q]);
+        for (int q = 0; q < 5; ++q) S[q][tid] = ok ? s5b[q] : 0.0;
+        __syncthreads();
+        if (ok) {
+            double sum = s5b[2];
+            if (b2) sum += S[4][tid - 2 * st];
+            if (b1) sum += S[3][tid - st];
+            if (a1) sum += S[1][tid + st];
+            if (a2) sum += S[0][tid + 2 * st];
+            if (inside) CA(a.QD[d], I, NQB, qbv[vv], c0) = sum;
+            else aadd(CAp(a.Qb, I, NQB, qbv[vv], c0), sum);
+            if (!b2) aadd(CAp(a.Qb, I, NQB, qbv[vv], cs[0]), s5b[0]);
+            if (!b1) aadd(CAp(a.Qb, I, NQB, qbv[vv], cs[1]), s5b[1]);
+            if (!a1) aadd(CAp(a.Qb, I, NQB, qbv[vv], cs[3]), s5b[3]);
+            if (!a2) aadd(CAp(a.Qb, I, NQB, qbv[vv], cs[4]), s5b[4]);
+        }
     }
-    aadd(CAp(a.Qb, I, NQB, QB_U + d, c0), unb);
-    aadd(CAp(a.Qb, I, NQB, QB_C, c0), ccb);
-    aadd(EAp(a.FLb, I, 1, 0, ec), flatb);
+    if (!ok) return;
+    if (inside) CA(a.QD[d], I, NQB, QB_C, c0) = ccb;
+    else aadd(CAp(a.Qb, I, NQB, QB_C, c0), ccb);
+    EA(a.FLb[d], I, 1, 0, ec) = flatb;
 }
 
 // ------------------------------------------------------------------ A_flat
@@ -585,7 +787,7 @@ __global__ __launch_bounds__(256) void A_flat(Plan p, Ctx x, ACtx a)
     if (!plan_cell(p, m, i, j, k)) return;
     const FInst &I = p.inst[m];
     const idx_t e = eidx(I, i, j, k);
-    const double fb = EA(a.FLb, I, 1, 0, e);
+    const double fb = EA(a.FLb[0], I, 1, 0, e) + EA(a.FLb[1], I, 1, 0, e) + EA(a.FLb[2], I, 1, 0, e);
     if (fb != 0.0) {
         double cur = 1.0;
         int arg = -1;
@@ -619,37 +821,29 @@ __global__ __launch_bounds__(256) void A_flat(Plan p, Ctx x, ACtx a)
             for (int s = 0; s < 7; ++s) aadd(CAp(a.Qb, I, NQB, QB_P, cc[s]), p7b[s]);
         }
     }
-    if (i >= 0 && j >= 0 && k >= 0) {
-        const double db = EA(a.DVb, I, 1, 0, e);
-        if (db != 0.0) {
-            const double gx = FOURTH * db / I.dx[0], gy = FOURTH * db / I.dx[1], gz = FOURTH * db / I.dx[2];
-#define QB(comp, a_, b_, c_) CAp(a.Qb, I, NQB, comp, cidx(I, a_, b_, c_))
-            aadd(QB(QB_U, i, j, k), gx);
-            aadd(QB(QB_U, i - 1, j, k), -gx);
-            aadd(QB(QB_U, i, j, k - 1), gx);
-            aadd(QB(QB_U, i - 1, j, k - 1), -gx);
-            aadd(QB(QB_U, i, j - 1, k), gx);
-            aadd(QB(QB_U, i - 1, j - 1, k), -gx);
-            aadd(QB(QB_U, i, j - 1, k - 1), gx);
-            aadd(QB(QB_U, i - 1, j - 1, k - 1), -gx);
-            aadd(QB(QB_V, i, j, k), gy);
-            aadd(QB(QB_V, i, j - 1, k), -gy);
-            aadd(QB(QB_V, i, j, k - 1), gy);
-            aadd(QB(QB_V, i, j - 1, k - 1), -gy);
-            aadd(QB(QB_V, i - 1, j, k), gy);
-            aadd(QB(QB_V, i - 1, j - 1, k), -gy);
-            aadd(QB(QB_V, i - 1, j, k - 1), gy);
-            aadd(QB(QB_V, i - 1, j - 1, k - 1), -gy);
-            aadd(QB(QB_W, i, j, k), gz);
-            aadd(QB(QB_W, i, j, k - 1), -gz);
-            aadd(QB(QB_W, i, j - 1, k), gz);
-            aadd(QB(QB_W, i, j - 1, k - 1), -gz);
-            aadd(QB(QB_W, i - 1, j, k), gz);
-            aadd(QB(QB_W, i - 1, j, k - 1), -gz);
-            aadd(QB(QB_W, i - 1, j - 1, k), gz);
-            aadd(QB(QB_W, i - 1, j - 1, k - 1), -gz);
-#undef QB
-        }
+    // div(u): the velocities of zone (i,j,k) from its eight nodes, 0..n
+    double n8[2][2][2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int ni = i + (q & 1), nj = j + ((q >> 1) & 1), nk = k + (q >> 2);
+        n8[q >> 2][(q >> 1) & 1][q & 1] =
+            ni <= I.n[0] && nj <= I.n[1] && nk <= I.n[2] ? EA(a.DVb, I, 1, 0, eidx(I, ni, nj, nk)) : 0.0;
+    }
+    const double du = FOURTH / I.dx[0] * ((n8[0][0][0] - n8[0][0][1]) + (n8[0][1][0] - n8[0][1][1]) +
+                                          (n8[1][0][0] - n8[1][0][1]) + (n8[1][1][0] - n8[1][1][1]));
+    const double dv = FOURTH / I.dx[1] * ((n8[0][0][0] - n8[0][1][0]) + (n8[0][0][1] - n8[0][1][1]) +
+                                          (n8[1][0][0] - n8[1][1][0]) + (n8[1][0][1] - n8[1][1][1]));
+    const double dw = FOURTH / I.dx[2] * ((n8[0][0][0] - n8[1][0][0]) + (n8[0][0][1] - n8[1][0][1]) +
+                                          (n8[0][1][0] - n8[1][1][0]) + (n8[0][1][1] - n8[1][1][1]));
+    const idx_t c0 = cidx(I, i, j, k);
+    if (i >= 0 && i < I.n[0] && j >= 0 && j < I.n[1] && k >= 0 && k < I.n[2]) {
+        CA(a.QD[0], I, NQB, QB_U, c0) += du;
+        CA(a.QD[0], I, NQB, QB_V, c0) += dv;
+        CA(a.QD[0], I, NQB, QB_W, c0) += dw;
+    } else {
+        aadd(CAp(a.Qb, I, NQB, QB_U, c0), du);
+        aadd(CAp(a.Qb, I, NQB, QB_V, c0), dv);
+        aadd(CAp(a.Qb, I, NQB, QB_W, c0), dw);
     }
 }
 
@@ -659,13 +853,8 @@ __global__ __launch_bounds__(256) void A_prim(Plan p, Ctx x, ACtx a)
     int m, i, j, k;
     if (!plan_cell(p, m, i, j, k)) return;
     const FInst &I = p.inst[m];
-    const idx_t c = cidx(I, i, j, k);
-    double u0[NVAR], ua[NVAR], u1[NVAR];
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) u0[n] = a.Uold[(long)NVAR * I.offD + (long)n * I.nD + c];
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) ua[n] = u0[n];
-    clean_hydro(ua, x.tab);
+    idx_t c = cidx(I, i, j, k);
+    double u1[NVAR], qb[NQB], ub[NHB];
 #pragma unroll
     for (int n = 0; n < NU1; ++n) u1[n] = CA(x.U1, I, NU1, n, c);  // clean(clean(U)) of the forward
     const SpeciesPairs XU = cell_species(x.U1X, I);
@@ -675,12 +864,21 @@ __global__ __launch_bounds__(256) void A_prim(Plan p, Ctx x, ACtx a)
         u1[UFS + 2 * pr] = v.x;
         if (2 * pr + 1 < NSPEC) u1[UFS + 2 * pr + 1] = v.y;
     }
-    double qb[NQB], ub[NHB];
 #pragma unroll
-    for (int q = 0; q < NQB; ++q) qb[q] = CA(a.Qb, I, NQB, q, c);
+    for (int q = 0; q < NQB; ++q)
+        qb[q] = CA(a.Qb, I, NQB, q, c) + CA(a.QD[0], I, NQB, q, c) + CA(a.QD[1], I, NQB, q, c) +
+                CA(a.QD[2], I, NQB, q, c);
 #pragma unroll
     for (int h = 0; h < NHB; ++h) ub[h] = CA(a.U1b, I, NHB, h, c);
     ctoprim_b(u1, x.tab, qb, ub);
+    // the old state is read behind these results (the compiler would start
+    // everything at once and spill)
+#pragma unroll
+    for (int h = 0; h < NHB; ++h) asm volatile("" : "+v"(c), "+v"(ub[h]));
+    double u0[NVAR], ua[NVAR];
+#pragma unroll
+    for (int n = 0; n < NVAR; ++n) ua[n] = u0[n] = a.Uold[(long)NVAR * I.offD + (long)n * I.nD + c];
+    clean_hydro(ua, x.tab);
     clean_cell_b(ua, x.tab, ub);
     clean_cell_b(u0, x.tab, ub);
 #pragma unroll
@@ -718,8 +916,9 @@ struct mc_adjoint {
     int nsteps = 0;
     double *ckpt = nullptr;       // max_steps x NVAR x nD
     std::vector<double> dts;
-    double *abuf = nullptr;       // adjoint intermediates (cleared every step)
-    long abuf_n = 0;
+    double *abuf = nullptr;       // adjoint intermediates
+    long abuf_n = 0;              // of them from the start, cleared every step
+    Lines lines_final, lines_trans1, lines_trace;
     double *ub0 = nullptr, *ub1 = nullptr;  // NHB x nD each
     ACtx a;
     // Kept intermediates: step n of the forward pass writes its primitives,
@@ -758,25 +957,58 @@ static int adjoint_keep_sets(mc_adjoint *A, bool report)
     return 0;
 }
 
+// Bricks of 256 threads along each direction: the length that wastes least
+// (threads without a zone, zones that two bricks share; 64^3: 16 along, A_trans1
+// 354 us against 414 with 8 and 381 with 32).
+static Lines make_lines(const int *n, int ring, int ovl)
+{
+    Lines q;
+    q.ring = ring;
+    q.ovl = ovl;
+    auto up = [](int a, int b) { return (a + b - 1) / b; };
+    for (int d = 0; d < 3; ++d) {
+        const int c0 = n[0] + 2 * ring, c1 = n[1] + 2 * ring, c2 = n[2] + 2 * ring;  // zones across
+        long best = -1;
+        for (int L = 64; L >= 8; L /= 2) {
+            const int W = 256 / L, along = ovl ? up(n[d], L - ovl) : up(n[d] + 2, L);
+            const int nb0 = d == 0 ? along : up(c0, W);
+            const int nb1 = d == 1 ? along : (d == 0 ? up(c1, W) : c1);
+            const long nb = (long)nb0 * nb1 * (d == 2 ? along : c2);
+            if (best < 0 || nb < best) {
+                best = nb;
+                q.L[d] = L;
+                q.W[d] = W;
+                q.nb0[d] = nb0;
+                q.nb1[d] = nb1;
+                q.nb[d] = (int)nb;
+            }
+        }
+    }
+    return q;
+}
+
 static void launch_adj(mc_adjoint *A, int stage, hipStream_t s)
 {
     FusedLevel *F = A->F;
+    if (stage == FST_FINAL || stage == FST_TRANS1 || stage == FST_TRACE) {
+        const Lines &q = stage == FST_FINAL ? A->lines_final : (stage == FST_TRANS1 ? A->lines_trans1 : A->lines_trace);
+        const dim3 g(3 * std::max(q.nb[0], std::max(q.nb[1], q.nb[2]))), b(256);
+        if (stage == FST_FINAL) hipLaunchKernelGGL(A_final, g, b, 0, s, q, F->inst, F->ctx, A->a);
+        else if (stage == FST_TRANS1) hipLaunchKernelGGL(A_trans1, g, b, 0, s, q, F->inst, F->ctx, A->a);
+        else hipLaunchKernelGGL(A_trace, g, b, 0, s, q, F->inst, F->ctx, A->a);
+        return;
+    }
     Plan p = get_plan(F, stage);
     const int nb = plan_blocks(F, p);
     const int nt = p.bx * p.by * p.bz;
     if (nb <= 0) return;
-    static const int ny[FST_N] = {1, 1, 1, 3, 3, 6, 3, 1};
-    // face stages: directions / pairs interleaved brick by brick, as forward
-    const bool interleave = ny[stage] > 1;
-    dim3 g(interleave ? nb * ny[stage] : nb, interleave ? 1 : ny[stage]), b(nt);
+    // face stage: directions interleaved brick by brick, as forward
+    const dim3 g(stage == FST_FLUX1 ? 3 * nb : nb), b(nt);
     F->ctx.tab = eos_table();
     switch (stage) {
     case FST_PRIM: hipLaunchKernelGGL(A_prim, g, b, 0, s, p, F->ctx, A->a); break;
     case FST_FLAT: hipLaunchKernelGGL(A_flat, g, b, 0, s, p, F->ctx, A->a); break;
-    case FST_TRACE: hipLaunchKernelGGL(A_trace, g, b, 0, s, p, F->ctx, A->a); break;
     case FST_FLUX1: hipLaunchKernelGGL(A_flux1, g, b, 0, s, p, F->ctx, A->a); break;
-    case FST_TRANS1: hipLaunchKernelGGL(A_trans1, g, b, 0, s, p, F->ctx, A->a); break;
-    case FST_FINAL: hipLaunchKernelGGL(A_final, g, b, 0, s, p, F->ctx, A->a); break;
     case FST_UPDATE: hipLaunchKernelGGL(A_update, g, b, 0, s, p, F->ctx, A->a); break;
     }
 }
@@ -813,11 +1045,14 @@ mc_adjoint_t *mc_adjoint_create(const int *n_cell, const double *prob_lo, const 
     A->nD = (long)n_cell[0] * n_cell[1] * n_cell[2];
     A->nE = fused_next(A->F, 0);  // the reverse kernels index with the engine's stride
     A->max_steps = max_steps;
-    // intermediates: U1b, Qb (cells), FLb, DVb, SMb, SPb, FDb, FTb, FNb (extended)
+    // intermediates: U1b, Qb (cells) and DVb, cleared every step; SMb, SPb,
+    // CG, ZF, ZT.  Sb lies in ZT, which is written after A_final has read it;
+    // CGF, FLb and QD in ZF, which A_trans1 is the last to read.
     const long nD = A->nD, nE = A->nE;
-    A->abuf_n = (long)(NHB + NQB) * nD + (2 + 6 * NSB + 3 * NFB + 6 * NFB + 3 * NNB) * nE;
+    A->abuf_n = (long)(NHB + NQB) * nD + nE;
+    const long rest = (3 * (2 * NSB + 2) + 12 * NZB) * nE;
     bool ok = !check_hip(hipMalloc(&A->ckpt, sizeof(double) * NVAR * nD * (size_t)max_steps), "hipMalloc(ckpt)") &&
-              !check_hip(hipMalloc(&A->abuf, sizeof(double) * A->abuf_n), "hipMalloc(adjoint)") &&
+              !check_hip(hipMalloc(&A->abuf, sizeof(double) * (A->abuf_n + rest)), "hipMalloc(adjoint)") &&
               !check_hip(hipMalloc(&A->ub0, sizeof(double) * NHB * nD), "hipMalloc(adjoint)") &&
               !check_hip(hipMalloc(&A->ub1, sizeof(double) * NHB * nD), "hipMalloc(adjoint)");
     if (!ok) {
@@ -832,24 +1067,29 @@ mc_adjoint_t *mc_adjoint_create(const int *n_cell, const double *prob_lo, const 
     q += NHB * nD;
     a.Qb = q;
     q += NQB * nD;
-    a.FLb = q;
-    q += nE;
     a.DVb = q;
     q += nE;
+    auto take = [&](double *&p, long n) {
+        p = q;
+        q += n;
+    };
     for (int d = 0; d < 3; ++d) {
-        a.SMb[d] = q;
-        q += NSB * nE;
-        a.SPb[d] = q;
-        q += NSB * nE;
-        a.FDb[d] = q;
-        q += NFB * nE;
-        a.FNb[d] = q;
-        q += NNB * nE;
+        take(a.SMb[d], NSB * nE);
+        take(a.SPb[d], NSB * nE);
+        take(a.CG[d], 2 * nE);
     }
-    for (int c = 0; c < 6; ++c) {
-        a.FTb[c] = q;
-        q += NFB * nE;
+    for (int c = 0; c < 6; ++c) take(a.ZF[c], NZB * nE);
+    for (int c = 0; c < 6; ++c) take(a.ZT[c], NZB * nE);
+    a.Sb = a.ZT[0];
+    q = a.ZF[0];
+    for (int d = 0; d < 3; ++d) {
+        take(a.CGF[d], 4 * nE);
+        take(a.FLb[d], nE);
+        take(a.QD[d], NQB * nD);
     }
+    A->lines_final = make_lines(A->n, 0, 2);
+    A->lines_trans1 = make_lines(A->n, 1, 2);
+    A->lines_trace = make_lines(A->n, 1, 0);
     return A;
 }
 
