@@ -217,7 +217,9 @@ void mc_set_problem(double p_ambient, double dens_ambient, double exp_energy, do
 
 /* ---- level driver: one AMR level, a list of boxes tiling the domain ----
    MC_MODE_PLAIN replays the reference's per-box kernel sequence through the
-   Part 1 entry points; MC_MODE_FUSED advances all boxes with one launch per
+   Part 1 entry points, except that clean_state is one launch for all boxes
+   and a box's apply_av, normalize_species_fluxes and store_flux are one launch
+   a direction (the same arithmetic); MC_MODE_FUSED advances all boxes with one launch per
    stage (bit-identical results).  In fused mode mc_level_advance includes
    post_timestep's clean_state and mc_level_post_timestep does nothing,
    except on the coarse side of a flux register (mc_level_set_flux_registers),

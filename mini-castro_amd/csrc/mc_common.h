@@ -113,6 +113,7 @@ __device__ __forceinline__ int logical_block()
 struct BoxIter {
     int lo0, lo1, lo2, nx, ny;
     long n;
+    double inx, iny;  // 1 / nx, 1 / ny if iter_cell may divide by them, else 0
 };
 __host__ __device__ inline BoxIter make_iter(const Box &b)
 {
@@ -123,11 +124,27 @@ __host__ __device__ inline BoxIter make_iter(const Box &b)
     it.nx = b.hi[0] - b.lo[0] + 1;
     it.ny = b.hi[1] - b.lo[1] + 1;
     it.n = box_npts(b);
+    const bool small = it.n < (1l << 31);
+    it.inx = small ? 1.0 / it.nx : 0.0;
+    it.iny = small ? 1.0 / it.ny : 0.0;
     return it;
 }
+// Cell t of the box.  (t + 1/2) / nx is at least 1 / (2 nx) away from an
+// integer and for t < 2^31 the product's error is below 2^-20 / nx, so its
+// integer part is t / nx: two products instead of two 64-bit divisions of some
+// hundred instructions each ahead of every kernel's first load.
 __device__ __forceinline__ bool iter_cell(const BoxIter &it, long t, int &i, int &j, int &k)
 {
     if (t >= it.n) return false;
+    if (it.inx != 0.0) {
+        const int tt = (int)t;
+        const int r = (int)(((double)tt + 0.5) * it.inx);
+        const int kk = (int)(((double)r + 0.5) * it.iny);
+        i = it.lo0 + (tt - r * it.nx);
+        j = it.lo1 + (r - kk * it.ny);
+        k = it.lo2 + kk;
+        return true;
+    }
     int tt = (int)(t % it.nx);
     long r = t / it.nx;
     i = it.lo0 + tt;

@@ -34,6 +34,18 @@ void initdata_with(const ProblemConsts &pc, const int *lo, const int *hi, double
 
 // Asynchronous estdt over box bx of a state FAB on sbox: min-reduces the
 // CFL time step of every cell into *dt_dev (no synchronisation).
+// a box of an arena of FABs
+struct BoxDesc {
+    BoxIter it;
+    long off;  // of its first value, in doubles
+};
+// clean_state of every box of an arena (d: nbox boxes, nmax cells the largest)
+void launch_clean_boxes(const BoxDesc *d, int nbox, long nmax, double *arena, hipStream_t s);
+// apply_av, normalize_species_fluxes and store_flux of direction idir on the
+// faces of a box
+void launch_finish_flux(const Box &b, int idir, double dxd, const double *div, const Box &divb, const double *u,
+                        const Box &ub, double *flux, const Box &fb, double *fo, const Box &fob, const double *area,
+                        const Box &areab, double dt, hipStream_t s);
 void launch_estdt(const Box &bx, const double *state, const Box &sbox, const double *dx, double *dt_dev,
                   hipStream_t s);
 

@@ -45,13 +45,10 @@ struct FabDesc {
 // FillPatch of Sborder (grown by 4) from S_old: exact copies of the owning
 // box's value; periodic images, or the nearest domain cell (first-order
 // extrapolation) outside the domain.
-__global__ __launch_bounds__(kBlock) void k_fill_patch(BoxIter it, double *dst, long dst_sn, const double *src_arena,
-                                                       const FabDesc *fabs, const int *owner, int gran, int mx,
-                                                       int my, int n0, int n1, int n2, int periodic)
+__device__ __forceinline__ void fill_patch_cell(long t, int i, int j, int k, double *dst, long dst_sn,
+                                                const double *src_arena, const FabDesc *fabs, const int *owner,
+                                                int gran, int mx, int my, int n0, int n1, int n2, int periodic)
 {
-    int i, j, k;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (!iter_cell(it, t, i, j, k)) return;
     int g0 = i, g1 = j, g2 = k;
     if (periodic) {
         g0 = ((g0 % n0) + n0) % n0;
@@ -69,6 +66,19 @@ __global__ __launch_bounds__(kBlock) void k_fill_patch(BoxIter it, double *dst, 
     const double *s = src_arena + f.off + (g0 - f.lo[0]) + fx * (g1 - f.lo[1]) + fxy * (g2 - f.lo[2]);
 #pragma unroll 4
     for (int c = 0; c < NVAR; ++c) dst[t + dst_sn * c] = s[fn * c];
+}
+__global__ __launch_bounds__(kBlock) void k_fill_patch(const BoxDesc *boxes, int nbox, double *dst_arena,
+                                                       const double *src_arena, const FabDesc *fabs, const int *owner,
+                                                       int gran, int mx, int my, int n0, int n1, int n2, int periodic)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int b = blockIdx.y; b < nbox; b += gridDim.y) {
+        const BoxIter it = boxes[b].it;
+        int i, j, k;
+        if (iter_cell(it, t, i, j, k))
+            fill_patch_cell(t, i, j, k, dst_arena + boxes[b].off, it.n, src_arena, fabs, owner, gran, mx, my, n0, n1,
+                            n2, periodic);
+    }
 }
 
 // MultiFab::Saxpy(S_new, dt, hydro_source): s = s + dt*h
@@ -148,6 +158,8 @@ struct mc_level {
     long n_valid = 0, n_grown = 0;
     double *S_new = nullptr, *S_old = nullptr, *Sborder = nullptr, *src = nullptr;
     FabDesc *fabs_dev = nullptr;
+    BoxDesc *desc_dev = nullptr;  // the valid boxes, then the grown ones
+    long max_valid = 0, max_grown = 0;  // cells of the largest of each
     int *owner_dev = nullptr;
     int gran = 1, mx = 0, my = 0;
     // plain-path temporaries, sized for the largest box
@@ -240,8 +252,13 @@ mc_level_t *mc_level_create(const int *n_cell, const double *prob_lo, const doub
     const int mz = n_cell[2] / L->gran;
     std::vector<int> owner((size_t)L->mx * L->my * mz, -1);
     std::vector<FabDesc> fd(nbox);
+    std::vector<BoxDesc> bd(2 * (size_t)nbox);
     for (int b = 0; b < nbox; ++b) {
         const Box &bx = L->boxes[b];
+        bd[b] = BoxDesc{make_iter(bx), L->off_valid[b]};
+        bd[nbox + b] = BoxDesc{make_iter(grow1(bx, 4)), L->off_grown[b]};
+        L->max_valid = std::max(L->max_valid, bd[b].it.n);
+        L->max_grown = std::max(L->max_grown, bd[nbox + b].it.n);
         for (int d = 0; d < 3; ++d) {
             fd[b].lo[d] = bx.lo[d];
             fd[b].hi[d] = bx.hi[d];
@@ -267,6 +284,8 @@ mc_level_t *mc_level_create(const int *n_cell, const double *prob_lo, const doub
     L->Sborder = dalloc(L->n_grown, ok);
     L->dt_dev = dalloc(1, ok);
     if (ok) ok = !check_hip(hipMalloc(&L->fabs_dev, sizeof(FabDesc) * nbox), "hipMalloc(fabs)");
+    if (ok) ok = !check_hip(hipMalloc(&L->desc_dev, sizeof(BoxDesc) * bd.size()), "hipMalloc(boxes)");
+    if (ok) ok = !check_hip(hipMemcpy(L->desc_dev, bd.data(), sizeof(BoxDesc) * bd.size(), hipMemcpyHostToDevice), "h2d");
     if (ok) ok = !check_hip(hipMalloc(&L->owner_dev, sizeof(int) * owner.size()), "hipMalloc(owner)");
     if (ok) ok = !check_hip(hipMemcpy(L->fabs_dev, fd.data(), sizeof(FabDesc) * nbox, hipMemcpyHostToDevice), "h2d");
     if (ok) ok = !check_hip(hipMemcpy(L->owner_dev, owner.data(), sizeof(int) * owner.size(), hipMemcpyHostToDevice), "h2d");
@@ -360,6 +379,7 @@ void mc_level_destroy(mc_level_t *L)
     for (double *p : ps)
         if (p) (void)hipFree(p);
     if (L->fabs_dev) (void)hipFree(L->fabs_dev);
+    if (L->desc_dev) (void)hipFree(L->desc_dev);
     if (L->owner_dev) (void)hipFree(L->owner_dev);
     if (L->stream) (void)hipStreamDestroy(L->stream);
     delete L;
@@ -587,31 +607,24 @@ int mc_level_init_data(mc_level_t *L, double p_ambient, double dens_ambient, dou
     return check_hip(hipStreamSynchronize(L->stream), "init_data");
 }
 
-// Castro::clean_state over every box of an arena (ng ghost cells).
-static void clean_state(mc_level_t *L, double *arena, const std::vector<long> &off, int ng)
+// Castro::clean_state over every box of an arena: the valid boxes, or grown by
+// four cells (S_border)
+static void clean_state(mc_level_t *L, double *arena, bool grown)
 {
-    for (size_t b = 0; b < L->boxes.size(); ++b) {
-        const Box fb = grow1(L->boxes[b], ng);
-        double *s = arena + off[b];
-        enforce_minimum_density(fb.lo, fb.hi, s, fb.lo, fb.hi);
-        normalize_species(fb.lo, fb.hi, s, fb.lo, fb.hi);
-        reset_internal_e(fb.lo, fb.hi, s, fb.lo, fb.hi);
-        compute_temp(fb.lo, fb.hi, s, fb.lo, fb.hi);
-    }
+    const int nb = (int)L->boxes.size();
+    launch_clean_boxes(grown ? L->desc_dev + nb : L->desc_dev, nb, grown ? L->max_grown : L->max_valid, arena, L->stream);
 }
 
 static void fill_patch(mc_level_t *L)
 {
-    for (size_t b = 0; b < L->boxes.size(); ++b) {
-        const Box gb = grow1(L->boxes[b], 4);
-        BoxIter it = make_iter(gb);
-        hipLaunchKernelGGL(k_fill_patch, dim3(grid_for(it.n)), dim3(kBlock), 0, L->stream, it,
-                           L->Sborder + L->off_grown[b], (long)it.n, L->S_old, L->fabs_dev, L->owner_dev, L->gran,
-                           L->mx, L->my, L->n_cell[0], L->n_cell[1], L->n_cell[2], L->bc == MC_BC_PERIODIC);
-    }
+    const int nb = (int)L->boxes.size();
+    hipLaunchKernelGGL(k_fill_patch, dim3(grid_for(L->max_grown), std::min(nb, 65535)), dim3(kBlock), 0, L->stream,
+                       L->desc_dev + nb, nb, L->Sborder, L->S_old, L->fabs_dev, L->owner_dev, L->gran, L->mx, L->my,
+                       L->n_cell[0], L->n_cell[1], L->n_cell[2], L->bc == MC_BC_PERIODIC);
 }
 
-// Source/Castro_hydro.cpp:31-397 for one box, through the C ABI.
+// Source/Castro_hydro.cpp:31-397 for one box, through the C ABI but for the
+// last three steps of its fluxes, which one kernel takes together.
 static void hydro_box(mc_level_t *L, int ib, double dt)
 {
     const double *dx = L->dx;
@@ -678,13 +691,9 @@ static void hydro_box(mc_level_t *L, int ib, double dt)
                      gebx[d].hi, L->q_int, obx.lo, obx.hi, L->qe[d], gebx[d].lo, gebx[d].hi, qaux, qbx.lo, qbx.hi,
                      d + 1);
     }
-    for (int d = 0; d < 3; ++d) {
-        apply_av(ebx[d].lo, ebx[d].hi, d + 1, dx, L->divb, obx.lo, obx.hi, state, fb.lo, fb.hi, L->flux[d],
-                 gebx[d].lo, gebx[d].hi);
-        normalize_species_fluxes(ebx[d].lo, ebx[d].hi, L->flux[d], gebx[d].lo, gebx[d].hi);
-        store_flux(ebx[d].lo, ebx[d].hi, L->fluxes_out[d], ebx[d].lo, ebx[d].hi, L->flux[d], gebx[d].lo, gebx[d].hi,
-                   L->area[d], areab[d].lo, areab[d].hi, dt);
-    }
+    for (int d = 0; d < 3; ++d)  // apply_av, normalize_species_fluxes, store_flux
+        launch_finish_flux(ebx[d], d + 1, dx[d], L->divb, obx, state, fb, L->flux[d], gebx[d], L->fluxes_out[d], ebx[d],
+                           L->area[d], areab[d], dt, L->stream);
     // the flux registers take this box's store_flux output before the next
     // box reuses the buffer (Castro_advance.cpp:82-88 reads the level's
     // fluxes after the advance: the same values)
@@ -754,16 +763,16 @@ int mc_level_advance(mc_level_t *L, double dt)
     if (alloc_plain(L)) return -1;
     void *prev = mc_get_stream();
     mc_set_stream(L->stream);
-    clean_state(L, L->S_old, L->off_valid, 0); /* :51 */
+    clean_state(L, L->S_old, false); /* :51 */
     (void)check_hip(hipMemcpyAsync(L->S_new, L->S_old, L->n_valid * sizeof(double), hipMemcpyDeviceToDevice,
                                    L->stream), "Copy"); /* :55 */
     fill_patch(L);                                 /* :62 */
-    clean_state(L, L->Sborder, L->off_grown, 4);   /* :66 */
+    clean_state(L, L->Sborder, true);   /* :66 */
     fill_const(L->stream, L->src, L->n_valid, 0.0); /* hydro_source.setVal(0), Castro_hydro.cpp:17 */
     for (size_t b = 0; b < L->boxes.size(); ++b) hydro_box(L, (int)b, dt); /* :70 */
     hipLaunchKernelGGL(k_saxpy, dim3(grid_for(L->n_valid)), dim3(kBlock), 0, L->stream, L->n_valid, L->S_new, L->src,
                        dt); /* :74 */
-    clean_state(L, L->S_new, L->off_valid, 0); /* :78 */
+    clean_state(L, L->S_new, false); /* :78 */
     mc_set_stream(prev);
     return check_hip(hipGetLastError(), "advance");
 }
@@ -776,7 +785,7 @@ int mc_level_post_timestep(mc_level_t *L)
     if (L->mode == MC_MODE_FUSED && sync_from_fused(L)) return -1;
     void *prev = mc_get_stream();
     mc_set_stream(L->stream);
-    clean_state(L, L->S_new, L->off_valid, 0); /* Castro.cpp:369 */
+    clean_state(L, L->S_new, false); /* Castro.cpp:369 */
     mc_set_stream(prev);
     return check_hip(hipGetLastError(), "post_timestep");
 }
