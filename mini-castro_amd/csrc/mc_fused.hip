@@ -831,13 +831,7 @@ __global__ void K_dt(Ctx x, int ninst, double stop_time)
         if ((x.time[m] + dt_0) > (stop_time - eps)) dt_0 = stop_time - x.time[m];
     x.dt_cur[m] = dt_0;
     x.dt_est[m] = DBL_MAX;
-}
-
-__global__ void K_tick(Ctx x, int ninst)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= ninst) return;
-    x.time[m] += x.dt_cur[m];
+    x.time[m] += dt_0;  // of the step that follows, whose stages read dt alone
     x.steps[m] += 1;
 }
 
@@ -1163,6 +1157,33 @@ void fill(double *p, long n, double v, hipStream_t s)
     if (n > 0) hipLaunchKernelGGL(K_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
 }
 
+// Brick of the stages that solve the EOS cell by cell.  Rows of 64 are the
+// fastest (256^3: K_update 4.04 ms, rows of 32 4.04 to 4.16, of 16 4.4 and
+// more; 128^3: K_prim 349 us, 388 and more with 32) unless they stick out of the
+// domain, where the work of idle lanes is a narrower row's gain: from a tenth
+// of the lanes on (96^3: K_prim 188 us, rows of 32 158, K_update 279 and 257;
+// 48^3: 36 us, rows of 16 30, 53 and 47).  Below 100,000 cells there are more
+// CUs than bricks either way (45 x 37 x 29: 35 us, rows of 16 39).
+static KernelTiling cell_tiling(const std::vector<FInst> &inst)
+{
+    static const KernelTiling cand[] = {{64, 4, 1}, {32, 2, 2}, {16, 4, 2}};
+    KernelTiling t = cand[0];
+    double best = 0.0, cells = 0.0;
+    for (const FInst &I : inst) cells += (double)I.n[0] * I.n[1] * I.n[2];
+    if (cells < 100000.0) return t;
+    for (const KernelTiling &c : cand) {
+        double lanes = 0.0;
+        for (const FInst &I : inst)
+            lanes += (double)((I.n[0] + c.bx - 1) / c.bx) * ((I.n[1] + c.by - 1) / c.by) *
+                     ((I.n[2] + c.bz - 1) / c.bz) * (c.bx * c.by * c.bz);
+        if (best == 0.0 || 1.1 * lanes < best) {
+            best = lanes;
+            t = c;
+        }
+    }
+    return t;
+}
+
 FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int slab)
 {
     FusedLevel *F = new FusedLevel();
@@ -1259,7 +1280,8 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     F->totW = offW;
     F->totP = offP;
     for (int s = 0; s < NSTAGE; ++s) F->tiling[s] = KernelTiling{64, 2, 2};
-    F->tiling[ST_EST] = F->tiling[ST_PRIM] = F->tiling[ST_UPDATE] = KernelTiling{64, 4, 1};
+    F->tiling[ST_FLAT] = KernelTiling{16, 2, 2};  // stencils in all directions (256^3: 706 us, 64 x 2 x 2 750)
+    F->tiling[ST_EST] = F->tiling[ST_PRIM] = F->tiling[ST_UPDATE] = cell_tiling(F->hinst);
     F->tiling[ST_TFLUX] = F->tiling[ST_TRANS1C] = F->tiling[ST_FINALC] = KernelTiling{16, 16, 64};
     bool ok = !check_hip(hipMalloc(&F->inst, sizeof(FInst) * F->ninst), "hipMalloc(inst)") &&
               !check_hip(hipMemcpy(F->inst, F->hinst.data(), sizeof(FInst) * F->ninst, hipMemcpyHostToDevice), "h2d");
@@ -1571,7 +1593,6 @@ static void enqueue_step(FusedLevel *F, double stop_time, hipStream_t s)
     F->ctx.tab = eos_table();
     hipLaunchKernelGGL(K_dt, dim3(1), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
     for (int sl = 0; sl < F->nslab; ++sl) enqueue_slab(F, sl, s);
-    hipLaunchKernelGGL(K_tick, dim3(1), dim3(256), 0, s, F->ctx, F->ninst);
 }
 
 // Eager steps with a HIP event pair around every stage launch on stream s;
@@ -1614,8 +1635,7 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
                 launch_stage(F, st, s, ny[st], sl);
                 (void)hipEventRecord(E[2 * q + 1], s);
             }
-        hipLaunchKernelGGL(K_tick, dim3(1), dim3(256), 0, s, F->ctx, F->ninst);
-    }
+        }
     if (!rc) rc = check_hip(hipStreamSynchronize(s), "timed steps");
     for (int st = 0; st <= NSTAGE; ++st) {
         stage_ms[st] = 0.0;
