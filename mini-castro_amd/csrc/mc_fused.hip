@@ -1591,7 +1591,7 @@ static void enqueue_slab(FusedLevel *F, int sl, hipStream_t s)
 static void enqueue_step(FusedLevel *F, double stop_time, hipStream_t s)
 {
     F->ctx.tab = eos_table();
-    hipLaunchKernelGGL(K_dt, dim3(1), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
+    hipLaunchKernelGGL(K_dt, dim3((F->ninst + 255) / 256), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
     for (int sl = 0; sl < F->nslab; ++sl) enqueue_slab(F, sl, s);
 }
 
@@ -1625,7 +1625,7 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
         hipEvent_t *E = ev.data() + 2 * per * (size_t)n;
         size_t q = 0;
         (void)hipEventRecord(E[2 * q], s);
-        hipLaunchKernelGGL(K_dt, dim3(1), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
+        hipLaunchKernelGGL(K_dt, dim3((F->ninst + 255) / 256), dim3(256), 0, s, F->ctx, F->ninst, stop_time);
         (void)hipEventRecord(E[2 * q + 1], s);
         ++q;
         for (int sl = 0; sl < F->nslab; ++sl)
