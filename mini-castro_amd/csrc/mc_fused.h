@@ -66,7 +66,10 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
 // Kernel variants of a step (bit flags; 0, the default, runs K_tflux,
 // K_trans1c and K_final): FV_SPLIT_TRACE runs K_trace + K_flux1 instead of
 // K_tflux, FV_FACE_TRANS1 K_trans1 instead of K_trans1c, FV_CELL_FINAL
-// K_finalc instead of K_final.  Results are the same bit for bit.
+// K_finalc instead of K_final.  Results are the same bit for bit.  Without
+// FV_FACE_TRANS1 a step's launches of 200,000 cells and more run K_transfinal
+// for both the transverse and the final stage; a stage by itself
+// (fused_run_stage) does not.
 enum { FV_SPLIT_TRACE = 1, FV_FACE_TRANS1 = 2, FV_CELL_FINAL = 4, FV_ALL = 7 };
 void fused_set_variant(FusedLevel *F, int flags);
 // true: the step ends after the advance's clean_state (no post_timestep clean,

@@ -11,12 +11,15 @@
 //   K_trans1  faces   one-direction transverse update + flux  F^{t|d}
 //   K_final   faces   two-direction transverse update + final flux,
 //                     artificial viscosity
+//   K_transfinal  columns, K_trans1 and K_final of large launches in one
+//                     (mc_transverse.h)
 //   K_species columns the thirteen species from their traces to their final
 //                     fluxes (mc_species.h), launched with the final fluxes
 //   K_update  cells   species flux normalisation, flux divergence and p dV
 //                     source, S_new = S_old + dt src, clean_state twice, estdt
 //                     min-reduction
-//   K_dt      1 block the CFL / change_max / init_shrink time-step control
+//   K_dt      members the CFL / change_max / init_shrink time-step control and
+//                     the clock
 //
 // Why the result equals the per-box path bit for bit: every stage applies the
 // same device functions (mc_cell.h, mc_hydro.h, mc_eos.h) to the same
@@ -454,8 +457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
 // along t and above along d) is first copied into LDS, one global load per
 // face and pair of components; the block's LDS is sized by the launch
 // (trans1_tile_cells).
-// Held to 5 waves per SIMD (96 VGPRs, no spills): 12.50 against 13.02 ms
-// at the 4 waves its 99 VGPRs would give.
+// Held to 5 waves per SIMD (96 VGPRs, no spills; 256^3 4.0 ms).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void K_trans1(Plan p, Ctx x)
 {
     extern __shared__ double ftile[];  // 7 components x nT cells
@@ -1850,9 +1852,13 @@ int fused_run_stage(FusedLevel *F, int stage, hipStream_t s)
         set_error("fused_run_stage: no such stage");
         return -1;
     }
+    // by itself a stage reads and writes the arrays between the stages
+    const bool keep = F->keep_transverse;
+    F->keep_transverse = true;
     if (whole_instance_stage(stage)) launch_stage(F, stage, s, ny[stage]);
     else
         for (int sl = 0; sl < F->nslab; ++sl) launch_stage(F, stage, s, ny[stage], sl);
+    F->keep_transverse = keep;
     return check_hip(hipGetLastError(), "fused_run_stage");
 }
 
