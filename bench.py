@@ -52,26 +52,53 @@ def _counts(n):
     return cell, ring, face, tface, fface
 
 
-def _stage_bytes(stage, n):
+def _kernel_bytes(kernel, n):
     cell, ring, face, tface, fface = _counts(n)
-    NS, NF, NQ, NN = 19, 20, 21, 22   # state, flux, primitive, final-flux components
+    NS, NF, NQ, NN = 6, 8, 9, 11     # state, flux, primitive, final-flux components, without the species
+    U1, X = 7, 13                    # cleaned state before the species, the species
     doubles = {
-        "prim": (20 + 20 + 20 + NQ) * cell,                        # U in; clean(U) in place, U1, Q out
-        "flat": 4 * cell + 2 * ring,                               # p, u, v, w in; flatn, div out
-        "trace": NQ * cell + ring + 3 * 2 * NS * ring,             # Q, flatn in; minus/plus states out
-        "flux1": 3 * (2 * NS + NF) * face + 2 * cell,              # states in, F^d out; c, gamc in
+        "K_prim": (20 + 20 + U1 + X + NQ) * cell,                    # U in; clean(U) in place, U1, Q out
+        "K_flat": 4 * cell + 2 * ring,                               # p, u, v, w in; flatn, div out
+        "K_trace": NQ * cell + ring + 3 * 2 * (NS + 1) * ring,       # Q, flatn in; minus/plus states, densities out
+        "K_flux1": 3 * (2 * NS + NF) * face + 2 * cell,              # states in, F^d out; c, gamc in
         # trace + flux1 in one launch: the states it stores are read back by
         # the same launch, so they count once (written)
-        "tflux": NQ * cell + ring + 3 * 2 * NS * ring + 3 * NF * face,  # Q, flatn in; states, F^d out
-        "trans1": 3 * 2 * NS * face + 3 * NF * face + cell + 6 * NF * tface,  # t-states, F^d, gamc in; F^{t|d} out
-        "trans1c": 3 * 2 * NS * face + 3 * NF * face + cell + 6 * NF * tface,  # the same, by cells
-        "final": (3 * 2 * NS * face + 6 * NF * tface + ring + 20 * cell + 2 * cell
-                  + 3 * NN * fface),                               # states, F^{t|d}, div, U1, c/gamc in; final flux out
-        "finalc": (3 * 2 * NS * face + 6 * NF * tface + ring + 20 * cell + 2 * cell
-                   + 3 * NN * fface),                              # the same, by cells
-        "update": 3 * NN * fface + 20 * cell + 20 * cell,          # final fluxes, U in; U out
-    }[stage]
+        "K_tflux": NQ * cell + ring + 3 * 2 * (NS + 1) * ring + 3 * NF * face,  # Q, flatn in; states, F^d out
+        "K_trans1": 3 * 2 * NS * face + 3 * NF * face + cell + 6 * NF * tface,  # t-states, F^d, gamc in; F^{t|d} out
+        "K_trans1c": 3 * 2 * NS * face + 3 * NF * face + cell + 6 * NF * tface,  # the same, by cells
+        "K_final": (3 * 2 * NS * face + 6 * NF * tface + ring + 6 * cell + 2 * cell
+                    + 3 * NN * fface),                               # states, F^{t|d}, div, U1, c/gamc in; final flux out
+        "K_finalc": (3 * 2 * NS * face + 6 * NF * tface + ring + 6 * cell + 2 * cell
+                     + 3 * NN * fface),                              # the same, by cells
+        # trans1 and final in one launch: states, F^d, div, U1, c/gamc in; mass
+        # flux and Riemann weight of F^{t|d}, final flux out
+        "K_transfinal": (3 * 2 * NS * face + 3 * NF * face + ring + 6 * cell + 2 * cell + 6 * 2 * tface
+                         + 3 * NN * fface),
+        # species, velocity, 1/rho, flatn, state densities, mass fluxes and
+        # weights, div in; species fluxes out
+        "K_species": ((X + 4) * cell + ring + 6 * ring + 3 * 2 * face + 6 * 2 * tface + 3 * 3 * fface
+                      + 3 * X * fface),
+        "K_update": 3 * (NN - 3 + X) * fface + 20 * cell + 20 * cell,  # final fluxes, U in; U out
+    }[kernel]
     return 8 * doubles
+
+
+JOINED_CELLS = 200000  # levels of this size run the transverse and final fluxes in one kernel
+
+
+def stage_kernels(stage, n, variant):
+    """The kernels a launch of the stage runs on a whole level of n cells."""
+    joined = n[0] * n[1] * n[2] >= JOINED_CELLS and not variant & 2  # Level.FACE_TRANS1
+    if stage in ("final", "finalc"):
+        return ["K_species"] if joined else ["K_" + stage, "K_species"]
+    if stage == "trans1c" and joined:
+        return ["K_transfinal"]
+    return ["K_" + stage]
+
+
+def _sum_known(values):
+    values = list(values)
+    return sum(values) if all(values) else None
 
 
 STAGES_WITH_BYTES = ("prim", "flat", "trace", "flux1", "tflux", "trans1", "trans1c", "final", "finalc", "update")
@@ -501,10 +528,9 @@ def main():
     # counters, committed summary) against the zone-update's 320 B.
     w_flop = reference_flop_per_zone_update(cfg["name"])
     ran = [st for st in STAGES_WITH_BYTES if stages[st][1]]   # the stages this step runs
-    tr = [measured_traffic("mc::K_" + st, cfg["name"]) for st in ran]
-    step_traffic = sum(tr) if all(tr) else None
-    hw = [measured_fp64_ops("mc::K_" + st, cfg["name"]) for st in ran]
-    hw_step = sum(hw) if all(hw) else None
+    kernels = {st: stage_kernels(st, n, variant) for st in ran}
+    step_traffic = _sum_known(measured_traffic("mc::" + k, cfg["name"]) for st in ran for k in kernels[st])
+    hw_step = _sum_known(measured_fp64_ops("mc::" + k, cfg["name"]) for st in ran for k in kernels[st])
     roofline = {
         "bound": "fp64", "unit": "TFLOP/s", "peak": FP64_PEAK / 1e12,
         "achieved": (value * w_flop / 1e12) if w_flop else None,
@@ -530,11 +556,11 @@ def main():
     dom = max(ran, key=lambda k: stages[k][0])
     tot_ms, nl = stages[dom]
     avg_s = tot_ms / nl / 1e3
-    traffic_alg = _stage_bytes(dom, n)
+    traffic_alg = sum(_kernel_bytes(k, n) for k in kernels[dom])
     achieved = traffic_alg / avg_s
-    traffic = measured_traffic("mc::K_" + dom, cfg["name"])
+    traffic = _sum_known(measured_traffic("mc::" + k, cfg["name"]) for k in kernels[dom])
     roofline["dominant_stage"] = {
-        "kernel": "mc::K_" + dom, "bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
+        "kernel": " + ".join("mc::" + k for k in kernels[dom]), "bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
         "unit": "GB/s", "frac": achieved / HBM_PEAK, "traffic": traffic, "avg_launch_ms": tot_ms / nl,
         "bytes": "the stage's own input and output arrays (every distinct element once per launch)",
         "algorithmic_bytes_per_launch": traffic_alg,

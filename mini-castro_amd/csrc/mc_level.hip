@@ -2,8 +2,8 @@
 // clean_state / estTimeStep on one AMR level of boxes (single GPU).
 //
 // Plain mode replays the reference's per-box kernel sequence through the
-// drop-in C ABI (Source/Castro_hydro.cpp:31-397: 36 launches per box, plus
-// the four clean_state kernels at each of its four call sites and estdt).
+// drop-in C ABI (Source/Castro_hydro.cpp:31-397: 30 launches per box, and
+// estdt), with clean_state and FillPatch one launch for all boxes.
 // Fused mode hands the whole box list to the batched kernels (mc_fused.hip).
 //
 // Device memory layout: every MultiFab (S_new, S_old, Sborder, hydro

@@ -9,8 +9,8 @@
 // bytes: at 256^3 the traces and first fluxes took 10.4 ms, the transverse
 // stage 14.2, the final one 12.3.  Here a block owns a tile of columns and
 // marches in z, so a species is read once (and its tile's halo) and three
-// fluxes are written: 9.1 ms and 28 GB for all thirteen, the hydro stages alone
-// 4.3, 5.0 and 4.9 ms.
+// fluxes are written: 9.4 ms and 26 GB for all thirteen, the hydro stages alone
+// 4.3, 5.0 and 4.6 ms.
 //
 // What bounds it: FP64 issue.  A wavefront issues about 1,200 vector
 // instructions a plane for its 64 columns and two species, 60% of the rate

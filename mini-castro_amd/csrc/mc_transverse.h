@@ -144,13 +144,16 @@ __device__ __forceinline__ void finish(idx_t &e, TDiff &t)
 //
 // K_trans1c and K_final write and read the six transverse fluxes, 8 doubles a
 // face each, and read every state again; here 2 doubles a face are left of
-// them.  256^3: 6.2 ms against 5.0 + 4.6.  A CU holds two blocks (registers),
-// so what a plane waits for counts: of 14 GB read and 6.6 GB written (3.3
-// TB/s), and 35% busy VALUs, neither is the bound.  Reading a face's zones for
-// the viscosity together instead of as they are used took it from 6.8 to 6.2,
-// keeping a plane's states across two corrections from 7.6 to 7.0 and the
-// next plane's first loads ahead of the last barrier to 6.8; keeping more
-// spills (7.8).
+// them.  256^3: 6.2 ms against 5.0 + 4.6.  A CU holds two blocks (registers)
+// and its VALUs are 35% busy: what a plane waits for counts.  It moves 39 GB
+// past the L2s where its arrays hold 15.5, as a plane of an XCD's 64 blocks
+// does not fit its L2 between two uses of a state; but with the z- and
+// x-states and the z-flux kept in LDS from use to use (46 pairs read a plane
+// instead of 62, neighbouring rows by lane permutes to make room) it took 6.4.
+// Reading a face's zones for the viscosity together instead of as they are
+// used took it from 6.8 to 6.2, keeping a plane's states across two
+// corrections from 7.6 to 7.0 and the next plane's first loads ahead of the
+// last barrier to 6.8; keeping more spills (7.8).
 __global__ __launch_bounds__(SPEC_TX *SPEC_TY) __attribute__((amdgpu_waves_per_eu(2))) void K_transfinal(SpecPlan sp,
                                                                                                         Ctx x)
 {
