@@ -66,49 +66,52 @@ __host__ __device__ __forceinline__ D2 dsqrt(D2 x)
 __host__ __device__ __forceinline__ D2 dmax(D2 x, double c) { return x.v > c ? x : dc(c); }
 __host__ __device__ __forceinline__ D2 dmax(D2 x, D2 y) { return x.v >= y.v ? x : y; }
 
-// Hermite bases (Source/eos.F90:740-1031) on duals
-__host__ __device__ __forceinline__ D2 dpsi0_(D2 z) { return (z * z * z) * (z * (-6.0 * z + 15.0) - 10.0) + 1.0; }
-__host__ __device__ __forceinline__ D2 ddpsi0_(D2 z) { return (z * z) * (z * (-30.0 * z + 60.0) - 30.0); }
-__host__ __device__ __forceinline__ D2 dddpsi0_(D2 z) { return z * (z * (-120.0 * z + 180.0) - 60.0); }
-__host__ __device__ __forceinline__ D2 dpsi1_(D2 z) { return z * ((z * z) * (z * (-3.0 * z + 8.0) - 6.0) + 1.0); }
-__host__ __device__ __forceinline__ D2 ddpsi1_(D2 z) { return z * z * (z * (-15.0 * z + 32.0) - 18.0) + 1.0; }
-__host__ __device__ __forceinline__ D2 dddpsi1_(D2 z) { return z * (z * (-60.0 * z + 96.0) - 36.0); }
-__host__ __device__ __forceinline__ D2 dpsi2_(D2 z) { return 0.5 * z * z * (z * (z * (-1.0 * z + 3.0) - 3.0) + 1.0); }
-__host__ __device__ __forceinline__ D2 ddpsi2_(D2 z) { return 0.5 * z * (z * (z * (-5.0 * z + 12.0) - 9.0) + 2.0); }
-__host__ __device__ __forceinline__ D2 dddpsi2_(D2 z) { return 0.5 * (z * (z * (-20.0 * z + 36.0) - 18.0) + 2.0); }
-__host__ __device__ __forceinline__ D2 dxpsi0_(D2 z) { return z * z * (2.0 * z - 3.0) + 1.0; }
-__host__ __device__ __forceinline__ D2 dxpsi1_(D2 z) { return z * (z * (z - 2.0) + 1.0); }
-
-struct DW6 {
-    D2 w0, w1, w2, w0m, w1m, w2m;
+// One derivative: the table weights depend on the density or on the temperature
+// alone, and their D2 would carry a zero through every product.
+struct D1 {
+    double v, g;
 };
+__host__ __device__ __forceinline__ D1 operator*(D1 x, D1 y) { return D1{x.v * y.v, x.g * y.v + x.v * y.g}; }
+__host__ __device__ __forceinline__ D1 operator+(D1 x, double c) { return D1{x.v + c, x.g}; }
+__host__ __device__ __forceinline__ D1 operator-(D1 x, double c) { return D1{x.v - c, x.g}; }
+__host__ __device__ __forceinline__ D1 operator-(double c, D1 x) { return D1{c - x.v, -x.g}; }
+__host__ __device__ __forceinline__ D1 operator*(D1 x, double c) { return D1{x.v * c, x.g * c}; }
+__host__ __device__ __forceinline__ D1 operator*(double c, D1 x) { return D1{x.v * c, x.g * c}; }
 
-__device__ __forceinline__ D2 dh5(const Nodes &N, const DW6 &T, const DW6 &D)
+// Hermite bases (Source/eos.F90:740-1031) on duals
+__host__ __device__ __forceinline__ D1 dpsi0_(D1 z) { return (z * z * z) * (z * (-6.0 * z + 15.0) - 10.0) + 1.0; }
+__host__ __device__ __forceinline__ D1 ddpsi0_(D1 z) { return (z * z) * (z * (-30.0 * z + 60.0) - 30.0); }
+__host__ __device__ __forceinline__ D1 dddpsi0_(D1 z) { return z * (z * (-120.0 * z + 180.0) - 60.0); }
+__host__ __device__ __forceinline__ D1 dpsi1_(D1 z) { return z * ((z * z) * (z * (-3.0 * z + 8.0) - 6.0) + 1.0); }
+__host__ __device__ __forceinline__ D1 ddpsi1_(D1 z) { return z * z * (z * (-15.0 * z + 32.0) - 18.0) + 1.0; }
+__host__ __device__ __forceinline__ D1 dddpsi1_(D1 z) { return z * (z * (-60.0 * z + 96.0) - 36.0); }
+__host__ __device__ __forceinline__ D1 dpsi2_(D1 z) { return 0.5 * z * z * (z * (z * (-1.0 * z + 3.0) - 3.0) + 1.0); }
+__host__ __device__ __forceinline__ D1 ddpsi2_(D1 z) { return 0.5 * z * (z * (z * (-5.0 * z + 12.0) - 9.0) + 2.0); }
+__host__ __device__ __forceinline__ D1 dddpsi2_(D1 z) { return 0.5 * (z * (z * (-20.0 * z + 36.0) - 18.0) + 2.0); }
+__host__ __device__ __forceinline__ D1 dxpsi0_(D1 z) { return z * z * (2.0 * z - 3.0) + 1.0; }
+__host__ __device__ __forceinline__ D1 dxpsi1_(D1 z) { return z * (z * (z - 2.0) + 1.0); }
+
+// Biquintic and bicubic weights by density (g: d/drho) and temperature (g: d/dT)
+struct DW6 {
+    D1 w0, w1, w2, w0m, w1m, w2m;
+};
+// a density weight times a temperature weight
+__host__ __device__ __forceinline__ D2 dtwo(D1 d, D1 t) { return D2{d.v * t.v, d.g * t.v, d.v * t.g}; }
+
+// One table column at the four nodes of a cell.  It is read behind the sum
+// before it (the compiler would read all thirteen and spill).
+struct Col {
+    double a, b, c, d;
+};
+__device__ __forceinline__ Col node_col(const double *node, unsigned &off, D2 &behind, int q)
 {
-    D2 acc = dc(0.0);
-#define MC_DH5(q, wd, wmd, wt, wmt)                                                                      \
-    acc = acc + N.a[q] * (wd * wt) + N.b[q] * (wmd * wt) + N.c[q] * (wd * wmt) + N.d[q] * (wmd * wmt);
-    MC_DH5(NF, D.w0, D.w0m, T.w0, T.w0m)
-    MC_DH5(NFT, D.w0, D.w0m, T.w1, T.w1m)
-    MC_DH5(NFTT, D.w0, D.w0m, T.w2, T.w2m)
-    MC_DH5(NFD, D.w1, D.w1m, T.w0, T.w0m)
-    MC_DH5(NFDD, D.w2, D.w2m, T.w0, T.w0m)
-    MC_DH5(NFDT, D.w1, D.w1m, T.w1, T.w1m)
-    MC_DH5(NFDDT, D.w2, D.w2m, T.w1, T.w1m)
-    MC_DH5(NFDTT, D.w1, D.w1m, T.w2, T.w2m)
-    MC_DH5(NFDDTT, D.w2, D.w2m, T.w2, T.w2m)
-    return acc;
+    asm volatile("" : "+v"(off), "+v"(behind.v));
+    const double *n0 = node + off + q;
+    return Col{n0[0], n0[EOS_NODE], n0[(long)EOS_IMAX * EOS_NODE], n0[(long)EOS_IMAX * EOS_NODE + EOS_NODE]};
 }
-
-__device__ __forceinline__ D2 dh3(const Nodes &N, D2 t0, D2 t1, D2 t0m, D2 t1m, D2 d0, D2 d1, D2 d0m, D2 d1m)
+__device__ __forceinline__ void add_col(D2 &acc, const Col &N, D1 wd, D1 wdm, D1 wt, D1 wtm)
 {
-    D2 acc = dc(0.0);
-    MC_DH5(NDPDF, d0, d0m, t0, t0m)
-    MC_DH5(NDPDFT, d0, d0m, t1, t1m)
-    MC_DH5(NDPDFD, d1, d1m, t0, t0m)
-    MC_DH5(NDPDFDT, d1, d1m, t1, t1m)
-#undef MC_DH5
-    return acc;
+    acc = acc + N.a * dtwo(wd, wt) + N.b * dtwo(wdm, wt) + N.c * dtwo(wd, wtm) + N.d * dtwo(wdm, wtm);
 }
 
 // EOS outputs on the path with their derivatives in (rho, T).
@@ -140,23 +143,17 @@ __device__ __forceinline__ EosD eos_dual(const EosTable &tab, D2 den, D2 temp, D
     const D2 pion = kergavo * ytot1 * den * temp;
     const D2 eion = 1.5 * pion * deni;
 
-    Nodes N;
-    const double *n0 = tab.node + ((long)(iat - 1) + (long)EOS_IMAX * (jat - 1)) * EOS_NODE;
-    load_node(n0, N.a, 13);
-    load_node(n0 + EOS_NODE, N.b, 13);
-    load_node(n0 + (long)EOS_IMAX * EOS_NODE, N.c, 13);
-    load_node(n0 + (long)EOS_IMAX * EOS_NODE + EOS_NODE, N.d, 13);
+    unsigned off = (unsigned)(((iat - 1) + EOS_IMAX * (jat - 1)) * EOS_NODE);
 
-    D2 xd = (din - dI) * ddi;
-    if (xd.v < 0.0) xd = dc(0.0);
-    const D2 mxd = 1.0 - xd;
-    D2 xt = (temp - tJ) * dti;
-    if (xt.v < 0.0) xt = dc(0.0);
-    const D2 mxt = 1.0 - xt;
+    // zbar / abar and the density do not depend on T, nor T on the density
+    D1 xd = D1{(din.v - dI) * ddi, din.a * ddi};
+    if (xd.v < 0.0) xd = D1{0.0, 0.0};
+    const D1 mxd = 1.0 - xd;
+    D1 xt = D1{(temp.v - tJ) * dti, temp.b * dti};
+    if (xt.v < 0.0) xt = D1{0.0, 0.0};
+    const D1 mxt = 1.0 - xt;
 
-    // density weights, then one temperature weight set at a time (keeps the
-    // live dual registers to two sets)
-    DW6 D, dD, T;
+    DW6 D, dD, T, dT, ddT;
     D.w0 = dpsi0_(xd);
     D.w1 = dpsi1_(xd) * dd;
     D.w2 = dpsi2_(xd) * dd2;
@@ -175,26 +172,49 @@ __device__ __forceinline__ EosD eos_dual(const EosTable &tab, D2 den, D2 temp, D
     T.w0m = dpsi0_(mxt);
     T.w1m = -1.0 * dpsi1_(mxt) * dt;
     T.w2m = dpsi2_(mxt) * dt2;
-    const D2 free = dh5(N, T, D);
-    const D2 df_d = dh5(N, T, dD);
-    T.w0 = ddpsi0_(xt) * dti;
-    T.w1 = ddpsi1_(xt);
-    T.w2 = ddpsi2_(xt) * dt;
-    T.w0m = -1.0 * ddpsi0_(mxt) * dti;
-    T.w1m = ddpsi1_(mxt);
-    T.w2m = -1.0 * ddpsi2_(mxt) * dt;
-    const D2 df_t = dh5(N, T, D);
-    const D2 df_dt = dh5(N, T, dD);
-    T.w0 = dddpsi0_(xt) * dt2i;
-    T.w1 = dddpsi1_(xt) * dti;
-    T.w2 = dddpsi2_(xt);
-    T.w0m = dddpsi0_(mxt) * dt2i;
-    T.w1m = -1.0 * dddpsi1_(mxt) * dti;
-    T.w2m = dddpsi2_(mxt);
-    const D2 df_tt = dh5(N, T, D);
-    const D2 xt0 = dxpsi0_(xt), xt1 = dxpsi1_(xt) * dt, xt0m = dxpsi0_(mxt), xt1m = -1.0 * dxpsi1_(mxt) * dt;
-    const D2 x0 = dxpsi0_(xd), x1 = dxpsi1_(xd) * dd, x0m = dxpsi0_(mxd), x1m = -1.0 * dxpsi1_(mxd) * dd;
-    D2 dpepdd = ye * dh3(N, xt0, xt1, xt0m, xt1m, x0, x1, x0m, x1m);
+    dT.w0 = ddpsi0_(xt) * dti;
+    dT.w1 = ddpsi1_(xt);
+    dT.w2 = ddpsi2_(xt) * dt;
+    dT.w0m = -1.0 * ddpsi0_(mxt) * dti;
+    dT.w1m = ddpsi1_(mxt);
+    dT.w2m = -1.0 * ddpsi2_(mxt) * dt;
+    ddT.w0 = dddpsi0_(xt) * dt2i;
+    ddT.w1 = dddpsi1_(xt) * dti;
+    ddT.w2 = dddpsi2_(xt);
+    ddT.w0m = dddpsi0_(mxt) * dt2i;
+    ddT.w1m = -1.0 * dddpsi1_(mxt) * dti;
+    ddT.w2m = dddpsi2_(mxt);
+    D2 free = dc(0.0), df_d = dc(0.0), df_t = dc(0.0), df_dt = dc(0.0), df_tt = dc(0.0);
+    // the five sums together, column by column (64^3: A_prim 104 us; with the
+    // thirteen columns of the four nodes and weights of three components in
+    // registers, 512 of them and 110 spilled, 162)
+#define MC_COL(q, i, j)                                                 \
+    {                                                                   \
+        const Col N = node_col(tab.node, off, df_tt, q);                \
+        add_col(free, N, D.w##i, D.w##i##m, T.w##j, T.w##j##m);         \
+        add_col(df_d, N, dD.w##i, dD.w##i##m, T.w##j, T.w##j##m);       \
+        add_col(df_t, N, D.w##i, D.w##i##m, dT.w##j, dT.w##j##m);       \
+        add_col(df_dt, N, dD.w##i, dD.w##i##m, dT.w##j, dT.w##j##m);    \
+        add_col(df_tt, N, D.w##i, D.w##i##m, ddT.w##j, ddT.w##j##m);    \
+    }
+    MC_COL(NF, 0, 0)
+    MC_COL(NFT, 0, 1)
+    MC_COL(NFTT, 0, 2)
+    MC_COL(NFD, 1, 0)
+    MC_COL(NFDD, 2, 0)
+    MC_COL(NFDT, 1, 1)
+    MC_COL(NFDDT, 2, 1)
+    MC_COL(NFDTT, 1, 2)
+    MC_COL(NFDDTT, 2, 2)
+#undef MC_COL
+    const D1 xt0 = dxpsi0_(xt), xt1 = dxpsi1_(xt) * dt, xt0m = dxpsi0_(mxt), xt1m = -1.0 * dxpsi1_(mxt) * dt;
+    const D1 x0 = dxpsi0_(xd), x1 = dxpsi1_(xd) * dd, x0m = dxpsi0_(mxd), x1m = -1.0 * dxpsi1_(mxd) * dd;
+    D2 dpepdd = dc(0.0);
+    add_col(dpepdd, node_col(tab.node, off, df_tt, NDPDF), x0, x0m, xt0, xt0m);
+    add_col(dpepdd, node_col(tab.node, off, dpepdd, NDPDFT), x0, x0m, xt1, xt1m);
+    add_col(dpepdd, node_col(tab.node, off, dpepdd, NDPDFD), x1, x1m, xt0, xt0m);
+    add_col(dpepdd, node_col(tab.node, off, dpepdd, NDPDFDT), x1, x1m, xt1, xt1m);
+    dpepdd = ye * dpepdd;
     if (dpepdd.v < 0.0) dpepdd = dc(0.0);
 
     // e and its temperature derivative (for Gamma_1)

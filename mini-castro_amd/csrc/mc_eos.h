@@ -91,24 +91,6 @@ struct W6 {
     double w0, w1, w2, w0m, w1m, w2m;
 };
 
-// The four table nodes of a cell, 13 columns each.
-struct Nodes {
-    double a[EOS_NODE], b[EOS_NODE], c[EOS_NODE], d[EOS_NODE];  // (i,j) (i+1,j) (i,j+1) (i+1,j+1)
-};
-
-__device__ __forceinline__ void load_node(const double *p, double *o, int ncol)
-{
-    const double2 *q = reinterpret_cast<const double2 *>(p);
-#pragma unroll
-    for (int c = 0; c < EOS_NODE / 2; ++c) {
-        if (2 * c < ncol) {
-            double2 v = q[c];
-            o[2 * c] = v.x;
-            o[2 * c + 1] = v.y;
-        }
-    }
-}
-
 // One column of a biquintic or bicubic sum: the four nodes' values a b c d
 // (nodes (i,j) (i+1,j) (i,j+1) (i+1,j+1)) with the density weights (wd, wmd)
 // and temperature weights (wt, wmt), added to acc in h5's term order (the
