@@ -230,7 +230,7 @@ constexpr int NQT = FQ_G + 1;  // components of the tile (all but 1/rho)
 // STAGED: the primitives of cells pos-2 .. pos+2 come from the block's LDS
 // tile (component c of cell pos-2+q at tile[c * QTILE + self + q * sr])
 // instead of the cell arrays.
-template <bool STAGED>
+template <bool STAGED, bool STREAM = false>
 __device__ __forceinline__ void trace_hydro(const Ctx &x, int m, const FInst &I, int d, int i, int j, int k,
                                             bool own_p, FaceH &fp, FaceH &fm, const double *tile = nullptr,
                                             int self = 0, int sr = 0)
@@ -306,9 +306,9 @@ __device__ __forceinline__ void trace_hydro(const Ctx &x, int m, const FInst &I,
         f.rhoe = e_;
     };
     auto store_state = [&](double *S, idx_t ee, const StateH &o) {
-        EF2(S, I, NFS, FS_RHO, ee) = dbl2{o.rho, o.u};
-        EF2(S, I, NFS, FS_V, ee) = dbl2{o.v, o.w};
-        EF2(S, I, NFS, FS_P, ee) = dbl2{o.p, o.rhoe};
+        store2<STREAM>(EF2(S, I, NFS, FS_RHO, ee), dbl2{o.rho, o.u});
+        store2<STREAM>(EF2(S, I, NFS, FS_V, ee), dbl2{o.v, o.w});
+        store2<STREAM>(EF2(S, I, NFS, FS_P, ee), dbl2{o.p, o.rhoe});
     };
     double rho_p;
     {
@@ -381,6 +381,8 @@ __device__ __forceinline__ int below_of(int tid, int st) { return tid - st; }
 // minus state (the same values that brick stores) but not its plus state,
 // and solves no Riemann problem.  The sub-launches are the directions,
 // interleaved block by block like the other face stages.
+// Two thirds of its traffic are stores; STREAM sends them past the caches.
+template <bool STREAM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K_tflux(Plan3 p3, Ctx x)
 {
     __shared__ FaceH lds_h[256];           // the minus states
@@ -437,7 +439,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
     __syncthreads();
     FaceH fp, fm;
     if (ok) {
-        trace_hydro<true>(x, m, I, d, i, j, k, l > 0, fp, fm, tile, self, sr);
+        trace_hydro<true, STREAM>(x, m, I, d, i, j, k, l > 0, fp, fm, tile, self, sr);
         lds_h[tid] = fm;
     }
     __syncthreads();
@@ -447,7 +449,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
     // cells pos - 1 and pos: tile offsets 1 and 2 from the thread's row
     riemann_hydro(L, fp, tile[FQ_C * QTILE + self + sr], tile[FQ_C * QTILE + self + 2 * sr],
                   tile[FQ_G * QTILE + self + sr], tile[FQ_G * QTILE + self + 2 * sr], o);
-    store_tflux_h(x.FD[d], I, eidx(I, i, j, k), d, o);
+    store_tflux_h<STREAM>(x.FD[d], I, eidx(I, i, j, k), d, o);
 }
 
 // trans1 (Source/trans.F90:14-243) of the t-face states by the d-flux, then
@@ -1048,6 +1050,22 @@ static SpecPlan column_plan(FusedLevel *F, int slab, int per_tile, int &nblocks)
     return SpecPlan{tab, sb.blk0, F->ninst, sb.lz};
 }
 
+// cells of a launch over a slab
+static long launch_cells(const FusedLevel *F, int slab)
+{
+    long cells = 0;
+    for (const FInst &I : F->hsinst[slab]) cells += (long)I.n[0] * I.n[1] * I.zn;
+    return cells;
+}
+
+// K_tflux writes 528 bytes a cell, from 500,000 cells on more than the 256 MB
+// between the L2s and the memory hold until the next kernel reads them.
+// Stores past the caches then leave them to its inputs (128^3: 0.55 ms against
+// 0.66, 256^3 3.95 and 4.08, 192^3 in slabs of 32 planes 1.93 and 2.28 a step);
+// of what fits, the next kernel reads less from them (a step of 45 x 37 x 29
+// 231 us against 227, of the adjoint's 64^3 1.5% of its forward pass).
+constexpr long STREAM_MIN = 500000;
+
 // Whether a step that runs the transverse stage by cells joins it with the
 // final fluxes (K_transfinal).  Its blocks march through few planes on a small
 // level and wait for memory with nothing else on their CU; from some 200,000
@@ -1060,9 +1078,7 @@ constexpr long JOINT_MIN = 200000;
 static bool joins_transverse(const FusedLevel *F, int slab)
 {
     if ((F->variant & FV_FACE_TRANS1) || F->keep_transverse) return false;
-    long cells = 0;
-    for (const FInst &I : F->hsinst[slab]) cells += (long)I.n[0] * I.n[1] * I.zn;
-    return cells >= JOINT_MIN;
+    return launch_cells(F, slab) >= JOINT_MIN;
 }
 
 int plan_blocks(FusedLevel *F, const Plan &p)
@@ -1109,7 +1125,11 @@ static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, in
         const int nb = std::max(q.nb[0], std::max(q.nb[1], q.nb[2]));
         if (nb <= 0) return;
         const KernelTiling &t = F->tiling[stage];
-        if (stage == ST_TFLUX) hipLaunchKernelGGL(K_tflux, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
+        if (stage == ST_TFLUX) {
+            if (launch_cells(F, slab) >= STREAM_MIN)
+                hipLaunchKernelGGL(K_tflux<true>, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
+            else hipLaunchKernelGGL(K_tflux<false>, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
+        }
         else if (stage == ST_TRANS1C) hipLaunchKernelGGL(K_trans1c, dim3(6 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);
         else {
             hipLaunchKernelGGL(K_finalc, dim3(3 * nb), dim3(t.bx * t.by), 0, s, q, F->ctx);

@@ -382,6 +382,16 @@ __device__ __forceinline__ FaceH to_face(const QStateH &o, int d)
 }
 
 // Non-species part of a transverse-stage flux; momenta in absolute order.
+// A store of a pair; STREAM: past the caches, for data nothing reads before
+// they have let it go.
+template <bool STREAM>
+__device__ __forceinline__ void store2(gdbl2 &d, const dbl2 &v)
+{
+    if constexpr (STREAM) __builtin_nontemporal_store(v, &d);
+    else d = v;
+}
+
+template <bool STREAM = false>
 __device__ __forceinline__ void store_tflux_h(double *F, const FInst &I, idx_t e, int d, const RiemannH &o)
 {
     // momentum FF_MX + d is the normal one; then FF_MY (d = 0) or FF_MX, then
@@ -389,10 +399,10 @@ __device__ __forceinline__ void store_tflux_h(double *F, const FInst &I, idx_t e
     const double mx = d == 0 ? o.f_mn : o.f_mt;
     const double my = d == 0 ? o.f_mt : (d == 1 ? o.f_mn : o.f_mtt);
     const double mz = d == 2 ? o.f_mn : o.f_mtt;
-    EF2(F, I, NFF, FF_RHO, e) = dbl2{o.f_rho, o.fpl};
-    EF2(F, I, NFF, FF_MX, e) = dbl2{mx, my};
-    EF2(F, I, NFF, FF_MZ, e) = dbl2{mz, o.f_E};
-    EF2(F, I, NFF, FF_GP, e) = dbl2{o.g_p, o.g_un};
+    store2<STREAM>(EF2(F, I, NFF, FF_RHO, e), dbl2{o.f_rho, o.fpl});
+    store2<STREAM>(EF2(F, I, NFF, FF_MX, e), dbl2{mx, my});
+    store2<STREAM>(EF2(F, I, NFF, FF_MZ, e), dbl2{mz, o.f_E});
+    store2<STREAM>(EF2(F, I, NFF, FF_GP, e), dbl2{o.g_p, o.g_un});
 }
 
 // Riemann problem on face (i,j,k) of direction d (cells i-e_d and i)
