@@ -780,6 +780,10 @@ int mc_level_advance(mc_level_t *L, double dt)
 int mc_level_post_timestep(mc_level_t *L)
 {
     if (L->mode == MC_MODE_FUSED && !L->defer_post) return 0; /* folded into the fused update */
+    if (!eos_ready()) {  // the clean reads the table
+        set_error("mc_level_post_timestep: EOS table not initialised");
+        return -1;
+    }
     // a fused coarse level of a register: the clean runs on S_new, which the
     // engine takes back at the next step
     if (L->mode == MC_MODE_FUSED && sync_from_fused(L)) return -1;
