@@ -1161,6 +1161,10 @@ int mc_adjoint_backward(mc_adjoint_t *A, const double *Ub_final, double *Ub0)
         set_error("mc_adjoint_backward: bad arguments or no forward pass");
         return -1;
     }
+    if (!eos_ready()) {
+        set_error("mc_adjoint_backward: EOS table not loaded");
+        return -1;
+    }
     hipStream_t s = cur_stream();
     FusedLevel *F = A->F;
     const long nD = A->nD;
