@@ -428,7 +428,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void K
         } else {
             a = i0 + c % p.bx;
             b = j0 + c / p.bx;
-            cz = k0 - 2 + r;
+            // a brick's layers above the range read its last one: their planes
+            // may be beyond those a slab's ring buffer has (plane_w)
+            cz = min(k0 - 2 + r, I.zlo + I.zn + 2);
         }
         const idx_t ce = widx(I, a, b, cz);
 #pragma unroll
