@@ -269,7 +269,8 @@ int mc_level_sync(mc_level_t *L);
    fluxes: about 1.8 KB per cell together) for the whole level, or for one
    z-slab of `planes` cell planes at a time, the stages then running slab
    after slab (the state's 0.16 KB per cell plus 1.8 KB per cell of one slab
-   and its neighbouring planes).  Results are the same bit for bit.  planes = -1 (the
+   and its neighbouring planes; up to 2,000,000 cells the primitives, 0.24 KB
+   of the 1.8, stay whole).  Results are the same bit for bit.  planes = -1 (the
    default) keeps the whole level when that takes at most half the free
    device memory, else picks the deepest slab that does; 0 forces the whole
    level.  Changing it rebuilds the engine (state and clock kept).

@@ -1152,7 +1152,7 @@ static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, in
     switch (stage) {
     case ST_EST: hipLaunchKernelGGL(K_est, g, b, 0, s, p, F->ctx); break;
     case ST_PRIM:
-        if (F->slab) {
+        if (F->ring) {
             if (slab == 0)  // the boundary planes the step's images are made from
                 hipLaunchKernelGGL(K_save_planes, dim3((unsigned)((F->totP + 255) / 256)), dim3(256), 0, s, F->inst,
                                    F->ninst, F->totP, F->ctx);
@@ -1208,6 +1208,22 @@ static KernelTiling cell_tiling(const std::vector<FInst> &inst)
     return t;
 }
 
+// Planes of an instance's primitives (Q, U1, U1X) in an engine of `slab`
+// planes (0: no slabs): all of them, made by one K_prim before the first slab,
+// or a ring of the slab's and WHALO either side, to which every slab's K_prim
+// adds its own.  The ring saves memory alone: a launch of K_prim on a few
+// planes is no shorter than three Newton solves in turn take (some 18 us), and
+// a periodic instance's images are solved again (a step of 32^3 in slabs of 8
+// planes 479 us with the ring, 418 without; 96^3 of 16 2.48 and 2.38 ms; 128^3
+// of 32 4.48 and 4.44; 256^3 of 32 29.7 and 29.3).  Up to 2,000,000 cells it would save less
+// than half a gigabyte.
+constexpr long PRIM_WHOLE_MAX = 2000000;
+static int prim_planes(const int *n, int slab)
+{
+    if (slab <= 0 || (long)n[0] * n[1] * n[2] <= PRIM_WHOLE_MAX) return n[2];
+    return std::min(n[2], std::min(slab, n[2]) + 2 * WHALO);
+}
+
 FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int slab)
 {
     FusedLevel *F = new FusedLevel();
@@ -1243,7 +1259,7 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
             delete F;
             return nullptr;
         }
-        const int wR = F->slab ? std::min(F->slab, sp.n[2]) + 2 * WHALO : sp.n[2];
+        const int wR = prim_planes(sp.n, F->slab);
         I.nW = (long)I.n[0] * I.n[1] * wR;
         I.nQ = I.nW + (I.nW & 1);  // even, like nE
         I.offW = offW;
@@ -1253,7 +1269,8 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
         I.whi = sp.n[2] - 1;
         I.wz = 0;
         I.wR = 1 << 30;
-        if (F->slab) {  // images of a periodic instance have planes of their own
+        if (wR < sp.n[2]) {  // a ring: images of a periodic instance have planes of their own
+            F->ring = true;
             I.wwrap = 0;
             if (I.periodic) {
                 I.wlo = -(1 << 29);
@@ -1278,21 +1295,24 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
         for (FInst &I : F->hsinst[sl]) {
             I.zlo = sl * F->slab;
             I.zn = std::max(0, std::min(F->slab, I.n[2] - I.zlo));
+            if (I.nW == I.nD) continue;
             // the ring holds planes [zlo - WHALO, zlo + zn + WHALO), plane k in
             // slot k mod wR
             const int first = I.zlo - WHALO;
             I.wz = first - ((first % I.wR) + I.wR) % I.wR;
         }
-    // K_prim of slab sl adds the planes up to WHALO above it
+    // K_prim of slab sl adds the planes up to WHALO above it to a ring; that of
+    // the first makes all planes of an instance without one
     F->hpinst = F->hsinst;
     if (F->slab)
         for (int m = 0; m < F->ninst; ++m) {
             const FInst &H = F->hinst[m];
-            int k0 = H.periodic ? -WHALO : 0;
-            const int top = H.periodic ? H.n[2] + WHALO : H.n[2];
+            const bool whole = H.nW == H.nD;
+            int k0 = H.periodic && !whole ? -WHALO : 0;
+            const int top = H.periodic && !whole ? H.n[2] + WHALO : H.n[2];
             for (int sl = 0; sl < F->nslab; ++sl) {
                 FInst &I = F->hpinst[sl][m];
-                const int k1 = I.zn > 0 ? std::min(I.zlo + I.zn + WHALO, top) : k0;
+                const int k1 = whole ? top : (I.zn > 0 ? std::min(I.zlo + I.zn + WHALO, top) : k0);
                 I.zlo = k0;
                 I.zn = std::max(0, k1 - k0);
                 k0 = std::max(k0, k1);
@@ -1331,7 +1351,7 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     A(x.U1, NU1 * offW);
     A(x.U1X, 2L * NSPEC_PAIRS * offQ);
     A(x.Q, NFQ * offW);
-    if (F->slab) A(x.UB, NVAR * offP);
+    if (F->ring) A(x.UB, NVAR * offP);
     A(x.FL, offE);
     A(x.RW, 6 * offE);
     A(x.DV, offE);
@@ -1478,14 +1498,14 @@ size_t fused_bytes_for(const std::vector<FusedInstanceSpec> &spec, int slab)
     for (const auto &sp : spec) {
         const long nxy = (long)sp.n[0] * sp.n[1], nD = nxy * sp.n[2];
         const int ez = (slab > 0 ? std::min(slab, sp.n[2]) : sp.n[2]) + 2;
-        const long nW = slab > 0 ? nxy * (ez - 2 + 2 * WHALO) : nD;
+        const long nW = nxy * prim_planes(sp.n, slab);
         long nE = (long)(sp.n[0] + 2) * (sp.n[1] + 2) * ez;
         nE += nE & 1;
         cells += nD;
         win += nW;
         ext += nE;
         q += nW + (nW & 1);
-        if (slab > 0) planes += nxy * 2 * WHALO;
+        if (nW < nD) planes += nxy * 2 * WHALO;
     }
     const size_t per_ext = 2 + 6 + 3 * (2 * NFS + NFF + NFN) + 6 * NFF;
     return sizeof(double) *

@@ -49,8 +49,8 @@ struct FInst {
     long offD, offE;  // cell offsets in the cell / extended index spaces
     long nD, nE;      // cell counts
     // The primitives and the cleaned state (Q, U1, U1X) cover the whole
-    // instance, or in slabs a ring buffer of the slab's planes and WHALO
-    // more on either side: cell offset and count, and the same made even
+    // instance, or, of a large one in slabs, a ring buffer of the slab's planes
+    // and WHALO more on either side: cell offset and count, and the same made even
     // (U1X's pairs).
     long offW, nW, offQ, nQ;
     // plane k of these arrays is plane_w(I, k): wrapped or clamped to [wlo,
@@ -78,7 +78,7 @@ struct Plan {
 struct Ctx {
     const FInst *inst;
     double *U, *U1, *U1X, *Q, *FL, *DV;
-    double *UB;  // slabs: the state's first and last WHALO planes as the step found them
+    double *UB;  // with such rings: the state's first and last WHALO planes as the step found them
     double *RW;  // per ring cell and direction: the densities of its plus and minus states (3 pairs)
     double *SM[3], *SP[3], *FD[3], *FT[6], *FN[3];
     double *dt_cur, *dt_est, *time;
@@ -543,6 +543,7 @@ struct FusedLevel {
     // slab count, and one instance table per slab (zlo, zn set; slab 0 of a
     // whole-instance engine is `inst` itself)
     int slab = 0, nslab = 1;
+    bool ring = false;  // some instance's primitives are a ring of planes
     std::vector<FInst *> sinst;
     std::vector<std::vector<FInst>> hsinst;
     // and one per slab for K_prim, whose planes run ahead of the slab's

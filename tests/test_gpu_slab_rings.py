@@ -1,6 +1,8 @@
 """The ring of planes that holds an engine's primitives in slabs: large levels
 in slabs, shallow and deep, with a last slab of fewer planes, equal the
-whole-level engine bit for bit."""
+whole-level engine bit for bit; which levels keep one."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -41,3 +43,40 @@ def test_large_level_in_slabs_matches_whole_level(n, bc, slab, tflux):
         L.close()
     np.testing.assert_array_equal(out[0][0], out[1][0])
     assert out[0][1:] == out[1][1:]
+
+
+def nbytes(n, slab):
+    return mc.lib().mc_fused_bytes(1, (C.c_int * 3)(*n), slab)
+
+
+def test_small_levels_keep_whole_primitives():
+    """A level of up to 2,000,000 cells holds the state and the primitives whole
+    (50 doubles a cell), so that one launch makes them; a larger one holds the
+    primitives of the slab's neighbourhood, unless the level is no deeper.  The
+    face arrays take less than 200 doubles a cell of the slab and its ring."""
+    def face(n, slab):
+        return 8 * 200 * (n[0] + 2) * (n[1] + 2) * (slab + 2)
+    for n, slab in (((100, 100, 100), 4), ((2000, 1000, 1), 0), ((1000, 1000, 9), 1), ((1000, 1000, 9), 8)):
+        whole = 8 * 50 * n[0] * n[1] * n[2]
+        assert whole <= nbytes(n, slab) < whole + face(n, slab or n[2])
+    for n, slab in (((150, 150, 150), 4), ((420, 360, 14), 1), ((127, 126, 126), 31)):
+        planes = 20 * n[2] + 30 * (slab + 8) + 20 * 8
+        assert nbytes(n, slab) < 8 * n[0] * n[1] * planes + face(n, slab)
+
+
+def test_members_with_and_without_rings():
+    """Large members before, between and after small ones, periodic and not."""
+    members = [((8, 9, 30), 0), ((127, 126, 126), 0), ((30, 20, 40), 1), ((130, 128, 121), 1), ((12, 10, 5), 0)]
+    insts = []
+    for (n, bc), r in zip(members, (0.2, 0.8, 0.5, 0.7, 0.2)):
+        insts.append(small_cfg(n=16, bc=bc, n_cell=n, prob_hi=tuple(v / 32.0 for v in n), r_init=r))
+    out = []
+    for slab in (0, 20):
+        E = mc.Ensemble(insts, slab=slab)
+        E.init_data()
+        E.run(3)
+        out.append([(E.state(m), E.clock(m)) for m in range(len(insts))])
+        E.close()
+    for m, ((a, ca), (b, cb)) in enumerate(zip(*out)):
+        np.testing.assert_array_equal(a, b, err_msg="member %d" % m)
+        assert ca == cb and ca[2] == 3
