@@ -427,7 +427,9 @@ mc_ensemble_t *mc_ensemble_create_slabs(int ninst, const int *n_cell, const doub
 int mc_ensemble_slab(const mc_ensemble_t *E);
 /* device bytes the fused engine holds for these instances (state, cell
    arrays, face arrays) with z-slabs of `planes` cell planes (0: whole
-   instances); a host computation, no device needed */
+   instances), at most: large outflow instances in slabs hold 1.3 KB less for
+   each column of cells than periodic ones; a host computation, no device
+   needed */
 long mc_fused_bytes(int ninst, const int *n_cell, int planes);
 void mc_ensemble_destroy(mc_ensemble_t *E);
 int mc_ensemble_ninst(const mc_ensemble_t *E);

@@ -143,8 +143,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void K
     WA(x.Q, I, NFQ, FQ_G, cw) = q.gamc;
 }
 
-// Slabs: the first and last WHALO planes of every instance's state (wrapped
-// for instances shallower than that), before the step's first clean.
+// Rings: the first and last WHALO planes of every periodic instance's state
+// (wrapped for instances shallower than that), before the step's first clean.
+// Instances without such images, and without a ring, have none (192^3 outflow
+// in slabs of 32: 47 MB each way a step that nothing read).
 __global__ __launch_bounds__(256) void K_save_planes(const FInst *inst, int ninst, long n, Ctx x)
 {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1153,7 +1155,7 @@ static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, in
     case ST_EST: hipLaunchKernelGGL(K_est, g, b, 0, s, p, F->ctx); break;
     case ST_PRIM:
         if (F->ring) {
-            if (slab == 0)  // the boundary planes the step's images are made from
+            if (slab == 0 && F->totP)  // the boundary planes the step's images are made from
                 hipLaunchKernelGGL(K_save_planes, dim3((unsigned)((F->totP + 255) / 256)), dim3(256), 0, s, F->inst,
                                    F->ninst, F->totP, F->ctx);
             hipLaunchKernelGGL(K_prim<true>, g, b, 0, s, p, F->ctx);
@@ -1275,9 +1277,9 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
             if (I.periodic) {
                 I.wlo = -(1 << 29);
                 I.whi = 1 << 29;
+                offP += (long)I.n[0] * I.n[1] * 2 * WHALO;
             }
             I.wR = wR;
-            offP += (long)I.n[0] * I.n[1] * 2 * WHALO;
         }
         I.offD = offD;
         I.offE = offE;
@@ -1351,7 +1353,7 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     A(x.U1, NU1 * offW);
     A(x.U1X, 2L * NSPEC_PAIRS * offQ);
     A(x.Q, NFQ * offW);
-    if (F->ring) A(x.UB, NVAR * offP);
+    if (offP) A(x.UB, NVAR * offP);
     A(x.FL, offE);
     A(x.RW, 6 * offE);
     A(x.DV, offE);
@@ -1505,7 +1507,7 @@ size_t fused_bytes_for(const std::vector<FusedInstanceSpec> &spec, int slab)
         win += nW;
         ext += nE;
         q += nW + (nW & 1);
-        if (nW < nD) planes += nxy * 2 * WHALO;
+        if (nW < nD && sp.bc == 0) planes += nxy * 2 * WHALO;
     }
     const size_t per_ext = 2 + 6 + 3 * (2 * NFS + NFF + NFN) + 6 * NFF;
     return sizeof(double) *

@@ -78,7 +78,7 @@ struct Plan {
 struct Ctx {
     const FInst *inst;
     double *U, *U1, *U1X, *Q, *FL, *DV;
-    double *UB;  // with such rings: the state's first and last WHALO planes as the step found them
+    double *UB;  // periodic rings: the state's first and last WHALO planes as the step found them
     double *RW;  // per ring cell and direction: the densities of its plus and minus states (3 pairs)
     double *SM[3], *SP[3], *FD[3], *FT[6], *FN[3];
     double *dt_cur, *dt_est, *time;

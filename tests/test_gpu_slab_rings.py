@@ -80,3 +80,21 @@ def test_members_with_and_without_rings():
     for m, ((a, ca), (b, cb)) in enumerate(zip(*out)):
         np.testing.assert_array_equal(a, b, err_msg="member %d" % m)
         assert ca == cb and ca[2] == 3
+
+
+def test_saved_planes_of_periodic_members_only():
+    """Outflow and small members, which save no boundary planes, before and
+    between periodic ones that do."""
+    members = [((130, 128, 121), 1), ((9, 12, 40), 0), ((127, 126, 126), 0), ((131, 126, 122), 1), ((300, 210, 32), 0)]
+    insts = [small_cfg(n=16, bc=bc, n_cell=n, prob_hi=tuple(v / 32.0 for v in n), r_init=0.1 + 0.1 * m)
+             for m, (n, bc) in enumerate(members)]
+    out = []
+    for slab in (0, 9):
+        E = mc.Ensemble(insts, slab=slab)
+        E.init_data()
+        E.run(2)
+        out.append([(E.state(m), E.clock(m)) for m in range(len(insts))])
+        E.close()
+    for m, ((a, ca), (b, cb)) in enumerate(zip(*out)):
+        np.testing.assert_array_equal(a, b, err_msg="member %d" % m)
+        assert ca == cb
