@@ -108,6 +108,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void K
 #pragma unroll
         for (int n = 0; n < NVAR; ++n) u[n] = ub[n * np];
     }
+    // an image's unconverged solves are its source cell's, counted there
+    if (SLABS && !own) x.tab.newton_fail = nullptr;
     clean_cell(u, x.tab); /* S_old clean, Castro_advance.cpp:51 */
     // S_old is replaced by its clean in place: K_update starts from it
     // instead of cleaning S_old a second time (nothing between reads U)

@@ -9,7 +9,7 @@ import pytest
 import minicastro as mc
 from minicastro import configs
 from helpers import small_cfg, table_bin
-from test_gpu_species import mixed_flow
+from test_gpu_species import UEDEN, UEINT, mixed_flow
 
 pytestmark = pytest.mark.gpu
 
@@ -98,3 +98,28 @@ def test_saved_planes_of_periodic_members_only():
     for m, ((a, ca), (b, cb)) in enumerate(zip(*out)):
         np.testing.assert_array_equal(a, b, err_msg="member %d" % m)
         assert ca == cb
+
+
+def test_unconverged_solves_counted_once():
+    """Cells whose solves do not converge, at the periodic boundary in z: their
+    images in the ring are not counted again."""
+    n = (127, 126, 126)
+    hi = tuple(v / 16.0 for v in n)
+    cfg = small_cfg(n=16, bc=0)
+    S = mixed_flow(n, seed=3)
+    for c in ((5, 7, 0), (60, 1, 3), (100, 125, 124), (0, 64, 125), (30, 30, 60)):
+        S[c][[UEDEN, UEINT]] = np.inf
+    counts, states = [], []
+    for slab in (0, 40, 5):
+        L = mc.Level(n, configs.grid_boxes(n, 512), cfg["prob_lo"], hi, 0, mc.MODE_FUSED)
+        L.set_fused_slab(slab)
+        L.set_state(S)
+        mc.newton_failures(reset=True)
+        L.advance(1e-9)
+        L.sync()
+        counts.append(mc.newton_failures(reset=True))
+        states.append(L.state())
+        L.close()
+    assert counts[0] > 0 and counts == counts[:1] * 3
+    for s in states[1:]:
+        np.testing.assert_array_equal(s, states[0])
