@@ -414,7 +414,8 @@ void mc_advance_batch_release(void);
    MC_MODE_FUSED levels, mc_advance_batch, the adjoint) takes instances of
    fewer than 2^29 cells; with its face arrays covering whole instances (no
    z-slabs, and always for the adjoint) also fewer than 2^28 cells including
-   one ghost layer, (nx+2)(ny+2)(nz+2) < 2^28.  Larger ones are refused with
+   one ghost layer, (nx+2)(ny+2)(nz+2) < 2^28; in z-slabs of p planes fewer than
+   2^28 cells of nx ny min(nz, p+8).  Larger ones are refused with
    an error before any device memory is taken. */
 typedef struct mc_ensemble mc_ensemble_t;
 /* n_cell, prob_lo, prob_hi: 3 per instance; bc: one per instance */

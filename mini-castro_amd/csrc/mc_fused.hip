@@ -1265,6 +1265,12 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
         }
         const int wR = prim_planes(sp.n, F->slab);
         I.nW = (long)I.n[0] * I.n[1] * wR;
+        if (I.nW >= (1L << 28)) {  // 16-byte lane offsets of the species pairs (U1X) are 32-bit
+            set_error("fused engine: the planes of an instance's primitives (a slab's and four either side) may hold at "
+                      "most 2^28 cells (run it in shallower z-slabs)");
+            delete F;
+            return nullptr;
+        }
         I.nQ = I.nW + (I.nW & 1);  // even, like nE
         I.offW = offW;
         I.offP = offP;
