@@ -298,7 +298,11 @@ int mc_level_set_brick_order(mc_level_t *L, int stage, int zgroup);
 int mc_level_brick_order(mc_level_t *L, int stage);
 /* Launch one fused stage on the current device state (for timing).  The
    prim stage replaces the state by its clean and the update stage advances
-   it, both in place; the other stages leave it unchanged. */
+   it, both in place; the other stages leave it unchanged.  By itself a stage
+   reads the arrays the stages before it left and writes its own: the kernels
+   that a step joins (mc_level_set_stage_variant) run apart, and a final stage
+   straight after such a step runs trans1c first, once.  In z-slabs the stage
+   runs over every slab, and the arrays between the stages hold the last. */
 int mc_level_run_stage(mc_level_t *L, int stage);
 /* Fused mode: time every candidate brick of every stage of every kernel
    variant (reps launches each) on the data of one coarse step and keep the

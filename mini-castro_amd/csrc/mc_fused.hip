@@ -1638,6 +1638,14 @@ static void enqueue_slab(FusedLevel *F, int sl, hipStream_t s)
     for (int st : step_stages(F)) launch_stage(F, st, s, stage_ny[st], sl);
 }
 
+// what a step leaves of the transverse fluxes (FusedLevel::have_transverse)
+static void note_step(FusedLevel *F)
+{
+    F->have_transverse = true;
+    for (int sl = 0; sl < F->nslab; ++sl)
+        if (joins_transverse(F, sl)) F->have_transverse = false;
+}
+
 // enqueue one coarse step of every instance, slab after slab: K_prim on the
 // planes the slab's face stages are the first to read, the face stages, and
 // K_update.  A slab's update rewrites only its own cells of the state, whose
@@ -1660,6 +1668,7 @@ int fused_steps_timed(FusedLevel *F, int nsteps, double stop_time, hipStream_t s
         return -1;
     }
     if (!F->have_est && fused_estimate(F, s)) return -1;
+    if (nsteps > 0) note_step(F);
     const std::vector<int> slab_order = step_stages(F);
     const int nso = (int)slab_order.size();
     const int *ny = stage_ny;
@@ -1717,6 +1726,7 @@ int fused_steps(FusedLevel *F, int nsteps, double stop_time, hipStream_t s, bool
         return -1;
     }
     if (!F->have_est && fused_estimate(F, s)) return -1;
+    if (nsteps > 0) note_step(F);
     if (!use_graph) {
         for (int n = 0; n < nsteps; ++n) enqueue_step(F, stop_time, s);
         return check_hip(hipGetLastError(), "fused_steps");
@@ -1760,6 +1770,7 @@ int fused_advance_dt(FusedLevel *F, double dt, hipStream_t s)
     fill(F->ctx.dt_cur, F->ninst, dt, s);
     fill(F->ctx.dt_est, F->ninst, DBL_MAX, s);
     for (int sl = 0; sl < F->nslab; ++sl) enqueue_slab(F, sl, s);
+    note_step(F);
     F->have_est = true;
     return check_hip(hipGetLastError(), "fused_advance_dt");
 }
@@ -1907,9 +1918,16 @@ int fused_run_stage(FusedLevel *F, int stage, hipStream_t s)
     // by itself a stage reads and writes the arrays between the stages
     const bool keep = F->keep_transverse;
     F->keep_transverse = true;
+    // a final stage after a step whose K_transfinal left its transverse fluxes
+    // nowhere: they are made first
+    const bool make = (stage == ST_FINAL || stage == ST_FINALC) && !F->have_transverse;
     if (whole_instance_stage(stage)) launch_stage(F, stage, s, ny[stage]);
     else
-        for (int sl = 0; sl < F->nslab; ++sl) launch_stage(F, stage, s, ny[stage], sl);
+        for (int sl = 0; sl < F->nslab; ++sl) {
+            if (make) launch_stage(F, ST_TRANS1C, s, ny[ST_TRANS1C], sl);
+            launch_stage(F, stage, s, ny[stage], sl);
+        }
+    if (!F->slab && (make || stage == ST_TRANS1 || stage == ST_TRANS1C)) F->have_transverse = true;
     F->keep_transverse = keep;
     return check_hip(hipGetLastError(), "fused_run_stage");
 }
@@ -1975,6 +1993,7 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (!rc) rc = check_hip(hipEventCreate(&e0), "hipEventCreate") || check_hip(hipEventCreate(&e1), "hipEventCreate");
     if (!rc) enqueue_step(F, -1.0, s);  // every intermediate array now holds data of a real step
+    F->have_transverse = true;          // K_trans1 is timed below
     const int *ny = stage_ny;
     auto restore_state = [&]() {
         return check_hip(hipMemcpyAsync(x.U, saveU, nU, hipMemcpyDeviceToDevice, s), "autotune restore");

@@ -539,6 +539,9 @@ struct FusedLevel {
     // the transverse fluxes are read after the step (the adjoint's engine):
     // K_transfinal, which keeps them on the chip, is not used
     bool keep_transverse = false;
+    // the arrays F^{t|d} hold the last step's fluxes, not just their mass
+    // fluxes and weights
+    bool have_transverse = true;
     // z-slabs of the face stages: planes per slab (0: the whole instance),
     // slab count, and one instance table per slab (zlo, zn set; slab 0 of a
     // whole-instance engine is `inst` itself)
