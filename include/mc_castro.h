@@ -311,7 +311,9 @@ int mc_level_run_stage(mc_level_t *L, int stage);
    (the stage variant below; mc_level_stage_variant reports it); the state
    and the clock are restored.  bricks (11 x 3 ints) and best_ms (11) receive every stage's
    tiling and the tuned stages' time per launch (0 for est, which is not
-   tuned); either may be NULL. */
+   tuned; trans1c's of 200,000 cells and more is of the kernel that takes the
+   final stage's hydro fluxes with it, and final's and finalc's include the
+   species); either may be NULL. */
 int mc_level_autotune(mc_level_t *L, int reps, int *bricks, double *best_ms);
 /* Fused mode: kernel variants of the step, bit flags (0, the default, runs
    the stages tflux, trans1c and final): MC_VARIANT_SPLIT_TRACE runs the

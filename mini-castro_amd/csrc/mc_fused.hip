@@ -2093,9 +2093,10 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
             }
         }
         F->tiling[st] = best;
+        tb[st] = tbest;
         if (joined && !rc) {
-            // its share: the launch and the species that are left, less the
-            // faster final stage it replaces
+            // what the choice compares is its share: the launch and the species
+            // that are left, less the faster final stage it replaces
             float one = 0.f;
             double sp = 0.0;
             for (int r = 0; r < reps && !rc; ++r) {
@@ -2106,9 +2107,8 @@ int fused_autotune(FusedLevel *F, int reps, hipStream_t s, int *bricks, double *
                      check_hip(hipEventElapsedTime(&one, e0, e1), "hipEventElapsedTime");
                 sp += one;
             }
-            tbest = std::max(tbest + sp / reps - std::min(tb[ST_FINAL], tb[ST_FINALC]), 1e-6);
+            tb[st] = tbest + sp / reps - std::min(tb[ST_FINAL], tb[ST_FINALC]);
         }
-        tb[st] = tbest;
         if (bricks) {
             bricks[3 * st] = best.bx;
             bricks[3 * st + 1] = best.by;
