@@ -88,20 +88,38 @@ __global__ void k_reg_fine_add(Box fb, long n, double *reg, Arr flx, int dir, in
 }
 
 // FineAdd from the fused engine's final fluxes (one instance covering the
-// fine level, whole-instance face arrays): component c of face (i,j,k) in
-// direction dir is FN[dir] at eidx, and store_flux's dt * F * area is formed
-// as k_store_flux forms it before the sum of k_reg_fine_add
-__device__ __forceinline__ double fn_component(double *FN, const FInst &I, int c, idx_t e)
+// fine level, whole-instance face arrays): the components of face (i,j,k) in
+// direction dir are FN[dir] at eidx, and store_flux's dt * F * area is formed
+// as k_store_flux forms it before the sum of k_reg_fine_add.  A face's
+// components are taken together, since its species fluxes are normalised by
+// their own sum, and a store between them would hold the next loads back (few
+// threads, each waiting for memory: registers of four 32^3 boxes of a 64^3 level,
+// one CrseInit and two FineAdds 680 us; a component at a time 3540).
+struct FaceFlux {
+    double f[NVAR];
+};
+__device__ __forceinline__ FaceFlux fn_flux(double *FN, const FInst &I, idx_t e)
 {
-    if (c == UTEMP) return 0.0;
-    if (c < UFS) return EF(FN, I, NFN, c, e);
-    const int sp = c - UFS;
+    FaceFlux o;
+#pragma unroll
+    for (int c = 0; c < UTEMP; c += 2) {
+        const dbl2 v = EF2(FN, I, NFN, c, e);
+        o.f[c] = v.x;
+        o.f[c + 1] = v.y;
+    }
+    o.f[UTEMP] = 0.0;
     const SpeciesPairs X = species_pairs(FN, I, NFN, FN_X);
-    const dbl2 v = SP2(X, sp >> 1, e);
-    return ((sp & 1) ? v.y : v.x) * species_fac(X, e, EF(FN, I, NFN, URHO, e));
+    const double fac = species_fac(X, e, o.f[URHO]);
+#pragma unroll
+    for (int pr = 0; pr < NSPEC_PAIRS; ++pr) {
+        const dbl2 v = SP2(X, pr, e);
+        o.f[UFS + 2 * pr] = v.x * fac;
+        if (2 * pr + 1 < NSPEC) o.f[UFS + 2 * pr + 1] = v.y * fac;
+    }
+    return o;
 }
 
-__global__ void k_reg_fine_add_fn(Box fb, long n, double *reg, double *FN, const FInst *inst, int dir, int r0,
+__global__ __launch_bounds__(kBlock) void k_reg_fine_add_fn(Box fb, long n, double *reg, double *FN, const FInst *inst, int dir, int r0,
                                   int r1, int r2, double dt, double area, double mult)
 {
     int i, j, k;
@@ -109,26 +127,20 @@ __global__ void k_reg_fine_add_fn(Box fb, long n, double *reg, double *FN, const
     if (!iter_cell(make_iter(fb), t, i, j, k)) return;
     const FInst &I = inst[0];
     const long l = face_local(fb, i, j, k);
-    for (int c = 0; c < NVAR; ++c) {
-        double r = reg[l + n * c];
-        if (dir == 0) {
-            const int ii = r0 * i;
-            for (int koff = 0; koff < r2; ++koff)
-                for (int joff = 0; joff < r1; ++joff)
-                    r += mult * (dt * fn_component(FN, I, c, eidx(I, ii, r1 * j + joff, r2 * k + koff)) * area);
-        } else if (dir == 1) {
-            const int jj = r1 * j;
-            for (int koff = 0; koff < r2; ++koff)
-                for (int ioff = 0; ioff < r0; ++ioff)
-                    r += mult * (dt * fn_component(FN, I, c, eidx(I, r0 * i + ioff, jj, r2 * k + koff)) * area);
-        } else {
-            const int kk = r2 * k;
-            for (int joff = 0; joff < r1; ++joff)
-                for (int ioff = 0; ioff < r0; ++ioff)
-                    r += mult * (dt * fn_component(FN, I, c, eidx(I, r0 * i + ioff, r1 * j + joff, kk)) * area);
-        }
-        reg[l + n * c] = r;
-    }
+    // the fine faces of a coarse one: x fastest, then y, then z
+    const int a0 = dir == 0 ? 1 : r0, a1 = dir == 1 ? 1 : r1, a2 = dir == 2 ? 1 : r2;
+    double r[NVAR];
+#pragma unroll
+    for (int c = 0; c < NVAR; ++c) r[c] = reg[l + n * c];
+    for (int ko = 0; ko < a2; ++ko)
+        for (int jo = 0; jo < a1; ++jo)
+            for (int io = 0; io < a0; ++io) {
+                const FaceFlux v = fn_flux(FN, I, eidx(I, r0 * i + io, r1 * j + jo, r2 * k + ko));
+#pragma unroll
+                for (int c = 0; c < NVAR; ++c) r[c] += mult * (dt * v.f[c] * area);
+            }
+#pragma unroll
+    for (int c = 0; c < NVAR; ++c) reg[l + n * c] = r[c];
 }
 
 // ClearInternalBorders: zero the face cells another fine box shares
@@ -289,7 +301,7 @@ int flux_register_fine_add_fused(mc_flux_register *R, const FusedLevel *F, doubl
 // CrseInit of every register face from the fused engine of the coarse
 // level: register = mult * (dt * F * area), as store_flux and
 // k_reg_crse_init form it
-__global__ void k_reg_crse_init_fn(Box fb, long n, double *reg, double *FN, const FInst *inst, double dt,
+__global__ __launch_bounds__(kBlock) void k_reg_crse_init_fn(Box fb, long n, double *reg, double *FN, const FInst *inst, double dt,
                                    double area, double mult)
 {
     int i, j, k;
@@ -298,7 +310,9 @@ __global__ void k_reg_crse_init_fn(Box fb, long n, double *reg, double *FN, cons
     const FInst &I = inst[0];
     const idx_t e = eidx(I, i, j, k);
     const long l = face_local(fb, i, j, k);
-    for (int c = 0; c < NVAR; ++c) reg[l + n * c] = (dt * fn_component(FN, I, c, e) * area) * mult;
+    const FaceFlux v = fn_flux(FN, I, e);
+#pragma unroll
+    for (int c = 0; c < NVAR; ++c) reg[l + n * c] = (dt * v.f[c] * area) * mult;
 }
 
 int flux_register_crse_init_fused(mc_flux_register *R, const FusedLevel *F, double dt, const double *area,
