@@ -83,7 +83,9 @@ def _kernel_bytes(kernel, n):
     return 8 * doubles
 
 
-JOINED_CELLS = 200000  # levels of this size run the transverse and final fluxes in one kernel
+# levels of this size run the transverse and final fluxes in one kernel
+# (JOINT_MIN of mc_fused.hip)
+JOINED_CELLS = 200000
 
 
 def stage_kernels(stage, n, variant):
@@ -576,7 +578,7 @@ def main():
                         "unit": "TFLOP/s", "frac": rate / FP64_PEAK, "ops_per_launch": ops}
     roofline["fp64_stages"] = fp64 or None
 
-    # per-box path (the reference's kernel order) on the same workload
+    # per-box path (the plain level driver) on the same workload
     plain = None
     if a.plain_steps > 0:
         P = mc.Level(n, cfg["boxes"], cfg["prob_lo"], cfg["prob_hi"], cfg["bc"], mc.MODE_PLAIN)

@@ -254,7 +254,10 @@ int mc_level_run(mc_level_t *L, int nsteps, double stop_time, int use_graph);
 /* Fused mode: nsteps eager steps with HIP events around every stage launch on
    the level's stream; stage_ms[0..11] / launches[0..11] receive per-stage
    totals (stages as in mc_level_set_tiling; index 11: the time-step control
-   kernels).  A stage the step does not run reports 0 launches. */
+   kernels).  A stage the step does not run reports 0 launches.  The species
+   count under final (finalc); where the transverse and final fluxes are one
+   kernel (mc_level_set_stage_variant), it counts under trans1c, and final
+   holds the species alone. */
 int mc_level_run_timed(mc_level_t *L, int nsteps, double stop_time, double *stage_ms, int *launches);
 int mc_level_steps(const mc_level_t *L);
 /* Castro::post_timestep's blast-radius diagnostic (Source/Castro.cpp:371-424):
@@ -321,7 +324,9 @@ int mc_level_autotune(mc_level_t *L, int reps, int *bricks, double *best_ms);
    of one (tflux); MC_VARIANT_FACE_TRANS1 the transverse-flux stage face by
    face (trans1) instead of cell by cell (trans1c); MC_VARIANT_CELL_FINAL
    the final-flux stage cell by cell (finalc) instead of face by face
-   (final).  Results are the same bit for bit. */
+   (final).  Without MC_VARIANT_FACE_TRANS1, launches of 200,000 cells and more
+   run the transverse and final stages in one kernel of its own, tilings and
+   MC_VARIANT_CELL_FINAL or not.  Results are the same bit for bit. */
 #define MC_VARIANT_SPLIT_TRACE 1
 #define MC_VARIANT_FACE_TRANS1 2
 #define MC_VARIANT_CELL_FINAL 4

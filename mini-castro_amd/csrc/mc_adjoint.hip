@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256) void A_final(Lines q, const FInst *inst, Ctx x
             div1_b += fnb[h] * dxd * (CA(x.U1, I, NU1, n, cr) - CA(x.U1, I, NU1, n, cl));
             g[h] = fnb[h] * dxd * div1;
         }
-        // a face that two bricks have is counted in the lower one
+        // a face that two bricks have is counted in the upper one
         if (draw < 0.0 && (l < top || cd == nd)) {
             const double v = 0.1 * FOURTH * div1_b;
             aadd(EAp(a.DVb, I, 1, 0, ep), v);

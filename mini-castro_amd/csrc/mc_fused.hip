@@ -1003,7 +1003,9 @@ static int column_tiles(const FInst &I)
 // 256^3: 3.5 us a plane of each CU with two, 5 us with one); the candidate
 // with the least total is taken.  Above 64 planes nothing is gained (256^3:
 // 14.46 ms for K_final and K_species with chunks of at most 32 and 128 planes,
-// 14.42 with 64, 14.80 with 256).
+// 14.42 with 64, 14.80 with 256).  K_transfinal's own best chunks are the same
+// (64^3 146 us with the choice, 147 to 695 with 2 to 48 planes; 128^3 869, 921 to
+// 1330; 256^3 6.03 ms, 5.94 with 16 planes and 5.96 to 8.7 with others).
 static int column_chunk(const std::vector<FInst> &inst, int per_tile)
 {
     constexpr double cus = 256.0;
@@ -1079,7 +1081,12 @@ constexpr long STREAM_MIN = 500000;
 // joined against K_trans1c, K_final and K_species: 40^3 121 : 107, 48^3
 // 184 : 172, 56^3 227 : 224, 30 x 30 x 200 331 : 328, 128 x 40 x 40 291 : 296,
 // 64^3 373 : 407, 80^3 570 : 682, 96^3 1001 : 1171, 256^3 15.7 : 19.0 ms;
-// a step of 1000 members of 4^3 17.6 : 17.8 ms).
+// a step of 1000 members of 4^3 17.6 : 17.8 ms).  With their first bricks the
+// faster kernels of either stage are these two at every size: a step with
+// trans1c and final, trans1 and final, trans1c and finalc, trans1 and finalc
+// takes 107, 112, 116, 115 us at 16^3, 211, 219, 216, 221 at 40^3, 411, 430, 423,
+// 429 at 56^3, and with the first and third joined 621, 695, 635, 709 at 64^3,
+// 27.7, 31.0, 27.8, 31.7 ms at 256^3.
 constexpr long JOINT_MIN = 200000;
 static bool joins_transverse(const FusedLevel *F, int slab)
 {
@@ -1334,7 +1341,9 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
     F->totW = offW;
     F->totP = offP;
     for (int s = 0; s < NSTAGE; ++s) F->tiling[s] = KernelTiling{64, 2, 2};
-    F->tiling[ST_FLAT] = KernelTiling{16, 2, 2};  // stencils in all directions (256^3: 706 us, 64 x 2 x 2 750)
+    // stencils in all directions (us against 64 x 2 x 2: 16^3 7.4 : 8.0, 32^3 9.3 : 10.6,
+    // 48^3 13.2 : 12.7, 64^3 19.4 : 26.0, 96^3 44 : 47, 128^3 101 : 118, 256^3 708 : 748)
+    F->tiling[ST_FLAT] = KernelTiling{16, 2, 2};
     F->tiling[ST_EST] = F->tiling[ST_PRIM] = F->tiling[ST_UPDATE] = cell_tiling(F->hinst);
     F->tiling[ST_TFLUX] = F->tiling[ST_TRANS1C] = F->tiling[ST_FINALC] = KernelTiling{16, 16, 64};
     bool ok = !check_hip(hipMalloc(&F->inst, sizeof(FInst) * F->ninst), "hipMalloc(inst)") &&

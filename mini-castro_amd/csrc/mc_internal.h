@@ -32,8 +32,6 @@ struct ProblemConsts {
 void initdata_with(const ProblemConsts &pc, const int *lo, const int *hi, double *state, const int *state_lo,
                    const int *state_hi, const double *dx, const double *problo, const double *probhi);
 
-// Asynchronous estdt over box bx of a state FAB on sbox: min-reduces the
-// CFL time step of every cell into *dt_dev (no synchronisation).
 // a box of an arena of FABs
 struct BoxDesc {
     BoxIter it;
@@ -46,6 +44,8 @@ void launch_clean_boxes(const BoxDesc *d, int nbox, long nmax, double *arena, hi
 void launch_finish_flux(const Box &b, int idir, double dxd, const double *div, const Box &divb, const double *u,
                         const Box &ub, double *flux, const Box &fb, double *fo, const Box &fob, const double *area,
                         const Box &areab, double dt, hipStream_t s);
+// Asynchronous estdt over box bx of a state FAB on sbox: min-reduces the
+// CFL time step of every cell into *dt_dev (no synchronisation).
 void launch_estdt(const Box &bx, const double *state, const Box &sbox, const double *dx, double *dt_dev,
                   hipStream_t s);
 
