@@ -921,6 +921,7 @@ static bool ovl_tiling_ok(const KernelTiling &t)
 static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int slab, int ovl, bool prim = false)
 {
     const FInst *tab = slab < 0 ? F->inst : (prim ? F->pinst[slab] : F->sinst[slab]);
+    if (slab >= 0 && !prim) slab = F->like[slab];
     for (auto &pb : F->plans)
         if (pb.t.bx == t.bx && pb.t.by == t.by && pb.t.bz == t.bz && pb.t.zg == t.zg && pb.shift == sh &&
             pb.add == add && pb.slab == slab && pb.ovl == ovl && pb.prim == prim)
@@ -961,6 +962,7 @@ static Plan plan_for(FusedLevel *F, const KernelTiling &t, int sh, int add, int 
 Plan get_plan(FusedLevel *F, int stage, int slab)
 {
     if (whole_instance_stage(stage)) slab = -1;
+    if (stage == ST_PRIM && !F->ring) slab = 0;
     return plan_for(F, F->tiling[stage], stage_shift[stage], stage_add[stage], slab, -1, stage == ST_PRIM);
 }
 
@@ -1031,6 +1033,7 @@ static int column_chunk(const std::vector<FInst> &inst, int per_tile)
 static SpecPlan column_plan(FusedLevel *F, int slab, int per_tile, int &nblocks)
 {
     const FInst *tab = F->sinst[slab];
+    slab = F->like[slab];
     for (auto &sb : F->specs)
         if (sb.slab == slab && sb.per_tile == per_tile) {
             nblocks = sb.nblocks;
@@ -1049,6 +1052,12 @@ static SpecPlan column_plan(FusedLevel *F, int slab, int per_tile, int &nblocks)
     }
     b0[F->ninst] = acc;
     nblocks = sb.nblocks = acc;
+    if (F->ninst == 1 && !F->plans.empty()) {  // a kernel reads its one first block, 0: any plan's
+        sb.blk0 = F->plans[0].blk0;
+        sb.shared = true;
+        F->specs.push_back(sb);
+        return SpecPlan{tab, sb.blk0, 1, sb.lz};
+    }
     if (check_hip(hipMalloc(&sb.blk0, sizeof(int) * (F->ninst + 1)), "hipMalloc(column plan)") ||
         check_hip(hipMemcpy(sb.blk0, b0.data(), sizeof(int) * (F->ninst + 1), hipMemcpyHostToDevice), "plan h2d")) {
         nblocks = 0;
@@ -1124,6 +1133,7 @@ static void launch_transfinal(FusedLevel *F, hipStream_t s, int slab)
 static void launch_stage(FusedLevel *F, int stage, hipStream_t s, int ny = 1, int slab = 0)
 {
     F->ctx.tab = eos_table();
+    if (stage == ST_PRIM && slab > 0 && !F->ring) return;  // slab 0's launch made all planes
     if (stage == ST_TRANS1C || stage == ST_FINAL || stage == ST_FINALC)
         if (joins_transverse(F, slab)) {
             // the transverse stage has made the final fluxes: the species are left
@@ -1350,15 +1360,24 @@ FusedLevel *fused_create_set(const std::vector<FusedInstanceSpec> &spec, int sla
               !check_hip(hipMemcpy(F->inst, F->hinst.data(), sizeof(FInst) * F->ninst, hipMemcpyHostToDevice), "h2d");
     F->sinst.assign(F->nslab, nullptr);
     F->pinst.assign(F->nslab, nullptr);
+    // slabs whose instances have the same planes share their block tables
+    for (int sl = 0; sl < F->nslab; ++sl) {
+        int k = 0;
+        while (k < sl && !std::equal(F->hsinst[k].begin(), F->hsinst[k].end(), F->hsinst[sl].begin(),
+                                     [](const FInst &a, const FInst &b) { return a.zn == b.zn; }))
+            ++k;
+        F->like.push_back(k);
+    }
+    if (!F->ring) F->pinst[0] = F->inst;
     if (!F->slab) {
-        F->sinst[0] = F->pinst[0] = F->inst;
+        F->sinst[0] = F->inst;
     } else {
         auto table = [&](FInst *&d, const std::vector<FInst> &h) {
             return !check_hip(hipMalloc(&d, sizeof(FInst) * F->ninst), "hipMalloc(slab inst)") &&
                    !check_hip(hipMemcpy(d, h.data(), sizeof(FInst) * F->ninst, hipMemcpyHostToDevice), "h2d");
         };
         for (int sl = 0; sl < F->nslab && ok; ++sl)
-            ok = table(F->sinst[sl], F->hsinst[sl]) && table(F->pinst[sl], F->hpinst[sl]);
+            ok = table(F->sinst[sl], F->hsinst[sl]) && (!F->ring || table(F->pinst[sl], F->hpinst[sl]));
     }
     auto A = [&](double *&p, long n) {
         if (ok && check_hip(hipMalloc(&p, sizeof(double) * std::max(n, 1L)), "hipMalloc(fused)")) ok = false;
@@ -1459,13 +1478,13 @@ void fused_destroy(FusedLevel *F)
     for (auto &pb : F->plans)
         if (pb.blk0) (void)hipFree(pb.blk0);
     for (auto &sb : F->specs)
-        if (sb.blk0) (void)hipFree(sb.blk0);
-    if (F->slab) {
+        if (sb.blk0 && !sb.shared) (void)hipFree(sb.blk0);
+    if (F->slab)
         for (FInst *p : F->sinst)
             if (p) (void)hipFree(p);
+    if (F->ring)
         for (FInst *p : F->pinst)
             if (p) (void)hipFree(p);
-    }
     if (F->inst) (void)hipFree(F->inst);
     if (F->abox) (void)hipFree(F->abox);
     if (F->abstart) (void)hipFree(F->abstart);

@@ -525,6 +525,7 @@ struct FusedLevel {
     struct SpecBuf {
         int slab, per_tile, lz, nblocks = 0;
         int *blk0 = nullptr;
+        bool shared = false;  // another plan's
     };
     std::vector<SpecBuf> specs;
     // per stage: est prim flat trace flux1 trans1 final update tflux
@@ -549,6 +550,7 @@ struct FusedLevel {
     bool ring = false;  // some instance's primitives are a ring of planes
     std::vector<FInst *> sinst;
     std::vector<std::vector<FInst>> hsinst;
+    std::vector<int> like;  // the first slab with the same planes, whose block tables a slab takes
     // and one per slab for K_prim, whose planes run ahead of the slab's
     // (zlo, zn: the planes not yet in the ring, unwrapped)
     std::vector<FInst *> pinst;
