@@ -126,8 +126,17 @@ static int eos_upload(const double *tab)
         if (!iter_cell(it, t_, i, j, k)) return;                         \
     }
 
+// Kernels that solve the EOS are built for one wavefront per SIMD, which may hold
+// what it likes in registers, and for two.  Up to a block for each CU the first
+// are the faster (us: mc_eos_eval_batch of 5419 unordered points, modes 1, 2, 3:
+// 8.1, 21.9 and 15.9 against 8.3, 22.0 and 16.7; of 1,000,000: 117, 335 and 239
+// against 99, 313 and 225; ctoprim of 32^3 cells 18.7 against 20.6).
+constexpr long ONE_WAVE = 65536;
+
 // Source/Castro_hydro_nd.F90:73-170
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_ctoprim(BoxIter it, Arr u, Arr q, Arr qaux, EosTable tab)
+template <int WAVES>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void
+k_ctoprim(BoxIter it, Arr u, Arr q, Arr qaux, EosTable tab)
 {
     MC_CELL(it)
     double uc[NVAR];
@@ -762,11 +771,6 @@ k_eos_batch(int n, const double *rho, const double *T, const double *ev, const d
     }
 }
 
-// Up to a block for each CU a wavefront has its SIMD to itself, and the kernels
-// built for that may hold what they like in registers (5419 unordered points,
-// modes 1, 2, 3: 8.1, 21.9 and 15.9 us against 8.3, 22.0 and 16.7 of those built
-// for two; 1,000,000: 117, 335 and 239 against 99, 313 and 225).
-constexpr int EOS_ONE_WAVE = 65536;
 template <int WAVES>
 static void launch_eos_batch(int n, int mode, const double *rho, const double *T, const double *ev, const double *abar,
                              const double *zbar, double *out, hipStream_t s)
@@ -913,7 +917,7 @@ int mc_eos_eval_batch(int n, int mode, const double *rho, const double *T, const
         return -1;
     }
     if (n <= 0) return 0;
-    if (n <= EOS_ONE_WAVE) launch_eos_batch<1>(n, mode, rho, T, ev, abar, zbar, out, t_stream);
+    if (n <= ONE_WAVE) launch_eos_batch<1>(n, mode, rho, T, ev, abar, zbar, out, t_stream);
     else launch_eos_batch<2>(n, mode, rho, T, ev, abar, zbar, out, t_stream);
     return check_hip(hipGetLastError(), "k_eos_batch");
 }
@@ -972,8 +976,11 @@ void ctoprim(const int *lo, const int *hi, const double *u, const int *u_lo, con
 {
     REQUIRE_EOS();
     BoxIter it = make_iter(make_box(lo, hi));
-    hipLaunchKernelGGL(k_ctoprim, dim3(grid_for(it.n)), dim3(kBlock), 0, t_stream, it, ARR(u), ARR(q), make_arr(qaux, qa_lo, qa_hi),
-                       g_eos);
+    const Arr qa = make_arr(qaux, qa_lo, qa_hi);
+    if (it.n <= ONE_WAVE)
+        hipLaunchKernelGGL(k_ctoprim<1>, dim3(grid_for(it.n)), dim3(kBlock), 0, t_stream, it, ARR(u), ARR(q), qa, g_eos);
+    else
+        hipLaunchKernelGGL(k_ctoprim<2>, dim3(grid_for(it.n)), dim3(kBlock), 0, t_stream, it, ARR(u), ARR(q), qa, g_eos);
 }
 
 void enforce_minimum_density(const int *lo, const int *hi, double *state, const int *state_lo, const int *state_hi)

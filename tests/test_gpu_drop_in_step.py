@@ -111,3 +111,26 @@ def test_step_of_entry_points_matches_oracle(floors):
     # the boxes that share faces in y store the same fluxes on them
     a, c = faces[boxes[1], 1], faces[boxes[2], 1]
     np.testing.assert_array_equal(a[:, -1], c[:, 0])
+
+
+def test_ctoprim_of_a_large_box_equals_small_ones():
+    """A box of more cells than the kernel for one wavefront per SIMD takes, and
+    the same cells in smaller boxes of the same FABs."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    mc.load_table(table_bin())
+    n = (47, 40, 36)
+    assert 65536 < np.prod(n) < 2 * 65536
+    b = ((0, 0, 0), tuple(v - 1 for v in n))
+    u = Dev(*b, NVAR, mixed_flow(n, seed=5))
+    clean_state(u)
+    got = []
+    for cuts in ((0, 47), (0, 20, 47), (0, 1, 30, 47)):
+        q, qaux = Dev(*b, QVAR), Dev(*b, NQAUX)
+        for lo, hi in zip(cuts, cuts[1:]):
+            gpu_call("ctoprim", orc.iv(lo, 0, 0), orc.iv(hi - 1, 39, 35), u, q, qaux)
+        got.append((q.host(), qaux.host()))
+    for q, qaux in got[1:]:
+        np.testing.assert_array_equal(q, got[0][0])
+        np.testing.assert_array_equal(qaux, got[0][1])
