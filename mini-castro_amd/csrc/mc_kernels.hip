@@ -454,20 +454,10 @@ __global__ __launch_bounds__(kBlock) void k_apply_av(BoxIter it, int idir, doubl
         km = k - 1;
     }
     div1 = difmag * fmin(0.0, div1);
-    // a store holds later loads back, so ten components are read at a time
-    static_assert(NVAR % 10 == 0, "two halves");
-#pragma unroll
-    for (int h = 0; h < NVAR; h += 10) {
-        double f[10];
-#pragma unroll
-        for (int n = 0; n < 10; ++n) {
-            if (h + n == UTEMP) continue;
-            const double d1 = div1 * (u(i, j, k, h + n) - u(im, jm, km, h + n));
-            f[n] = flux(i, j, k, h + n) + dxd * d1;
-        }
-#pragma unroll
-        for (int n = 0; n < 10; ++n)
-            if (h + n != UTEMP) flux(i, j, k, h + n) = f[n];
+    for (int n = 0; n < NVAR; ++n) {
+        if (n == UTEMP) continue;
+        const double d1 = div1 * (u(i, j, k, n) - u(im, jm, km, n));
+        flux(i, j, k, n) = flux(i, j, k, n) + dxd * d1;
     }
 }
 
@@ -488,11 +478,7 @@ __global__ __launch_bounds__(kBlock) void k_store_flux(BoxIter it, Arr fo, Arr f
 {
     MC_CELL(it)
     const double a = area(i, j, k, 0);
-    double f[NVAR];  // all loads ahead of the stores, which would hold them back
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) f[n] = dt * fi(i, j, k, n) * a;
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n) fo(i, j, k, n) = f[n];
+    for (int n = 0; n < NVAR; ++n) fo(i, j, k, n) = dt * fi(i, j, k, n) * a;
 }
 
 // The three of them in one pass over the faces: their own read and write the
