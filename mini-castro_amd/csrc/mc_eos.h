@@ -192,23 +192,6 @@ __device__ __forceinline__ EosRows eos_rows(const EosTable &tab, int iat, int ja
     r.off = ((unsigned)(iat - 1) + (unsigned)EOS_IMAX * (unsigned)(jat - 1)) * (8u * EOS_NODE);
     return r;
 }
-// Pairs FROM..TO-1 row after row, for solves that stand alone: a wavefront's
-// loads of one row's pairs meet in its lines while the vector L1 has them.  Left
-// to order them, the compiler takes the pairs in turn, each over all four rows
-// (1,000,000 unordered (rho, T) evaluations 99 us, pair after pair 110).
-template <int FROM, int TO>
-__device__ __forceinline__ void eos_load_rows(const EosRows &r, EosCols *col)
-{
-    auto row = [&](auto put, long node) {
-#pragma unroll
-        for (int l = FROM; l < TO; ++l) put(col[l]) = *(const double2 *)(r.base + r.off + 16 * l + node);
-        asm volatile("" ::: "memory");
-    };
-    row([](EosCols &c) -> double2 & { return c.a; }, 0);
-    row([](EosCols &c) -> double2 & { return c.b; }, 8 * EOS_NODE);
-    row([](EosCols &c) -> double2 & { return c.c; }, 8L * EOS_IMAX * EOS_NODE);
-    row([](EosCols &c) -> double2 & { return c.d; }, 8L * EOS_IMAX * EOS_NODE + 8 * EOS_NODE);
-}
 // The next columns' address waits for the sums so far: without the tie the
 // compiler gathers every column of every sum first (104 registers of table
 // values, and one wavefront per SIMD or spills).
@@ -219,35 +202,22 @@ __device__ __forceinline__ void eos_load_rows(const EosRows &r, EosCols *col)
 __device__ constexpr int eos_dsel[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
 __device__ constexpr int eos_tsel[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
 
-// A temperature's table cell and its grid entry.
-struct EosTemp {
-    int jat;
-    double tJ, dt, dt2, dti, dt2i;
-};
-__device__ __forceinline__ EosTemp eos_temp_of(const EosTable &tab, int jat)
-{
-    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
-    return EosTemp{jat, g[G_X], g[G_D], g[G_D2], g[G_DI], g[G_D2I]};
-}
-__device__ __forceinline__ EosTemp eos_temp(const EosTable &tab, double temp)
-{
-    return eos_temp_of(tab, eos_cell(temp, eosc::tlo, eosc::tstpi, EOS_JMAX - 1));
-}
-
 // e and de/dT at temperature temp (Source/eos.F90:195-518): what a Newton
 // iteration needs.
 // The biquintic sums (Source/eos.F90:915-950) of the free energy and its
 // derivatives run column by column: every sum adds the reference's terms in
-// its order, EOS_CHUNK pairs of columns of the four nodes at a time.  HAVE: they
-// are in col already.
-template <bool HAVE>
-__device__ __forceinline__ void eos_energy_at(const EosTable &tab, const EosDen &s, double temp, const EosTemp &t,
-                                              EosCols *col, EosFull &o)
+// its order, EOS_CHUNK pairs of columns of the four nodes at a time.
+__device__ __forceinline__ void eos_energy(const EosTable &tab, const EosDen &s, double temp, int &jat_out,
+                                           EosFull &o)
 {
     using namespace eosc;
     const double den = s.den, deni = s.deni, ytot1 = s.ytot1, ye = s.ye;
-    EosRows rows = eos_rows(tab, s.iat, t.jat);
-    const double tJ = t.tJ, dt = t.dt, dt2 = t.dt2, dti = t.dti, dt2i = t.dt2i;
+    const int jat = eos_cell(temp, tlo, tstpi, EOS_JMAX - 1);
+    jat_out = jat;
+    EosRows rows = eos_rows(tab, s.iat, jat);
+    EosCols col[5];
+    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
+    const double tJ = g[G_X], dt = g[G_D], dt2 = g[G_D2], dti = g[G_DI], dt2i = g[G_D2I];
 
     const double tempi = 1.0 / temp;
     const double prad = asoli3 * temp * temp * temp * temp;
@@ -284,7 +254,7 @@ __device__ __forceinline__ void eos_energy_at(const EosTable &tab, const EosDen 
     double free = 0.0, df_t = 0.0, df_tt = 0.0;
 #pragma unroll
     for (int c2 = 0; c2 < 5; ++c2) {
-        if (!HAVE && c2 % EOS_CHUNK == 0) {
+        if (c2 % EOS_CHUNK == 0) {
             if (c2) MC_EOS_STEP(rows, free, df_t, df_tt);
 #pragma unroll
             for (int l = c2; l < c2 + EOS_CHUNK && l < 5; ++l) col[l] = rows.load(l);
@@ -310,27 +280,19 @@ __device__ __forceinline__ void eos_energy_at(const EosTable &tab, const EosDen 
     o.e = erad + eion + eele;
     o.dedT = deraddt + deiondt + deepdt;
 }
-__device__ __forceinline__ void eos_energy(const EosTable &tab, const EosDen &s, double temp, int &jat_out,
-                                           EosFull &o)
-{
-    const EosTemp t = eos_temp(tab, temp);
-    jat_out = t.jat;
-    EosCols col[5];
-    eos_energy_at<false>(tab, s, temp, t, col, o);
-}
 
 // The rest of an evaluation whose e and de/dT eos_energy left in o: pressure
-// and its derivatives, de/drho, gamma_1.  HAVE: pairs of columns that are in
-// col already (0, 5 or 7).
-template <int HAVE>
-__device__ __forceinline__ void eos_pressure_at(const EosTable &tab, const EosDen &s, double dd, double ddi, double temp,
-                                                const EosTemp &t, EosCols *col, EosFull &o)
+// and its derivatives, de/drho, gamma_1.
+__device__ __forceinline__ void eos_pressure(const EosTable &tab, const EosDen &s, double temp, int jat, EosFull &o)
 {
     using namespace eosc;
-    static_assert(HAVE == 0 || HAVE == 7 || HAVE == EOS_CHUNK, "groups of columns");
     const double den = s.den, deni = s.deni, ytot1 = s.ytot1, ye = s.ye;
-    EosRows rows = eos_rows(tab, s.iat, t.jat);
-    const double tJ = t.tJ, dt = t.dt, dt2 = t.dt2, dti = t.dti;
+    EosRows rows = eos_rows(tab, s.iat, jat);
+    EosCols col[7];
+    const double *g = tab.tg + (long)(jat - 1) * EOS_GRID;
+    const double tJ = g[G_X], dt = g[G_D], dt2 = g[G_D2], dti = g[G_DI];
+    const double *gd = tab.dg + (long)(s.iat - 1) * EOS_GRID;
+    const double dd = gd[G_D], ddi = gd[G_DI];
     const double xt = fmax((temp - tJ) * dti, 0.0);
     const double mxt = 1.0 - xt, xd = s.xd, mxd = 1.0 - s.xd;
 
@@ -360,8 +322,8 @@ __device__ __forceinline__ void eos_pressure_at(const EosTable &tab, const EosDe
     double df_d = 0.0, df_dt = 0.0, dpepdd = 0.0;
 #pragma unroll
     for (int c2 = 0; c2 < 7; ++c2) {
-        if (c2 >= HAVE && c2 % EOS_CHUNK == 0) {
-            if (c2 && !HAVE) MC_EOS_STEP(rows, df_d, df_dt, dpepdd);
+        if (c2 % EOS_CHUNK == 0) {
+            if (c2) MC_EOS_STEP(rows, df_d, df_dt, dpepdd);
 #pragma unroll
             for (int l = c2; l < c2 + EOS_CHUNK && l < 7; ++l) col[l] = rows.load(l);
         }
@@ -421,25 +383,13 @@ __device__ __forceinline__ void eos_pressure_at(const EosTable &tab, const EosDe
     o.dedr = denerdd;
 }
 #undef MC_EOS_STEP
-__device__ __forceinline__ void eos_pressure(const EosTable &tab, const EosDen &s, double temp, int jat, EosFull &o)
-{
-    const EosTemp t = eos_temp_of(tab, jat);
-    const double *gd = tab.dg + (long)(s.iat - 1) * EOS_GRID;
-    EosCols col[7];
-    eos_pressure_at<0>(tab, s, gd[G_D], gd[G_DI], temp, t, col, o);
-}
 
-// One whole evaluation that stands alone, from one reading of its columns.
+// e and de/dT of one state.  eos_rt_e calls this, not eos_energy, which changes the
+// order in which the compiler inlines: the same arithmetic, but K_prim of 256^3 takes
+// 3.10 ms with the direct call and 2.96 so.
 __device__ __forceinline__ void eos_eval(const EosTable &tab, const EosDen &s, double temp, int &jat, EosFull &o)
 {
-    const EosTemp t = eos_temp(tab, temp);
-    const double *gd = tab.dg + (long)(s.iat - 1) * EOS_GRID;
-    const double dd = gd[G_D], ddi = gd[G_DI];
-    EosCols col[7];
-    jat = t.jat;
-    eos_load_rows<0, 7>(eos_rows(tab, s.iat, t.jat), col);
-    eos_energy_at<true>(tab, s, temp, t, col, o);
-    eos_pressure_at<7>(tab, s, dd, ddi, temp, t, col, o);
+    eos_energy(tab, s, temp, jat, o);
 }
 
 // Result of a (rho, e) solve.
@@ -509,37 +459,7 @@ __device__ __forceinline__ double eos_rt_e(const EosTable &tab, double rho, doub
     eos_density(tab, rho, abar, zbar, s);
     EosFull o;
     int jat;
-    eos_energy(tab, s, T, jat, o);
-    return o.e;
-}
-
-// eos(eos_input_rp, ...): Newton on T for a target pressure; returns e.  An
-// iteration takes e, p and dp/dT from one reading of the table, whose grid
-// entries are read ahead of it: a small batch waits for one reading after
-// another (5419 unordered points 15.9 us; with energy and pressure apart in turn
-// 19.0; with p and dp/dT alone, and e once at the end, 17.6; 1,000,000: 226, 250
-// and 204).
-__device__ __forceinline__ double eos_rp_e(const EosTable &tab, double rho, double T0, double p_want, double abar,
-                                           double zbar, double *T_out)
-{
-    EosDen s;
-    eos_density(tab, rho, abar, zbar, s);
-    const double *gd = tab.dg + (long)(s.iat - 1) * EOS_GRID;
-    const double dd = gd[G_D], ddi = gd[G_DI];
-    double temp = T0;
-    bool converged = false;
-    EosFull o;
-    for (int iter = 1; iter <= EOS_MAX_NEWTON; ++iter) {
-        const EosTemp t = eos_temp(tab, temp);
-        EosCols col[EOS_CHUNK];
-        eos_load_rows<0, EOS_CHUNK>(eos_rows(tab, s.iat, t.jat), col);
-        eos_energy_at<true>(tab, s, temp, t, col, o);
-        eos_pressure_at<EOS_CHUNK>(tab, s, dd, ddi, temp, t, col, o);
-        if (converged) break;
-        converged = eos_newton(temp, o.p, p_want, o.dpdT);
-    }
-    if (!converged) eos_note_newton_failure(tab);
-    if (T_out) *T_out = temp;
+    eos_eval(tab, s, T, jat, o);
     return o.e;
 }
 

@@ -18,6 +18,7 @@
 #include "helmgen.h"
 #include "mc_common.h"
 #include "mc_eos.h"
+#include "mc_eos_once.h"
 #include "mc_hydro.h"
 #include "mc_cell.h"
 #include "mc_internal.h"
@@ -130,7 +131,7 @@ static int eos_upload(const double *tab)
 // what it likes in registers, and for two.  Up to a block for each CU the first
 // are the faster (us: mc_eos_eval_batch of 5419 unordered points, modes 1, 2, 3:
 // 8.1, 21.9 and 15.9 against 8.3, 22.0 and 16.7; of 1,000,000: 117, 335 and 239
-// against 99, 313 and 225; ctoprim of 32^3 cells 18.7 against 20.6).
+// against 96, 320 and 232; ctoprim of 32^3 cells 18.7 against 20.6).
 constexpr long ONE_WAVE = 65536;
 
 // Source/Castro_hydro_nd.F90:73-170
@@ -747,7 +748,7 @@ k_eos_batch(int n, const double *rho, const double *T, const double *ev, const d
         eos_density(tab, rho[c], abar[c], zbar[c], s);
         EosFull f;
         int jat;
-        eos_eval(tab, s, T[c], jat, f);
+        eos_rt(tab, s, T[c], jat, f);
         o[0] = T[c]; o[1] = f.p; o[2] = f.e; o[3] = sqrt(f.gam1 * f.p / rho[c]); o[4] = f.gam1; o[5] = f.dpde;
         o[6] = f.dpdr_e; o[7] = f.dedT; o[8] = s.iat; o[9] = jat;
     } else {
